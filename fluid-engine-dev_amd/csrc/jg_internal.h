@@ -168,9 +168,14 @@ struct jg_solver {
            *q = nullptr;
     float *rhs32 = nullptr, *r32 = nullptr, *z32 = nullptr, *d32A = nullptr, *d32B = nullptr,
           *q32 = nullptr, *e32 = nullptr;
-    // Velocity boundary conditions: projected faces, two validity masks.
+    // Velocity boundary conditions: projected values per listed face, two
+    // validity masks (1 between calls), the face lists, two bits per cell,
+    // and the lists' lengths (allocated last: all or none).
     double* bc_tmp = nullptr;
     int8_t* bc_valid = nullptr;
+    unsigned* bc_list = nullptr;
+    unsigned long long* bc_bits = nullptr;
+    unsigned* bc_count = nullptr;
     // Compressed (CSR) system of jg_csr_cg_solve_host and its CG vectors.
     struct Csr {
         size_t rows = 0, nnz = 0, cap_rows = 0, cap_nnz = 0;
@@ -220,6 +225,8 @@ struct jg_solver {
         rhs32 = r32 = z32 = d32A = d32B = q32 = e32 = nullptr;
         bc_tmp = nullptr;
         bc_valid = nullptr;
+        bc_list = bc_count = nullptr;
+        bc_bits = nullptr;
         csr = Csr{};
         part = scal = nullptr;
         ctl = nullptr;

@@ -444,40 +444,50 @@ int jg_constrain_velocity(jg_solver* s, int blocked, const double h[3], const do
     const idx_t nf[3] = {(idx_t)(d.nx + 1) * d.ny * d.nz, (idx_t)d.nx * (d.ny + 1) * d.nz,
                          (idx_t)d.nx * d.ny * (d.nz + 1)};
     const idx_t total = nf[0] + nf[1] + nf[2];
-    if (!s->bc_tmp) {
+    const idx_t words = (idx_t)bc_cell_words(d) * d.ny * d.nz;
+    hipStream_t st = s->stream;
+    if (!s->bc_count) {
         JG_TRY(dalloc(s, &s->bc_tmp, total));
         JG_TRY(dalloc(s, &s->bc_valid, 2 * total));
+        JG_TRY(dalloc(s, &s->bc_list, total));
+        JG_TRY(dalloc(s, &s->bc_bits, 2 * words));
+        k_bc_valid<<<nblocks_1d(2 * total), 256, 0, st>>>(s->bc_valid, 2 * total);
+        JG_TRY(check_launch(s, "constrain_velocity"));
+        JG_TRY(dalloc(s, &s->bc_count, 3));
     }
-    double* comp[3] = {u, v, w};
-    double* tmp[3] = {s->bc_tmp, s->bc_tmp + nf[0], s->bc_tmp + nf[0] + nf[1]};
-    int8_t* va[3] = {s->bc_valid, s->bc_valid + nf[0], s->bc_valid + nf[0] + nf[1]};
-    int8_t* vb[3] = {va[0] + total, va[1] + total, va[2] + total};
-    hipStream_t st = s->stream;
-    auto nb = [&](int a) { return nblocks_1d(nf[a]); };
-    // markers and collider velocity on covered faces
-    k_bc_init<0><<<nb(0), 256, 0, st>>>(g, collider_sdf, c, u, va[0]);
-    k_bc_init<1><<<nb(1), 256, 0, st>>>(g, collider_sdf, c, v, va[1]);
-    k_bc_init<2><<<nb(2), 256, 0, st>>>(g, collider_sdf, c, w, va[2]);
-    // free slip: extrapolation into the collider, validity ping-pong
-    for (unsigned it = 0; it < extrapolation_depth; ++it) {
-        int8_t* const* in = (it & 1) ? vb : va;
-        int8_t* const* out = (it & 1) ? va : vb;
-        k_bc_extrapolate<0><<<nb(0), 256, 0, st>>>(d, u, in[0], out[0]);
-        k_bc_extrapolate<1><<<nb(1), 256, 0, st>>>(d, v, in[1], out[1]);
-        k_bc_extrapolate<2><<<nb(2), 256, 0, st>>>(d, w, in[2], out[2]);
+    BcArgs p;
+    p.g = g;
+    p.c = c;
+    p.sdf = collider_sdf;
+    double* const comp[3] = {u, v, w};
+    for (int a = 0; a < 3; ++a) {
+        const idx_t off = a == 0 ? 0 : (a == 1 ? nf[0] : nf[0] + nf[1]);
+        p.comp[a] = comp[a];
+        p.tmp[a] = s->bc_tmp + off;
+        p.valid[0][a] = s->bc_valid + off;
+        p.valid[1][a] = s->bc_valid + total + off;
+        p.lists.f[a] = s->bc_list + off;
     }
-    // no flux inside the collider (reads all three components), then back
-    k_bc_project<0><<<nb(0), 256, 0, st>>>(g, collider_sdf, c, u, v, w, tmp[0]);
-    k_bc_project<1><<<nb(1), 256, 0, st>>>(g, collider_sdf, c, u, v, w, tmp[1]);
-    k_bc_project<2><<<nb(2), 256, 0, st>>>(g, collider_sdf, c, u, v, w, tmp[2]);
-    k_bc_finish<0><<<nb(0), 256, 0, st>>>(d, tmp[0], comp[0], closed_walls);
-    k_bc_finish<1><<<nb(1), 256, 0, st>>>(d, tmp[1], comp[1], closed_walls);
-    k_bc_finish<2><<<nb(2), 256, 0, st>>>(d, tmp[2], comp[2], closed_walls);
-    if (blocked) {
-        k_bc_blocked<0><<<nb(0), 256, 0, st>>>(g, collider_sdf, c, u);
-        k_bc_blocked<1><<<nb(1), 256, 0, st>>>(g, collider_sdf, c, v);
-        k_bc_blocked<2><<<nb(2), 256, 0, st>>>(g, collider_sdf, c, w);
-    }
+    p.lists.count = s->bc_count;
+    // The list leaves out faces by the cells that their samples can round
+    // into, which takes coordinates good to well under a cell: where the
+    // origin is so far off that they are not, every face is listed.
+    bool all = false;
+    const int cells[3] = {d.nx, d.ny, d.nz};
+    for (int a = 0; a < 3; ++a)
+        if (!((std::fabs(o[a]) + h[a] * (cells[a] + 1.0)) / h[a] < 1073741824.0)) all = true;
+    k_bc_bits<<<(unsigned)std::min<idx_t>((words + 31) / 32, 4096), 256, 0, st>>>(
+        collider_sdf, d, all ? 1 : 0, s->bc_bits, s->bc_count);
+    k_bc_dilate<<<(unsigned)((words + 255) / 256), 256, 0, st>>>(s->bc_bits, d, s->bc_bits + words);
+    const idx_t fwords = (idx_t)bc_face_words(d) * (d.ny + 1) * (d.nz + 1);
+    k_bc_list<<<(unsigned)((fwords + kBcListThreads - 1) / kBcListThreads), kBcListThreads, 0, st>>>(s->bc_bits + words, d, p.lists);
+    // the lists' lengths stay on the device: bounded grids that loop
+    const dim3 grid((unsigned)std::min<idx_t>((nf[0] + 255) / 256, 1024), 3, 1);
+    k_bc_init<<<grid, 256, 0, st>>>(p);
+    for (unsigned it = 0; it < extrapolation_depth; ++it)
+        k_bc_extrapolate<<<grid, 256, 0, st>>>(p, (int)(it & 1));
+    k_bc_project<<<grid, 256, 0, st>>>(p);
+    k_bc_finish<<<dim3(grid.x, 6, 1), 256, 0, st>>>(p, closed_walls, blocked ? 1 : 0);
     JG_TRY(check_launch(s, "constrain_velocity"));
     return sync(s);
 }

@@ -488,7 +488,7 @@ enum {
  * colliderSdf grid; DBL_MAX everywhere when there is no collider); collider
  * NULL means a resting collider (zero velocity and friction).  Jet's caller
  * passes extrapolation_depth = ceil(max CFL) (src/jet/grid_fluid_solver3.cpp:
- * 346-353).  Scratch: 8 B + 2 B per face, allocated on first use. */
+ * 346-353).  Scratch: 14 B per face and 2 bits per cell, allocated on first use. */
 int jg_constrain_velocity(jg_solver* s, int blocked, const double h[3], const double o[3],
                           double* u, double* v, double* w, const double* collider_sdf,
                           const jg_rigid_collider* collider, unsigned extrapolation_depth,

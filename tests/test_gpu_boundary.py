@@ -96,3 +96,37 @@ def test_constrain_velocity_rejects_bad_arguments(solver):
     oo = (C.c_double * 3)(0.0, 0.0, 0.0)
     lib = jetgpu.lib()
     assert lib.jg_constrain_velocity(solver.h, 0, hh, oo, None, None, None, None, None, 1, 63) != 0
+
+
+@pytest.mark.parametrize("n,scene,seed", [
+    ((63, 6, 5), "sphere", 21), ((64, 7, 6), "noise", 22), ((65, 5, 9), "corner", 23),
+    ((129, 4, 3), "noise", 24), ((2, 1, 70), "noise", 25), ((24, 20, 18), "far", 26),
+    ((30, 22, 26), "inside", 27), ((66, 9, 8), "nan", 28)])
+def test_constrain_velocity_face_lists(solver, oracle, n, scene, seed):
+    # The stages run over lists of the faces near the collider, made from a
+    # bit per cell in words of 64: rows shorter than a word, one longer and
+    # just over; scattered collider cells, a collider in a corner, one that
+    # fills the grid, NaN distances, and an origin so far off that face
+    # coordinates no longer resolve a cell (every face is listed then).
+    print(f"case constrain lists n={n} scene={scene}", flush=True)
+    far = (3e9, -2e9, 1e9) if scene == "far" else (0.1, -0.2, 0.05)
+    h, o, sdf, vel, motion = collider_scene(n, seed, origin=far)
+    r = np.random.default_rng(seed)
+    if scene == "noise":
+        sdf = np.where(r.random(sdf.shape) < 0.04, -r.random(sdf.shape), r.random(sdf.shape)) * h[0]
+    elif scene == "corner":
+        sdf[...] = h[0]
+        sdf[-2:, -2:, -2:] = -h[0]
+        sdf[0, 0, 0] = 0.0
+    elif scene == "far":
+        sdf = r.uniform(-1, 1, sdf.shape)
+    elif scene == "inside":
+        sdf = -1.0 - r.random(sdf.shape)
+    elif scene == "nan":
+        sdf[1, 2, 63] = np.nan
+        sdf[4, 4, 4] = np.inf
+    for blocked, depth in ((True, 4), (False, 1)):
+        got = run_gpu(solver, vel, sdf, h, o, motion, depth, 63, blocked)
+        want = run_oracle(oracle, vel, sdf, h, o, motion, depth, 63, blocked)
+        for a, b in zip(got, want):
+            assert np.array_equal(a, b, equal_nan=True)
