@@ -103,6 +103,42 @@ __device__ __forceinline__ double dpp_shift(double v) {
 
 // ---------------------------------------------------------------- reduce
 
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_or_zero(double v) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)u, CTRL, ROWS, 0xF, true);
+    const unsigned hi =
+        (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(u >> 32), CTRL, ROWS, 0xF, true);
+    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+
+// Sum of v over each row of 16 lanes, in the row's last lane (row_shr by 1,
+// 2, 4 and 8; a lane without a source adds zero).
+__device__ __forceinline__ double row_sum(double v) {
+    v += dpp_or_zero<0x111, 0xF>(v);
+    v += dpp_or_zero<0x112, 0xF>(v);
+    v += dpp_or_zero<0x114, 0xF>(v);
+    v += dpp_or_zero<0x118, 0xF>(v);
+    return v;
+}
+
+// Sum of v over the wave, in lane 63: the row sums, then row_bcast:15 and
+// row_bcast:31 carry them on.  Register moves throughout; six shuffles through
+// the LDS crossbar cost about 0.6 us of a grid-wide sum's 2.5.
+__device__ __forceinline__ double wave_sum(double v) {
+    v = row_sum(v);
+    v += dpp_or_zero<0x142, 0xA>(v);
+    v += dpp_or_zero<0x143, 0xC>(v);
+    return v;
+}
+
+__device__ __forceinline__ double lane_value(double v, int lane) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)u, lane);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(u >> 32), lane);
+    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+
 template <int NT>
 __device__ __forceinline__ double block_sum(double v, double* sh) {
     const int lane = threadIdx.x + threadIdx.y * blockDim.x;

@@ -148,6 +148,8 @@ inline int nblocks(const Geo& g) { return (int)(g.grid.x * g.grid.y * g.grid.z);
 
 struct jg_solver {
     int device = 0;
+    int cus = 0;               // compute units of the device
+    bool cooperative = false;  // it takes cooperative launches
     // Systems held back to back (a batch group of one hierarchy): every
     // array below holds nsys of them (jg_device.h, kSys*), and the V-cycle
     // and PCG launches cover all of them.  A view is one member of a group:
@@ -202,6 +204,7 @@ struct jg_solver {
     double* scal = nullptr;  // small result area
     jg::Ctl* ctl = nullptr;      // [0]: FP64 / outer, [1]: FP32 inner
     jg::Ctl* ctl_host = nullptr; // pinned mirror, two slots
+    unsigned long long* cg_slots = nullptr;  // grid sums of k_cg_grid
     bool f32_valid = false;
     std::vector<void*> allocs;
 
@@ -229,6 +232,7 @@ struct jg_solver {
         bc_bits = nullptr;
         csr = Csr{};
         part = scal = nullptr;
+        cg_slots = nullptr;
         ctl = nullptr;
         f32_valid = false;
     }

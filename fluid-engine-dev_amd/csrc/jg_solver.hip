@@ -23,6 +23,7 @@
 #include "jg_bottom.h"
 #include "jg_transfer.h"
 #include "jg_csr.h"
+#include "jg_cggrid.h"
 
 #include <cstdlib>
 
@@ -1048,6 +1049,43 @@ int pcg_iteration(jg_solver* s, const Pcg<T>& v, bool odd) {
     return check_launch(s, "pcg iteration");
 }
 
+// Rows per thread when the CG of v (FP64, no preconditioner) runs as one
+// cooperative launch (k_cg_grid), 0 when it does not: every row of the
+// system has to fit the registers of one block per CU, with at most kCgW
+// entries.  One row per thread as far as that goes: at 64^3 256 blocks of
+// one take 8.2 us an iteration, 128 blocks of two 10.4, though their sums
+// cost less.
+int cg_grid_rows(jg_solver* s, const Pcg<double>& v) {
+    const idx_t n = v.d.n(), per = (idx_t)std::min(s->cus, kCgMaxBlocks) * kCgThreads;
+    if (v.mg || s->nsys > 1 || !s->cooperative || n > 2 * per) return 0;
+    if (v.csr && (!v.ell || s->csr.ell_w > kCgW)) return 0;
+    return n > per ? 2 : 1;
+}
+
+// pcg_device through k_cg_grid; the state after pcg_init in, x and the
+// control block out.
+int cg_grid(jg_solver* s, const Pcg<double>& v, int C) {
+    if (!s->cg_slots) JG_TRY(dalloc(s, &s->cg_slots, 3 * kCgSumWords));
+    const idx_t n = v.d.n();
+    CgGridArgs a{v.A, v.ell ? *v.ell : EllDev{}, v.d, v.b, v.x, v.r, v.dA, v.ctl, s->cg_slots};
+    const dim3 grid((unsigned)((n + (idx_t)C * kCgThreads - 1) / ((idx_t)C * kCgThreads)));
+    const void* f = v.ell ? (C == 1 ? (const void*)k_cg_grid<1, true> : (const void*)k_cg_grid<2, true>)
+                          : (C == 1 ? (const void*)k_cg_grid<1, false> : (const void*)k_cg_grid<2, false>);
+    void* args[] = {&a};
+    do {
+        k_fill<unsigned long long><<<nblocks_1d(3 * kCgSumWords), NT, 0, s->stream>>>(s->cg_slots, 0ull,
+                                                                                  3 * kCgSumWords);
+        JG_HIP(hipLaunchCooperativeKernel(f, grid, dim3(kCgThreads), args, 0, s->stream));
+        JG_HIP(hipMemcpyAsync(s->ctl_host, v.ctl, sizeof(Ctl), hipMemcpyDeviceToHost, s->stream));
+        JG_TRY(sync(s));
+    } while (!s->ctl_host->done);
+    if (s->ctl_host->pad) {
+        s->err = "CG: a block of the cooperative launch did not arrive";
+        return JG_ERR_HIP;
+    }
+    return JG_OK;
+}
+
 // Jet's pcg control flow (include/jet/detail/cg-inl.h:15-94) on the device.
 // Vectors of type T; the matrix of level 0 is A; M is either the identity
 // (z aliases r) or the V-cycle.  x must be zero on entry (Jet zeroes it).
@@ -1055,6 +1093,10 @@ int pcg_iteration(jg_solver* s, const Pcg<T>& v, bool odd) {
 template <typename T>
 int pcg_device(jg_solver* s, const Pcg<T>& v, unsigned check_every) {
     JG_TRY(pcg_init<T>(s, v));
+    if constexpr (sizeof(T) == 8) {
+        const int rows = cg_grid_rows(s, v);
+        if (rows) return cg_grid(s, v, rows);
+    }
     JG_HIP(hipMemcpyAsync(s->ctl_host, v.ctl, sizeof(Ctl), hipMemcpyDeviceToHost, s->stream));
     JG_TRY(sync(s));
     if (s->ctl_host->done) return JG_OK;
@@ -1489,6 +1531,13 @@ int jg_solver_create(int device, jg_solver** out) {
         delete s;
         return JG_ERR_HIP;
     }
+    int coop = 0;
+    if (hipDeviceGetAttribute(&s->cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
+        hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, device) != hipSuccess) {
+        delete s;
+        return JG_ERR_HIP;
+    }
+    s->cooperative = coop != 0;
     // this device's address of the no-allocation scratch array (a failure is
     // reported by jg_relax_red_black_noalloc, the only user)
     (void)scratch_init(device);

@@ -218,3 +218,62 @@ def test_mgpcg_mixed_refinement_limit_is_not_convergence(solver):
     assert info.refinements == 1 and info.last_residual > 1e-10 and not info.converged
     info = solver.mgpcg(200, p, jetgpu.gpu_options(precision=jetgpu.JG_MIXED))
     assert info.last_residual <= 1e-10 and info.converged
+
+
+# One launch holds the whole CG up to two rows per thread of a 1024-thread
+# block on each of 256 CUs: a block less one row, exactly one, one more, the
+# last grid with one row per thread (64 x 64 x 64), the first with two, the
+# last of those (1024 x 512) and the first that takes the per-kernel loop.
+@pytest.mark.parametrize("shape", [(33, 31, 1), (32, 32, 1), (25, 41, 1), (64, 64, 64), (65, 64, 64),
+                                   (1024, 512, 1), (1024, 513, 1)])
+def test_cg_one_launch_matches_oracle(solver, oracle, shape):
+    print(f"case cg one launch shape={shape}", flush=True)
+    rng = np.random.default_rng(31)
+    nx, ny, nz = shape
+    A, _ = poisson_helper(nx, ny, nz)
+    A[..., 0] += 0.02  # some hundred iterations: past the 50-iteration refreshes
+    b = rng.uniform(-1, 1, (nz, ny, nx))
+    xo, io, ro, oko = oracle.cg_solve(A, b, 600, 1e-8)
+    solver.set_levels([shape])
+    solver.upload(0, A, b)
+    info = solver.cg(600, 1e-8)
+    x = solver.download_x()
+    assert io > 50 and abs(int(info.iterations) - io) <= 2 and bool(info.converged) == oko
+    # both stop at ||r|| <= 1e-8, and the smallest eigenvalue is 0.02
+    assert np.linalg.norm((x - xo).ravel()) <= 2 * 1e-8 / 0.02
+    again = solver.cg(600, 1e-8)
+    assert again.iterations == info.iterations and np.array_equal(solver.download_x(), x)
+    assert solver.cg(37, 0.0).iterations == 37
+
+
+def test_cg_one_launch_from_two_threads(solver):
+    # cooperative launches of two solvers in flight at once: each equals its
+    # solve alone, bit for bit
+    import threading
+
+    print("case cg one launch, two threads", flush=True)
+    rng = np.random.default_rng(32)
+    out, want = [None, None], []
+    solvers = [jetgpu.Solver(0) for _ in range(2)]
+    try:
+        for q, s in enumerate(solvers):
+            A = random_stencil(64, 60, 64 + 8 * q, rng)
+            s.set_levels([(64, 60, 64 + 8 * q)])
+            s.upload(0, A, rng.uniform(-1, 1, A.shape[:3]))
+            s.cg(300, 0.0)
+            want.append(s.download_x())
+
+        def work(q):
+            for _ in range(10):
+                solvers[q].cg(300, 0.0)
+            out[q] = solvers[q].download_x()
+
+        ts = [threading.Thread(target=work, args=(q,)) for q in range(2)]
+        for t in ts:
+            t.start()
+        for t in ts:
+            t.join()
+        assert np.array_equal(out[0], want[0]) and np.array_equal(out[1], want[1])
+    finally:
+        for s in solvers:
+            s.close()
