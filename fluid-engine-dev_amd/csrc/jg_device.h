@@ -26,6 +26,12 @@ struct Dims {
     __host__ __device__ idx_t n() const { return (idx_t)nx * ny * nz; }
 };
 
+// Smallest and largest cell that takes part in a solve, per axis (x, y, z;
+// jg_box.h).
+struct BoxScan {
+    int lo[3], hi[3];
+};
+
 // Device-resident scalars of one solve.  Only the finalize kernels write
 // them; every other kernel reads them, so an iteration needs no host round
 // trip and can be captured in a graph.

@@ -43,25 +43,7 @@ struct Level {
     // Variational pressure data (allocated by the first jg_fr_build): fluid
     // SDF at cell centres and face weights, float as Jet stores them.
     float *fs = nullptr, *uw = nullptr, *vw = nullptr, *ww = nullptr;
-    // Tuned z-chunk (0: untuned) and launch shape of the fused sweep, per
-    // sweep kind (kSweepPlain, kSweepZero, kSweepCorrect).
-    int zc64[3] = {0, 0, 0}, zc32[3] = {0, 0, 0};
-    int sh64[3] = {0, 0, 0}, sh32[3] = {0, 0, 0};
-    // Two sweeps per launch, per kind: kPairNone (two single sweeps),
-    // kPairMarch (k_rb_sweep2, FP32) or kPairBrick (k_brick_sweep2), as the
-    // tuner measured fastest; and the z-chunk of k_rb_sweep2.
-    int pair64[3] = {0, 0, 0}, pair32[3] = {0, 0, 0};
-    int zc2_32[3] = {0, 0, 0};
-    // z-chunk of the zero-start two-sweep launch that also writes the
-    // residual (its 5-cell halo changes the tile and block counts); 0: use
-    // the zero-start kind's
-    int zc2res_32 = 0;
 };
-
-enum { kPairNone = 0, kPairMarch = 1, kPairBrick = 2 };
-
-// Sweep kinds tuned separately: they differ in registers and loads.
-enum { kSweepPlain = 0, kSweepZero = 1, kSweepCorrect = 2, kNumSweepKinds = 3 };
 
 template <typename T>
 struct Prec;
@@ -72,12 +54,6 @@ struct Prec<double> {
     static double* b(Level& l) { return l.b64; }
     static double* t(Level& l) { return l.t64; }
     static double* y(Level& l) { return l.y64; }
-    static int& zc(Level& l, int kind = kSweepPlain) { return l.zc64[kind]; }
-    static int& sh(Level& l, int kind = kSweepPlain) { return l.sh64[kind]; }
-    static int& pair(Level& l, int kind) { return l.pair64[kind]; }
-    static int pair(const Level& l, int kind) { return l.pair64[kind]; }
-    static int zc2(const Level&, int) { return 0; }  // no FP64 z-marching two-sweep kernel
-    static int zc2res(const Level&) { return 0; }
 };
 template <>
 struct Prec<float> {
@@ -86,14 +62,6 @@ struct Prec<float> {
     static float* b(Level& l) { return l.b32; }
     static float* t(Level& l) { return l.t32; }
     static float* y(Level& l) { return l.y32; }
-    static int& zc(Level& l, int kind = kSweepPlain) { return l.zc32[kind]; }
-    static int& sh(Level& l, int kind = kSweepPlain) { return l.sh32[kind]; }
-    static int& pair(Level& l, int kind) { return l.pair32[kind]; }
-    static int pair(const Level& l, int kind) { return l.pair32[kind]; }
-    static int zc2(const Level& l, int kind) { return l.zc2_32[kind]; }
-    static int zc2res(const Level& l) {
-        return l.zc2res_32 > 0 ? l.zc2res_32 : l.zc2_32[kSweepZero];
-    }
 };
 
 struct Geo {
@@ -205,6 +173,13 @@ struct jg_solver {
     jg::Ctl* ctl = nullptr;      // [0]: FP64 / outer, [1]: FP32 inner
     jg::Ctl* ctl_host = nullptr; // pinned mirror, two slots
     unsigned long long* cg_slots = nullptr;  // grid sums of k_cg_grid
+    // Solves in a box (jg_box.h): the scan's result (and its pinned mirror),
+    // the dense rows of every level, right-hand side and solution.
+    jg::BoxScan *box_scan = nullptr, *box_host = nullptr;
+    jg::Row<double>* box_rows = nullptr;
+    double *box_b = nullptr, *box_x = nullptr;
+    size_t box_cells = 0;
+    bool box_failed = false;
     bool f32_valid = false;
     std::vector<void*> allocs;
 
@@ -214,6 +189,7 @@ struct jg_solver {
     ~jg_solver() {
         release();
         if (ctl_host) (void)hipHostFree(ctl_host);
+        if (box_host) (void)hipHostFree(box_host);
         if (ev0) (void)hipEventDestroy(ev0);
         if (ev1) (void)hipEventDestroy(ev1);
         for (hipEvent_t e : evp)
@@ -233,6 +209,11 @@ struct jg_solver {
         csr = Csr{};
         part = scal = nullptr;
         cg_slots = nullptr;
+        box_scan = nullptr;
+        box_rows = nullptr;
+        box_b = box_x = nullptr;
+        box_cells = 0;
+        box_failed = false;
         ctl = nullptr;
         f32_valid = false;
     }

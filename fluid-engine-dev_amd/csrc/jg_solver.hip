@@ -7,9 +7,10 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cfloat>
 #include <cmath>
-#include <cstdio>
 #include <cstring>
+#include <functional>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -24,6 +25,7 @@
 #include "jg_transfer.h"
 #include "jg_csr.h"
 #include "jg_cggrid.h"
+#include "jg_box.h"
 
 #include <cstdlib>
 
@@ -73,34 +75,37 @@ hipError_t scratch_address(int device, double** out) {
 
 // ------------------------------------------------------- level kernels
 
-// z-chunk of the fused sweep when no tuned value exists: enough blocks to
-// fill the chip, chunks long enough that the 4-plane pipeline fill stays a
-// small overhead.  JG_SWEEP_ZC overrides everything (tuning experiments).
-int sweep_zc_env() {
-    static const int env = [] {
-        const char* e = std::getenv("JG_SWEEP_ZC");
-        return e ? std::atoi(e) : 0;
-    }();
-    return env;
+// Planes per block of a z-marching launch of `tiles` columns (over all
+// systems) on nz planes, when `slots` blocks run at once and a block's
+// pipeline and halo cost `halo` plane steps: the chunk that makes the rounds
+// of blocks, each zc + halo steps, cheapest -- the mean of whole rounds (a
+// last round that is nearly empty costs like a full one while its blocks
+// wait on their own chains) and of the blocks' share (bandwidth).  Against
+// timing every chunk of {2, 4, 8, ... 64} on 43 level shapes from 24^3 to
+// 512^3, this picks within 0 to 3% of the fastest on average, and it is free
+// to take a chunk between them: 256 x 160 x 256 cells run 245 two-sweep
+// blocks of 38 planes instead of 210 of 48.
+int march_zc(int nz, long tiles, long slots, int halo) {
+    int best = nz;
+    double cost = 1e300;
+    for (int chunks = 1; chunks <= nz; ++chunks) {
+        const int zc = std::min(nz, (((nz + chunks - 1) / chunks) + 1) & ~1);  // even
+        if (zc > 64 && tiles > slots / 4) continue;  // longer only to cut the halo of few columns
+        const long blocks = tiles * ((nz + zc - 1) / zc);
+        const double share = (double)blocks / slots;
+        const double c = 0.5 * (std::ceil(share) + share) * (zc + halo);
+        if (c < cost) {
+            cost = c;
+            best = zc;
+        }
+        if (zc <= 2) break;
+    }
+    return best;
 }
 
-// JG_TUNE_LOG=1 prints every autotuner timing to stderr.
-bool tune_log() {
-    static const bool on = [] {
-        const char* e = std::getenv("JG_TUNE_LOG");
-        return e && *e && *e != '0';
-    }();
-    return on;
-}
-
-int sweep_zc(const Dims& d, int tuned) {
-    if (sweep_zc_env() > 0) return std::min(sweep_zc_env(), d.nz);
-    if (tuned > 0) return std::min(tuned, d.nz);
+int sweep_zc(const jg_solver* s, const Dims& d) {
     const long tiles = (long)((d.nx + kSwIX - 1) / kSwIX) * ((d.ny + kSwIY - 1) / kSwIY);
-    const long gz = std::max<long>(1, (1024 + tiles - 1) / tiles);
-    long zc = (d.nz + gz - 1) / gz;
-    zc = std::max<long>(8, std::min<long>(64, zc));
-    return (int)std::min<long>(zc, d.nz);
+    return march_zc(d.nz, tiles * s->nsys, s->cus, 3);
 }
 
 // Grids of a launch over every system of s (one, or a batch group): the
@@ -115,20 +120,27 @@ inline dim3 grid_1d(int nb, const jg_solver* s) { return dim3((unsigned)nb, (uns
 // One fused red-black sweep (see jg_sweep.h).  first: colour updated first
 // (0 = red, forward; 1 = black, backward).  xin == nullptr: x starts at zero.
 // coarse != nullptr: add the prolongation of coarse to x on load.
-// p_bx/p_bb != nullptr: emit b.x and b.b partials.  shape: index into
-// kSweepShapes.  Returns the number of b.x / b.b partials written (the
-// block count; 0 without partials, or when the grid has more blocks than a
-// slot holds -- the caller then reduces with k_dot).
-template <typename T, int RP, int PD>
-void launch_sweep_shape(jg_solver* s, int code, dim3 grid, const Row<T>* A, const T* b,
-                        const T* xin, T* xout, const Dims& d, int zc, T omega, const T* coarse,
-                        double* p_bx, double* p_bb, const Ctl* ctl) {
-    const dim3 block(kSwLX, kSwLY / RP, 1);
-#define JG_SWEEP_CASE(C, F, Z, K, D)                                                            \
-    case C:                                                                                     \
-        k_rb_sweep<T, F, Z, K, D, RP, PD><<<grid, block, 0, s->stream>>>(A, b, xin, xout, d, zc, \
-                                                                       omega, coarse, p_bx,    \
-                                                                       p_bb, ctl);             \
+// p_bx/p_bb != nullptr: emit b.x and b.b partials.  Returns the number of
+// b.x / b.b partials written (the block count; 0 without partials, or when
+// the grid has more blocks than a slot holds -- the caller then reduces with
+// k_dot).
+template <typename T>
+int launch_sweep(jg_solver* s, const Row<T>* A, const T* b, const T* xin, T* xout, const Dims& d,
+                 int first, const T* coarse, double* p_bx, double* p_bb, T omega, const Ctl* ctl) {
+    int zc = sweep_zc(s, d);
+    const long cols = (long)((d.nx + kSwIX - 1) / kSwIX) * ((d.ny + kSwIY - 1) / kSwIY);
+    // one b.x / b.b partial per block: keep the block count within a slot
+    while (p_bx && zc < d.nz && cols * ((d.nz + zc - 1) / zc) > kMaxPartials) ++zc;
+    dim3 grid((d.nx + kSwIX - 1) / kSwIX, (d.ny + kSwIY - 1) / kSwIY, (d.nz + zc - 1) / zc);
+    if ((long)grid.x * grid.y * grid.z > kMaxPartials) p_bx = p_bb = nullptr;  // caller uses k_dot
+    const int nb = (int)(grid.x * grid.y * grid.z);  // per system
+    grid = grid_sys(grid, s);
+    const int code = (first ? 8 : 0) | (xin ? 0 : 4) | (coarse ? 2 : 0) | (p_bx ? 1 : 0);
+    const dim3 block(kSwLX, kSwLY, 1);
+#define JG_SWEEP_CASE(C, F, Z, K, D)                                                              \
+    case C:                                                                                       \
+        k_rb_sweep<T, F, Z, K, D><<<grid, block, 0, s->stream>>>(A, b, xin, xout, d, zc, omega,   \
+                                                                 coarse, p_bx, p_bb, ctl);        \
         break;
     switch (code) {
         JG_SWEEP_CASE(0, 0, false, false, false)
@@ -149,38 +161,6 @@ void launch_sweep_shape(jg_solver* s, int code, dim3 grid, const Row<T>* A, cons
         JG_SWEEP_CASE(15, 1, true, true, true)
     }
 #undef JG_SWEEP_CASE
-}
-
-template <typename T>
-int launch_sweep(jg_solver* s, const Row<T>* A, const T* b, const T* xin, T* xout, const Dims& d,
-                 int first, const T* coarse, double* p_bx, double* p_bb, T omega, const Ctl* ctl,
-                 int tuned_zc = 0, int shape = 0) {
-    int zc = sweep_zc(d, tuned_zc);
-    const long cols = (long)((d.nx + kSwIX - 1) / kSwIX) * ((d.ny + kSwIY - 1) / kSwIY);
-    // one b.x / b.b partial per block: keep the block count within a slot
-    while (p_bx && zc < d.nz && cols * ((d.nz + zc - 1) / zc) > kMaxPartials) ++zc;
-    dim3 grid((d.nx + kSwIX - 1) / kSwIX, (d.ny + kSwIY - 1) / kSwIY, (d.nz + zc - 1) / zc);
-    if ((long)grid.x * grid.y * grid.z > kMaxPartials) p_bx = p_bb = nullptr;  // caller uses k_dot
-    const int nb = (int)(grid.x * grid.y * grid.z);  // per system
-    grid = grid_sys(grid, s);
-    const int code = (first ? 8 : 0) | (xin ? 0 : 4) | (coarse ? 2 : 0) | (p_bx ? 1 : 0);
-    switch (shape) {
-        case 1:
-            launch_sweep_shape<T, 2, 2>(s, code, grid, A, b, xin, xout, d, zc, omega, coarse, p_bx,
-                                        p_bb, ctl);
-            break;
-        case 2:
-            launch_sweep_shape<T, 1, 1>(s, code, grid, A, b, xin, xout, d, zc, omega, coarse, p_bx,
-                                        p_bb, ctl);
-            break;
-        case 3:
-            launch_sweep_shape<T, 1, 2>(s, code, grid, A, b, xin, xout, d, zc, omega, coarse, p_bx,
-                                        p_bb, ctl);
-            break;
-        default:
-            launch_sweep_shape<T, 2, 1>(s, code, grid, A, b, xin, xout, d, zc, omega, coarse, p_bx,
-                                        p_bb, ctl);
-    }
     return p_bx ? nb : 0;
 }
 
@@ -190,12 +170,11 @@ int launch_sweep(jg_solver* s, const Row<T>* A, const T* b, const T* xin, T* xou
 // a coarse correction.
 template <typename T>
 int launch_sweep2(jg_solver* s, const Row<T>* A, const T* b, const T* xin, T* xout, const Dims& d,
-                  int first, const T* coarse, T* res, T omega, const Ctl* ctl, int tuned_zc) {
+                  int first, const T* coarse, T* res, T omega, const Ctl* ctl) {
     if constexpr (sizeof(T) != 4) {
         return JG_ERR_UNSUPPORTED;
     } else {
         if (res && coarse) return JG_ERR_UNSUPPORTED;
-        const int zc = std::min(tuned_zc > 0 ? tuned_zc : 32, d.nz);
         // the tile of a zero-start launch without a correction has a one cell
         // narrower halo (jg_sweep2.h)
         const bool z = !xin && !coarse;
@@ -203,6 +182,9 @@ int launch_sweep2(jg_solver* s, const Row<T>* A, const T* b, const T* xin, T* xo
                            : (z ? S2Tile<false, true>::IX : S2Tile<false>::IX);
         const int iy = res ? (z ? S2Tile<true, true>::IY : S2Tile<true>::IY)
                            : (z ? S2Tile<false, true>::IY : S2Tile<false>::IY);
+        // one block per CU; a chunk adds 8 planes of halo, some of them cheap
+        const long tiles = (long)((d.nx + ix - 1) / ix) * ((d.ny + iy - 1) / iy) * s->nsys;
+        const int zc = march_zc(d.nz, tiles, s->cus, 6);
         const dim3 grid = grid_sys(dim3((d.nx + ix - 1) / ix, (d.ny + iy - 1) / iy, (d.nz + zc - 1) / zc), s);
         const dim3 block(kS2LX, kS2TY, 1);
         const int code = (first ? 8 : 0) | (xin ? 0 : 4) | (coarse ? 2 : 0) | (res ? 1 : 0);
@@ -262,24 +244,39 @@ constexpr idx_t kBrickMaxCells = idx_t(1) << 21;
 
 // Sweeps of one smoothing step, grouped into launches: 1 = one sweep,
 // kLaunchMarch / kLaunchBrick = two sweeps in one launch of k_rb_sweep2 /
-// k_brick_sweep2, where the tuner found that faster for the kind of the
-// launch's first sweep (kind_first for the first launch, plain afterwards).
+// k_brick_sweep2.  A brick launch costs by its bricks (FP32 12.5 ns, FP64
+// 26 ns each once the chip is full), the marching ones a chain of planes
+// that no small grid shortens.  Measured pairs of plain sweeps, us, as two
+// launches / march / bricks:
+//   FP32  64^3 (512 bricks) 20 / 25 / 8.6   128x48x128 (1536) 26 / 26 / 22
+//         112x64x144 (2016) 26 / 26 / 28    128^3 (4096)      45 / 34 / 51
+//   FP64  64^3 (512) 24 / - / 12   80x48x80 (600) 24 / - / 22
+//         96x80x72 (1080) 25 / - / 30
+// and a march launch also writes the residual for the restriction.  So:
+// bricks up to 1536 (FP32) or 768 (FP64) over all systems; above, march in
+// FP32 (a single system or a group) and single sweeps in FP64.
 // pairs > 0 forces two-sweep launches wherever two sweeps follow (FP32:
 // bricks up to 2^18 cells, else the z-marching kernel; FP64: bricks up to
 // kBrickMaxCells cells), pairs < 0 forbids them.
 constexpr int kLaunchSingle = 1, kLaunchMarch = 2, kLaunchBrick = 3;
 template <typename T>
-std::vector<int> sweep_plan(const Level& lv, unsigned n, int kind_first, int pairs) {
+std::vector<int> sweep_plan(const jg_solver* s, const Dims& d, unsigned n, int pairs) {
+    const long bricks = (long)((d.nx + kBkB - 1) / kBkB) * ((d.ny + kBkB - 1) / kBkB) *
+                        ((d.nz + kBkB - 1) / kBkB) * s->nsys;
+    int two;
+    if (pairs > 0)  // FP32: bricks up to 64^3 cells, the z-marching kernel above
+        two = sizeof(T) == 4 ? (d.n() <= (idx_t(1) << 18) ? kLaunchBrick : kLaunchMarch)
+                             : (d.n() <= kBrickMaxCells ? kLaunchBrick : kLaunchSingle);
+    else if (sizeof(T) == 4)
+        two = bricks <= 1536 ? kLaunchBrick : kLaunchMarch;
+    else
+        two = bricks <= 768 ? kLaunchBrick : kLaunchSingle;
+    if (pairs < 0 || s->twod || d.n() <= BotCfg<T>::MaxCells) two = kLaunchSingle;
     std::vector<int> v;
-    const bool big = lv.d.n() > BotCfg<T>::MaxCells;
     for (unsigned k = 0; k < n;) {
-        int mode = Prec<T>::pair(lv, k == 0 ? kind_first : kSweepPlain);
-        if (pairs > 0)  // FP32: bricks up to 64^3 cells, the z-marching kernel above
-            mode = sizeof(T) == 4 ? (lv.d.n() <= (idx_t(1) << 18) ? kPairBrick : kPairMarch)
-                                  : (lv.d.n() <= kBrickMaxCells ? kPairBrick : kPairNone);
-        if (pairs < 0 || !big || n - k < 2) mode = kPairNone;
-        v.push_back(mode == kPairBrick ? kLaunchBrick : mode == kPairMarch ? kLaunchMarch : kLaunchSingle);
-        k += mode == kPairNone ? 1 : 2;
+        const int mode = n - k < 2 ? kLaunchSingle : two;
+        v.push_back(mode);
+        k += mode == kLaunchSingle ? 1 : 2;
     }
     return v;
 }
@@ -653,9 +650,8 @@ int vcycle(jg_solver* s, const T* r0, T* z0, const MgCfg<T>& c, const Ctl* ctl, 
             const T* in = nullptr;
             for (int k = 0; k < S; ++k) {
                 T* out = ((S - 1 - k) % 2 == 0) ? X(l) : Y;
-                const int kind = in ? kSweepPlain : kSweepZero;
                 launch_sweep<T>(s, A, B(l), in, out, d, k < fwd ? 0 : 1, nullptr, nullptr, nullptr,
-                                c.omega, ctl, Prec<T>::zc(lv, kind), Prec<T>::sh(lv, kind));
+                                c.omega, ctl);
                 in = out;
             }
             JG_TRY(check_launch(s, "coarsest"));
@@ -664,24 +660,20 @@ int vcycle(jg_solver* s, const T* r0, T* z0, const MgCfg<T>& c, const Ctl* ctl, 
         }
         const unsigned post = l == 0 ? c.post0 : c.post;
         // launches of the level ping-pong between x and y so the last lands in x
-        const std::vector<int> pre_plan = sweep_plan<T>(lv, c.pre, kSweepZero, c.pairs);
-        const size_t M = pre_plan.size() + sweep_plan<T>(lv, post, kSweepCorrect, c.pairs).size();
+        const std::vector<int> pre_plan = sweep_plan<T>(s, d, c.pre, c.pairs);
+        const size_t M = pre_plan.size() + sweep_plan<T>(s, d, post, c.pairs).size();
         auto buf = [&](size_t m) -> T* { return ((M - 1 - m) % 2 == 0) ? X(l) : Y; };
         const T* in = nullptr;
         for (size_t m = 0; m < pre_plan.size(); ++m) {
-            const int kind = in ? kSweepPlain : kSweepZero;
             if (pre_plan[m] == kLaunchBrick)
                 launch_brick2<T>(s, A, B(l), in, buf(m), d, 0, nullptr, c.omega, ctl);
             else if (pre_plan[m] == kLaunchMarch) {
                 const bool res = m + 1 == pre_plan.size();
                 JG_TRY(launch_sweep2<T>(s, A, B(l), in, buf(m), d, 0, nullptr,
-                                        res ? Prec<T>::t(lv) : nullptr, c.omega, ctl,
-                                        res && kind == kSweepZero ? Prec<T>::zc2res(lv)
-                                                                  : Prec<T>::zc2(lv, kind)));
+                                        res ? Prec<T>::t(lv) : nullptr, c.omega, ctl));
             }
             else
-                launch_sweep<T>(s, A, B(l), in, buf(m), d, 0, nullptr, nullptr, nullptr, c.omega, ctl,
-                                Prec<T>::zc(lv, kind), Prec<T>::sh(lv, kind));
+                launch_sweep<T>(s, A, B(l), in, buf(m), d, 0, nullptr, nullptr, nullptr, c.omega, ctl);
             in = buf(m);
         }
         pre_out[l] = in;  // nullptr: x is still zero
@@ -719,8 +711,8 @@ int vcycle(jg_solver* s, const T* r0, T* z0, const MgCfg<T>& c, const Ctl* ctl, 
         const Dims& d = lv.d;
         T* Y = Prec<T>::y(lv);
         const unsigned post = l == 0 ? c.post0 : c.post;
-        const size_t P0 = sweep_plan<T>(lv, c.pre, kSweepZero, c.pairs).size();
-        const std::vector<int> post_plan = sweep_plan<T>(lv, post, kSweepCorrect, c.pairs);
+        const size_t P0 = sweep_plan<T>(s, d, c.pre, c.pairs).size();
+        const std::vector<int> post_plan = sweep_plan<T>(s, d, post, c.pairs);
         const size_t M = P0 + post_plan.size();
         auto buf = [&](size_t m) -> T* { return ((M - 1 - m) % 2 == 0) ? X(l) : Y; };
         const T* coarse = X(l + 1);
@@ -734,7 +726,6 @@ int vcycle(jg_solver* s, const T* r0, T* z0, const MgCfg<T>& c, const Ctl* ctl, 
             for (size_t q = 0; q < post_plan.size(); ++q) {
                 const size_t m = P0 + q;
                 const bool last0 = (l == 0 && m + 1 == M);
-                const int kind = q == 0 ? kSweepCorrect : kSweepPlain;
                 const T* cor = q == 0 ? coarse : nullptr;
                 // the two-sweep kernel leaves r.z / r.r to one fused dot kernel
                 // (accumulating them in it costs more than that pass)
@@ -745,11 +736,9 @@ int vcycle(jg_solver* s, const T* r0, T* z0, const MgCfg<T>& c, const Ctl* ctl, 
                 if (post_plan[q] == kLaunchBrick)
                     launch_brick2<T>(s, A, B(l), in, buf(m), d, 1, cor, c.omega, ctl);
                 else if (post_plan[q] == kLaunchMarch)
-                    JG_TRY(launch_sweep2<T>(s, A, B(l), in, buf(m), d, 1, cor, nullptr, c.omega,
-                                            ctl, Prec<T>::zc2(lv, kind)));
+                    JG_TRY(launch_sweep2<T>(s, A, B(l), in, buf(m), d, 1, cor, nullptr, c.omega, ctl));
                 else
-                    nb = launch_sweep<T>(s, A, B(l), in, buf(m), d, 1, cor, pbx, pbb, c.omega, ctl,
-                                         Prec<T>::zc(lv, kind), Prec<T>::sh(lv, kind));
+                    nb = launch_sweep<T>(s, A, B(l), in, buf(m), d, 1, cor, pbx, pbb, c.omega, ctl);
                 if (dot) *dot_blocks = nb;
                 in = buf(m);
             }
@@ -757,161 +746,6 @@ int vcycle(jg_solver* s, const T* r0, T* z0, const MgCfg<T>& c, const Ctl* ctl, 
         JG_TRY(check_launch(s, "vcycle up"));
     }
     return JG_OK;
-}
-
-// Launch-shape and z-chunk autotuner of the fused sweep: times each
-// candidate on the level with the level's own matrix and scratch vectors,
-// separately for the three sweep kinds (plain, zero initial x, fused
-// correction), which differ in loads and registers.  Runs once per hierarchy
-// and precision, before a solve, so nothing live is overwritten.
-template <typename T>
-int autotune_sweeps(jg_solver* s) {
-    if (sweep_zc_env() > 0) return JG_OK;
-    const size_t L = s->lv.size();
-    for (size_t l = 0; l < L; ++l) {
-        Level& lv = s->lv[l];
-        if (Prec<T>::zc(lv) > 0) continue;
-        const Dims& d = lv.d;
-        if (d.n() <= BotCfg<T>::MaxCells) {  // handled by k_bottom
-            for (int kind = 0; kind < kNumSweepKinds; ++kind) Prec<T>::zc(lv, kind) = sweep_zc(d, 0);
-            continue;
-        }
-        const idx_t n = d.n();
-        k_fill<T><<<grid_1d(nblocks_1d(n), s), NT, 0, s->stream>>>(Prec<T>::t(lv), T(1), n);
-        k_fill<T><<<grid_1d(nblocks_1d(n), s), NT, 0, s->stream>>>(Prec<T>::y(lv), T(0.5), n);
-        // the correction kind reads the next level's x as its coarse vector
-        // (a 2-D hierarchy corrects in a separate launch: no correction kind)
-        const T* coarse = nullptr;
-        if (l + 1 < L && !s->twod) {
-            const idx_t cn = s->lv[l + 1].d.n();
-            coarse = Prec<T>::x(s->lv[l + 1]);
-            k_fill<T><<<grid_1d(nblocks_1d(cn), s), NT, 0, s->stream>>>(Prec<T>::x(s->lv[l + 1]), T(0.25), cn);
-        }
-        const int cands[] = {2, 4, 8, 12, 16, 24, 32, 48, 64};
-        float tbest[kNumSweepKinds] = {1e30f, 1e30f, 1e30f};
-        for (int kind = 0; kind < kNumSweepKinds; ++kind) {
-            if (kind == kSweepCorrect && !coarse) {
-                Prec<T>::zc(lv, kind) = Prec<T>::zc(lv, kSweepPlain);
-                Prec<T>::sh(lv, kind) = Prec<T>::sh(lv, kSweepPlain);
-                continue;
-            }
-            float best = 1e30f;
-            int best_zc = sweep_zc(d, 0), best_sh = 0;
-            for (int sh = 0; sh < kNumSweepShapes; ++sh) {
-                for (int zc : cands) {
-                    if (zc > d.nz) break;
-                    auto run = [&]() {
-                        launch_sweep<T>(s, Prec<T>::A(lv), Prec<T>::t(lv),
-                                        kind == kSweepZero ? nullptr : Prec<T>::y(lv), Prec<T>::x(lv),
-                                        d, 1, kind == kSweepCorrect ? coarse : nullptr, nullptr,
-                                        nullptr, T(1), nullptr, zc, sh);
-                    };
-                    run();
-                    JG_HIP(hipEventRecord(s->ev0, s->stream));
-                    for (int r = 0; r < 3; ++r) run();
-                    JG_HIP(hipEventRecord(s->ev1, s->stream));
-                    JG_TRY(sync(s));
-                    float ms = 0.f;
-                    JG_HIP(hipEventElapsedTime(&ms, s->ev0, s->ev1));
-                    if (tune_log())
-                        std::fprintf(stderr,
-                                     "jetgpu tune: %dx%dx%d %s kind %d shape %d (rp %d pd %d) zc %d: %.1f us\n",
-                                     d.nx, d.ny, d.nz, sizeof(T) == 4 ? "f32" : "f64", kind, sh,
-                                     kSweepShapes[sh].rp, kSweepShapes[sh].pd, zc, ms * 1e3f / 3);
-                    if (ms < best) {
-                        best = ms;
-                        best_zc = zc;
-                        best_sh = sh;
-                    }
-                }
-            }
-            Prec<T>::sh(lv, kind) = best_sh;
-            Prec<T>::zc(lv, kind) = best_zc;
-            tbest[kind] = best;
-        }
-        // Two sweeps per launch: one launch replaces a sweep of this kind
-        // followed by a plain sweep, when it is faster than that pair.
-        auto time3 = [&](auto&& run) -> float {
-            run();
-            float ms = 0.f;
-            if (hipEventRecord(s->ev0, s->stream) != hipSuccess) return -1.f;
-            for (int r = 0; r < 3; ++r) run();
-            if (hipEventRecord(s->ev1, s->stream) != hipSuccess || sync(s) != JG_OK ||
-                hipEventElapsedTime(&ms, s->ev0, s->ev1) != hipSuccess)
-                return -1.f;
-            return ms;
-        };
-        for (int kind = 0; kind < kNumSweepKinds; ++kind) {
-            Prec<T>::pair(lv, kind) = kPairNone;
-            if (s->twod) continue;  // the 2-D cycle launches single sweeps
-            if (kind == kSweepCorrect && !coarse) continue;
-            const T* xin = kind == kSweepZero ? nullptr : Prec<T>::y(lv);
-            const T* cor = kind == kSweepCorrect ? coarse : nullptr;
-            float best = tbest[kind] + tbest[kSweepPlain];
-            if constexpr (sizeof(T) == 4) {
-                const int cands2[] = {8, 12, 16, 24, 32, 48, 64};
-                float best2 = 1e30f;
-                int best_zc = 32;
-                for (int zc : cands2) {
-                    if (zc > d.nz && zc != cands2[0]) break;
-                    const float ms = time3([&]() {
-                        launch_sweep2<T>(s, Prec<T>::A(lv), Prec<T>::t(lv), xin, Prec<T>::x(lv), d, 1,
-                                         cor, nullptr, T(1), nullptr, zc);
-                    });
-                    if (ms < 0.f) return JG_ERR_HIP;
-                    if (tune_log())
-                        std::fprintf(stderr, "jetgpu tune: %dx%dx%d f32 kind %d two-sweep zc %d: %.1f us\n",
-                                     d.nx, d.ny, d.nz, kind, zc, ms * 1e3f / 3);
-                    if (ms < best2) {
-                        best2 = ms;
-                        best_zc = zc;
-                    }
-                }
-                lv.zc2_32[kind] = best_zc;
-                if (best2 < best) {
-                    best = best2;
-                    Prec<T>::pair(lv, kind) = kPairMarch;
-                }
-                if (kind == kSweepZero) {
-                    // the residual-writing form of the zero-start launch (the
-                    // last pre-smoothing launch of a level), residual into y
-                    float best3 = 1e30f;
-                    for (int zc : cands2) {
-                        if (zc > d.nz && zc != cands2[0]) break;
-                        const float ms = time3([&]() {
-                            launch_sweep2<T>(s, Prec<T>::A(lv), Prec<T>::t(lv), nullptr,
-                                             Prec<T>::x(lv), d, 0, nullptr, Prec<T>::y(lv), T(1),
-                                             nullptr, zc);
-                        });
-                        if (ms < 0.f) return JG_ERR_HIP;
-                        if (tune_log())
-                            std::fprintf(stderr,
-                                         "jetgpu tune: %dx%dx%d f32 two-sweep with residual zc %d: %.1f us\n",
-                                         d.nx, d.ny, d.nz, zc, ms * 1e3f / 3);
-                        if (ms < best3) {
-                            best3 = ms;
-                            lv.zc2res_32 = zc;
-                        }
-                    }
-                }
-            }
-            if (d.n() <= kBrickMaxCells) {
-                const float ms = time3([&]() {
-                    launch_brick2<T>(s, Prec<T>::A(lv), Prec<T>::t(lv), xin, Prec<T>::x(lv), d, 1, cor,
-                                     T(1), nullptr);
-                });
-                if (ms < 0.f) return JG_ERR_HIP;
-                if (tune_log())
-                    std::fprintf(stderr, "jetgpu tune: %dx%dx%d %s kind %d brick: %.1f us\n", d.nx, d.ny,
-                                 d.nz, sizeof(T) == 4 ? "f32" : "f64", kind, ms * 1e3f / 3);
-                if (ms < best) {
-                    best = ms;
-                    Prec<T>::pair(lv, kind) = kPairBrick;
-                }
-            }
-        }
-    }
-    return check_launch(s, "autotune");
 }
 
 // --------------------------------------------------------------- PCG
@@ -1488,6 +1322,302 @@ void make_view(jg_solver* g, int i, jg_solver* v) {
 
 }  // namespace
 
+namespace {
+
+// jg_solver_cg on s's arrays (the grid's, or a box's); ev0 is recorded.
+int cg_run(jg_solver* s, unsigned max_iter, double tol, jg_solve_info* info,
+           const std::function<int()>& finish) {
+    Level& l0 = s->lv[0];
+    Ctl h;
+    init_ctl(&h, max_iter, tol, 0, 0.0);
+    JG_TRY(upload_ctl(s, s->ctl, h));
+    k_fill<double><<<nblocks_1d(l0.d.n()), NT, 0, s->stream>>>(s->x, 0.0, l0.d.n());
+    JG_TRY(pcg_device<double>(s, Pcg<double>{l0.A64, s->b, s->x, s->r, s->r, s->dA, s->dB, s->q, l0.d,
+                                              s->ctl, nullptr},
+                              1));
+    JG_TRY(finish());
+    JG_HIP(hipEventRecord(s->ev1, s->stream));
+    JG_HIP(hipMemcpyAsync(s->ctl_host, s->ctl, sizeof(Ctl), hipMemcpyDeviceToHost, s->stream));
+    JG_TRY(sync(s));
+    const Ctl& c = *s->ctl_host;
+    const bool nonfinite = c.nonfinite != 0;
+    if (info) {
+        std::memset(info, 0, sizeof(*info));
+        float ms = 0.f;
+        JG_HIP(hipEventElapsedTime(&ms, s->ev0, s->ev1));
+        info->solve_ms = ms;
+        info->iterations = c.iter;
+        info->last_residual = std::sqrt(std::fabs(c.sigma));
+        // FdmCgSolver3::solve's return (src/jet/fdm_cg_solver3.cpp:45-46)
+        info->converged = (info->last_residual <= tol) || (c.iter < max_iter);
+        JG_TRY(true_rel_residual(s, &info->rel_residual));
+    }
+    if (nonfinite) {
+        s->err = "non-finite value in CG reduction";
+        return JG_ERR_NONFINITE;
+    }
+    return JG_OK;
+}
+
+// jg_solver_mgpcg on s's arrays (the grid's, or a box's); ev0 is recorded.
+int mgpcg_run(jg_solver* s, unsigned max_iter, const jg_mg_params* p, const jg_gpu_options& opt,
+              double omega, jg_solve_info* info, const std::function<int()>& finish) {
+    Level& l0 = s->lv[0];
+    const idx_t n = l0.d.n();
+    int status = JG_OK;
+    unsigned iters = 0, refinements = 0;
+    double last_res = 0.0;
+    double bnorm = 0.0;  // mixed: ||b||, for the relative residual of the final x
+    double mixed_goal = -1.0;  // mixed: the FP64 residual norm the refinement had to reach
+    Ctl* ctl = s->ctl;
+    if (opt.precision == JG_MIXED) JG_TRY(ensure_f32(s));
+    k_fill<double><<<nblocks_1d(n), NT, 0, s->stream>>>(s->x, 0.0, n);
+    if (opt.precision != JG_MIXED) {
+        MgCfg<double> mg{p->restrict_iter, p->final_iter, p->correct_iter, p->coarsest_iter, omega};
+        mg.pairs = opt.sweep_pairs;
+        mg.jacobi = opt.smoother == JG_SMOOTH_JACOBI;
+        Ctl h;
+        init_ctl(&h, max_iter, p->max_tol, opt.stop_rule == JG_STOP_RELATIVE ? 1 : 0, opt.rel_tol);
+        JG_TRY(upload_ctl(s, ctl, h));
+        JG_TRY(pcg_device<double>(s, Pcg<double>{l0.A64, s->b, s->x, s->r, s->z, s->dA, s->dB, s->q,
+                                                  l0.d, ctl, &mg},
+                                  opt.check_every));
+        JG_HIP(hipMemcpyAsync(s->ctl_host, ctl, sizeof(Ctl), hipMemcpyDeviceToHost, s->stream));
+        JG_TRY(sync(s));
+        iters = s->ctl_host->iter;
+        last_res = std::sqrt(std::fabs(s->ctl_host->sigma));
+        if (s->ctl_host->nonfinite) status = JG_ERR_NONFINITE;
+    } else {
+        // Iterative refinement: FP64 residual and correction, FP32 MGPCG
+        // (FP32 stencil, smoother and V-cycle; FP64 dot accumulation).
+        MgCfg<float> mg{p->restrict_iter, p->final_iter, p->correct_iter, p->coarsest_iter,
+                        (float)omega};
+        mg.pairs = opt.sweep_pairs;
+        mg.jacobi = opt.smoother == JG_SMOOTH_JACOBI;
+        const int nb1 = nblocks_1d(n);
+        k_dot<double, double><<<nb1, NT, 0, s->stream>>>(s->b, s->b, n, s->slot(3), nullptr);
+        k_fin_sum<<<1, kFinThreads, 0, s->stream>>>(s->slot(3), nb1, s->scal + 2);
+        double bb = 0.0;
+        JG_HIP(hipMemcpyAsync(&bb, s->scal + 2, sizeof(double), hipMemcpyDeviceToHost, s->stream));
+        JG_TRY(sync(s));
+        bnorm = std::sqrt(bb);
+        const double goal = opt.stop_rule == JG_STOP_RELATIVE ? opt.rel_tol * bnorm : p->max_tol;
+        Ctl* ictl = s->ctl + 1;
+        for (unsigned outer = 0;; ++outer) {
+            double rr = 0.0;
+            if (outer == 0) {
+                // x = 0: b - A x is b itself (bit for bit), and its norm is known
+                k_convert<double, float><<<nb1, NT, 0, s->stream>>>(s->b, s->rhs32, n);
+                rr = bb;
+            } else {
+                const int nr = residual_dot64<float>(s, l0, s->rhs32, s->slot(3));
+                k_fin_sum<<<1, kFinThreads, 0, s->stream>>>(s->slot(3), nr, s->scal + 3);
+                JG_HIP(hipMemcpyAsync(&rr, s->scal + 3, sizeof(double), hipMemcpyDeviceToHost,
+                                      s->stream));
+                JG_TRY(sync(s));
+            }
+            last_res = std::sqrt(rr);
+            if (!std::isfinite(rr)) {
+                status = JG_ERR_NONFINITE;
+                break;
+            }
+            if (last_res <= goal || outer >= opt.max_refine || iters >= max_iter) break;
+            Ctl h;
+            // The last refinement only needs to close the remaining gap to
+            // the goal (with a factor 2 margin for the FP32 inner residual).
+            const double inner = std::max(opt.inner_rel_tol, std::min(0.5, 0.5 * goal / last_res));
+            init_ctl(&h, max_iter - iters, 0.0, 1, inner);
+            JG_TRY(upload_ctl(s, ictl, h));
+            k_fill<float><<<nb1, NT, 0, s->stream>>>(s->e32, 0.f, n);
+            JG_TRY(pcg_device<float>(s, Pcg<float>{l0.A32, s->rhs32, s->e32, s->r32, s->z32, s->d32A,
+                                                   s->d32B, s->q32, l0.d, ictl, &mg},
+                                     opt.check_every));
+            iters += s->ctl_host->iter;
+            if (s->ctl_host->nonfinite) {
+                // a value beyond FP32 range (or a NaN) in the inner solve: the
+                // correction is meaningless, and x keeps the last finite one
+                status = JG_ERR_NONFINITE;
+                break;
+            }
+            k_add_correction<<<nb1, NT, 0, s->stream>>>(s->x, s->e32, n);
+            JG_TRY(check_launch(s, "refinement"));
+            ++refinements;
+        }
+        mixed_goal = goal;
+    }
+    JG_TRY(finish());
+    JG_HIP(hipEventRecord(s->ev1, s->stream));
+    JG_TRY(sync(s));
+    if (info) {
+        std::memset(info, 0, sizeof(*info));
+        float ms = 0.f;
+        JG_HIP(hipEventElapsedTime(&ms, s->ev0, s->ev1));
+        info->solve_ms = ms;
+        info->iterations = iters;
+        info->refinements = refinements;
+        info->last_residual = last_res;
+        // FP64: Jet's rule (cg-inl.h:93 and fdm_mgpcg_solver3.cpp:78). Mixed: the
+        // outer loop stops on the true residual, so converged means it reached
+        // the goal; running out of refinements or iterations above it is not.
+        info->converged = opt.precision == JG_MIXED ? last_res <= mixed_goal
+                                                    : (last_res <= p->max_tol) || (iters < max_iter);
+        if (status != JG_OK) info->converged = 0;
+        if (opt.precision == JG_MIXED && bnorm > 0.0)
+            info->rel_residual = last_res / bnorm;  // the FP64 b - A x of the final x
+        else
+            JG_TRY(true_rel_residual(s, &info->rel_residual));
+        if (opt.stop_rule == JG_STOP_RELATIVE && status == JG_OK)
+            info->converged = info->rel_residual <= opt.rel_tol;
+    }
+    if (status == JG_ERR_NONFINITE) s->err = "non-finite value in MGPCG reduction";
+    return status;
+}
+
+// ------------------------------------------------ solves in a box (jg_box.h)
+
+// Grids from which a solve looks for its box: below, the scan's launches
+// and its wait (about 30 us) outweigh the cells it could leave out.
+constexpr idx_t kBoxMgCells = (idx_t(1) << 18) + 1, kBoxCgCells = idx_t(1) << 16;
+// A box of more than this share of the grid is not worth its copy.
+constexpr double kBoxShare = 0.85;
+
+// The box of the cells that take part in a solve of s's resident system,
+// aligned to the coarsest of L levels; share of the grid's cells in *share.
+int find_box(jg_solver* s, size_t L, double most, Box* box, double* share) {
+    const Level& l0 = s->lv[0];
+    const Dims& d = l0.d;
+    if (!s->box_scan) JG_TRY(dalloc(s, &s->box_scan, 2));
+    k_box_reset<<<1, 64, 0, s->stream>>>(s->box_scan);
+    const unsigned gx = (d.nx + 63) / 64;
+    const unsigned sy = (d.ny + 8 * kBoxY - 1) / (8 * kBoxY), sz = (d.nz + 7) / 8;
+    k_box_scan<true><<<dim3(gx, sy, sz), 64 * kBoxY, 0, s->stream>>>(l0.A64, s->b, d, most, s->box_scan);
+    const dim3 grid(gx, (d.ny + kBoxY - 1) / kBoxY, (d.nz + kBoxZ - 1) / kBoxZ);
+    k_box_scan<false><<<grid, 64 * kBoxY, 0, s->stream>>>(l0.A64, s->b, d, most, s->box_scan);
+    JG_TRY(check_launch(s, "box scan"));
+    JG_HIP(hipMemcpyAsync(s->box_host, s->box_scan, sizeof(BoxScan), hipMemcpyDeviceToHost, s->stream));
+    JG_TRY(sync(s));
+    const BoxScan r = *s->box_host;
+    const int dims[3] = {d.nx, d.ny, d.nz};
+    int n[3];
+    for (int a = 0; a < 3; ++a) {
+        const int g = a == 2 && s->twod ? 1 : 1 << (L - 1);
+        const int lo = std::max(0, std::min(r.lo[a], dims[a])), hi = std::max(0, std::min(r.hi[a] + 1, dims[a]));
+        box->o[a] = lo / g * g;
+        n[a] = std::max(0, (hi + g - 1) / g * g - box->o[a]);
+    }
+    box->n = Dims{n[0], n[1], n[2]};
+    *share = (double)box->n.n() / (double)d.n();
+    return JG_OK;
+}
+
+// The arrays of box solves: rows of every level, b and x, for boxes of up to
+// kBoxShare of the grid; kept until the hierarchy changes.  false: no room.
+bool box_reserve(jg_solver* s, size_t L) {
+    if (s->box_cells > 0 || s->box_failed) return !s->box_failed;
+    size_t cells = 0, first = 0;
+    for (size_t l = 0; l < L; ++l) cells += (size_t)(kBoxShare * (double)s->lv[l].d.n()) + 1;
+    first = (size_t)(kBoxShare * (double)s->lv[0].d.n()) + 1;
+    if (dalloc(s, &s->box_rows, cells) != JG_OK || dalloc(s, &s->box_b, first) != JG_OK ||
+        dalloc(s, &s->box_x, first) != JG_OK) {
+        (void)hipGetLastError();
+        s->box_failed = true;
+        return false;
+    }
+    s->box_cells = cells;
+    return true;
+}
+
+// Runs a solve (run(solver, finish), finish called when the solution is
+// there and before the closing event) on s, or on a solver whose dense
+// arrays hold the box of s that takes part.  That solver is a view: its
+// work vectors and control blocks are s's own, which are larger; A32 too, so
+// s's FP32 copy has to be made anew afterwards.
+template <typename Run>
+int solve_in_box(jg_solver* s, size_t L, idx_t from, double most, bool mixed, Run&& run) {
+    auto whole = [&]() { return run(s, [] { return (int)JG_OK; }); };
+    Level& l0 = s->lv[0];
+    if (l0.d.n() < from || s->nsys > 1) return whole();
+    Box box;
+    double share = 1.0;
+    JG_TRY(find_box(s, L, most, &box, &share));
+    if (share == 0.0 || share > kBoxShare || !box_reserve(s, s->lv.size())) return whole();
+    int* const odd = (int*)(s->box_scan + 1);
+    k_fill<int><<<1, NT, 0, s->stream>>>(odd, 0, 1);
+    jg_solver v;
+    v.device = s->device;
+    v.cus = s->cus;
+    v.cooperative = s->cooperative;
+    v.view = true;
+    v.stream = s->stream;
+    v.ev0 = s->ev0;
+    v.ev1 = s->ev1;
+    v.evp[0] = s->evp[0];
+    v.evp[1] = s->evp[1];
+    v.ctl_host = s->ctl_host;
+    v.twod = s->twod;
+    v.r = s->r;
+    v.z = s->z;
+    v.dA = s->dA;
+    v.dB = s->dB;
+    v.q = s->q;
+    v.rhs32 = s->rhs32;
+    v.r32 = s->r32;
+    v.z32 = s->z32;
+    v.d32A = s->d32A;
+    v.d32B = s->d32B;
+    v.q32 = s->q32;
+    v.e32 = s->e32;
+    v.part = s->part;
+    v.scal = s->scal;
+    v.ctl = s->ctl;
+    v.cg_slots = s->cg_slots;
+    v.b = s->box_b;
+    v.x = s->box_x;
+    v.lv.assign(s->lv.begin(), s->lv.begin() + L);
+    Row<double>* rows = s->box_rows;
+    for (size_t l = 0; l < L; ++l) {
+        Level& lv = v.lv[l];
+        const Dims full = lv.d;
+        Box bl = box;
+        for (int a = 0; a < 3; ++a) bl.o[a] >>= (a == 2 && s->twod) ? 0 : l;
+        bl.n = Dims{box.n.nx >> l, box.n.ny >> l, s->twod ? 1 : box.n.nz >> l};
+        lv.d = bl.n;
+        const Geo g = geo_planes(l == 0 ? bl.n : full);
+        Row<double>* const to64 = !mixed || l == 0 ? rows : nullptr;
+        Row<float>* const to32 = mixed ? lv.A32 : nullptr;
+        if (l == 0)
+            k_box_rows<false><<<g.grid, g.block, 0, s->stream>>>(lv.A64, full, bl, most, to64, to32, odd);
+        else
+            k_box_rows<true><<<g.grid, g.block, 0, s->stream>>>(lv.A64, full, bl, most, to64, to32, odd);
+        lv.A64 = rows;
+        rows += bl.n.n();
+    }
+    const Geo gb = geo_planes(box.n), gf = geo_planes(l0.d);
+    k_box_gather<<<gb.grid, gb.block, 0, s->stream>>>(s->b, l0.d, box, v.b);
+    v.f32_valid = mixed;
+    if (mixed) s->f32_valid = false;
+    int bad = 0;
+    int st = check_launch(s, "box");
+    if (st == JG_OK)
+        st = run(&v, [&]() -> int {
+            k_box_scatter<<<gf.grid, gf.block, 0, s->stream>>>(v.x, l0.d, box, s->x);
+            JG_HIP(hipMemcpyAsync(&s->box_host->lo[0], odd, sizeof(int), hipMemcpyDeviceToHost, s->stream));
+            return check_launch(s, "box scatter");
+        });
+    // the solver's own parts stay with s
+    bad = s->box_host->lo[0];
+    s->cg_slots = v.cg_slots;
+    s->allocs.insert(s->allocs.end(), v.allocs.begin(), v.allocs.end());
+    v.allocs.clear();
+    if (!v.err.empty()) s->err = v.err;
+    v.ctl_host = nullptr;
+    v.ev0 = v.ev1 = v.evp[0] = v.evp[1] = nullptr;
+    if ((st == JG_OK || st == JG_ERR_NONFINITE) && bad) return whole();
+    return st;
+}
+
+}  // namespace
+
 extern "C" {
 
 void jg_mg_params_default(jg_mg_params* p) {
@@ -1527,7 +1657,8 @@ int jg_solver_create(int device, jg_solver** out) {
         hipEventCreate(&s->ev0) != hipSuccess || hipEventCreate(&s->ev1) != hipSuccess ||
         hipEventCreateWithFlags(&s->evp[0], hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&s->evp[1], hipEventDisableTiming) != hipSuccess ||
-        hipHostMalloc((void**)&s->ctl_host, 2 * sizeof(Ctl), hipHostMallocDefault) != hipSuccess) {
+        hipHostMalloc((void**)&s->ctl_host, 2 * sizeof(Ctl), hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc((void**)&s->box_host, sizeof(BoxScan), hipHostMallocDefault) != hipSuccess) {
         delete s;
         return JG_ERR_HIP;
     }
@@ -1628,35 +1759,11 @@ int jg_solver_matrices_changed(jg_solver* s) {
 int jg_solver_cg(jg_solver* s, unsigned max_iter, double tol, jg_solve_info* info) {
     if (!s || s->lv.empty()) return JG_ERR_INVALID_ARG;
     JG_HIP(hipSetDevice(s->device));
-    Level& l0 = s->lv[0];
-    Ctl h;
-    init_ctl(&h, max_iter, tol, 0, 0.0);
-    JG_TRY(upload_ctl(s, s->ctl, h));
-    k_fill<double><<<nblocks_1d(l0.d.n()), NT, 0, s->stream>>>(s->x, 0.0, l0.d.n());
     JG_HIP(hipEventRecord(s->ev0, s->stream));
-    JG_TRY(pcg_device<double>(s, Pcg<double>{l0.A64, s->b, s->x, s->r, s->r, s->dA, s->dB, s->q, l0.d,
-                                              s->ctl, nullptr},
-                              1));
-    JG_HIP(hipEventRecord(s->ev1, s->stream));
-    JG_HIP(hipMemcpyAsync(s->ctl_host, s->ctl, sizeof(Ctl), hipMemcpyDeviceToHost, s->stream));
-    JG_TRY(sync(s));
-    const Ctl& c = *s->ctl_host;
-    if (info) {
-        std::memset(info, 0, sizeof(*info));
-        float ms = 0.f;
-        JG_HIP(hipEventElapsedTime(&ms, s->ev0, s->ev1));
-        info->solve_ms = ms;
-        info->iterations = c.iter;
-        info->last_residual = std::sqrt(std::fabs(c.sigma));
-        // FdmCgSolver3::solve's return (src/jet/fdm_cg_solver3.cpp:45-46)
-        info->converged = (info->last_residual <= tol) || (c.iter < max_iter);
-        JG_TRY(true_rel_residual(s, &info->rel_residual));
-    }
-    if (c.nonfinite) {
-        s->err = "non-finite value in CG reduction";
-        return JG_ERR_NONFINITE;
-    }
-    return JG_OK;
+    return solve_in_box(s, 1, kBoxCgCells, DBL_MAX, false,
+                        [&](jg_solver* v, const std::function<int()>& finish) {
+                            return cg_run(v, max_iter, tol, info, finish);
+                        });
 }
 
 int jg_mg_vcycle(jg_solver* s, const jg_mg_params* p, const jg_gpu_options* o, const double* r,
@@ -1671,7 +1778,6 @@ int jg_mg_vcycle(jg_solver* s, const jg_mg_params* p, const jg_gpu_options* o, c
     int nb = 0;
     if (opt.precision == JG_MIXED) {
         JG_TRY(ensure_f32(s));
-        JG_TRY(autotune_sweeps<float>(s));
         MgCfg<float> mg{p->restrict_iter, p->final_iter, p->correct_iter, p->coarsest_iter,
                         (float)omega};
         mg.pairs = opt.sweep_pairs;
@@ -1680,7 +1786,6 @@ int jg_mg_vcycle(jg_solver* s, const jg_mg_params* p, const jg_gpu_options* o, c
         JG_TRY(vcycle<float>(s, s->r32, s->z32, mg, nullptr, &nb));
         k_convert<float, double><<<nb1, NT, 0, s->stream>>>(s->z32, z, n);
     } else {
-        JG_TRY(autotune_sweeps<double>(s));
         MgCfg<double> mg{p->restrict_iter, p->final_iter, p->correct_iter, p->coarsest_iter, omega};
         mg.pairs = opt.sweep_pairs;
         mg.jacobi = opt.smoother == JG_SMOOTH_JACOBI;
@@ -1742,120 +1847,12 @@ int jg_solver_mgpcg(jg_solver* s, unsigned max_iter, const jg_mg_params* p,
     jg_gpu_options opt;
     double omega = 0.0;
     JG_TRY(mg_options(s, p, o, &opt, &omega));
-    Level& l0 = s->lv[0];
-    const idx_t n = l0.d.n();
-    int status = JG_OK;
-    unsigned iters = 0, refinements = 0;
-    double last_res = 0.0;
-    double bnorm = 0.0;  // mixed: ||b||, for the relative residual of the final x
-    double mixed_goal = -1.0;  // mixed: the FP64 residual norm the refinement had to reach
-    Ctl* ctl = s->ctl;
-    if (opt.precision == JG_MIXED) {
-        JG_TRY(ensure_f32(s));
-        JG_TRY(autotune_sweeps<float>(s));
-    } else {
-        JG_TRY(autotune_sweeps<double>(s));
-    }
-    k_fill<double><<<nblocks_1d(n), NT, 0, s->stream>>>(s->x, 0.0, n);
+    const bool mixed = opt.precision == JG_MIXED;
     JG_HIP(hipEventRecord(s->ev0, s->stream));
-    if (opt.precision != JG_MIXED) {
-        MgCfg<double> mg{p->restrict_iter, p->final_iter, p->correct_iter, p->coarsest_iter, omega};
-        mg.pairs = opt.sweep_pairs;
-        mg.jacobi = opt.smoother == JG_SMOOTH_JACOBI;
-        Ctl h;
-        init_ctl(&h, max_iter, p->max_tol, opt.stop_rule == JG_STOP_RELATIVE ? 1 : 0, opt.rel_tol);
-        JG_TRY(upload_ctl(s, ctl, h));
-        JG_TRY(pcg_device<double>(s, Pcg<double>{l0.A64, s->b, s->x, s->r, s->z, s->dA, s->dB, s->q,
-                                                  l0.d, ctl, &mg},
-                                  opt.check_every));
-        JG_HIP(hipMemcpyAsync(s->ctl_host, ctl, sizeof(Ctl), hipMemcpyDeviceToHost, s->stream));
-        JG_TRY(sync(s));
-        iters = s->ctl_host->iter;
-        last_res = std::sqrt(std::fabs(s->ctl_host->sigma));
-        if (s->ctl_host->nonfinite) status = JG_ERR_NONFINITE;
-    } else {
-        // Iterative refinement: FP64 residual and correction, FP32 MGPCG
-        // (FP32 stencil, smoother and V-cycle; FP64 dot accumulation).
-        MgCfg<float> mg{p->restrict_iter, p->final_iter, p->correct_iter, p->coarsest_iter,
-                        (float)omega};
-        mg.pairs = opt.sweep_pairs;
-        mg.jacobi = opt.smoother == JG_SMOOTH_JACOBI;
-        const int nb1 = nblocks_1d(n);
-        k_dot<double, double><<<nb1, NT, 0, s->stream>>>(s->b, s->b, n, s->slot(3), nullptr);
-        k_fin_sum<<<1, kFinThreads, 0, s->stream>>>(s->slot(3), nb1, s->scal + 2);
-        double bb = 0.0;
-        JG_HIP(hipMemcpyAsync(&bb, s->scal + 2, sizeof(double), hipMemcpyDeviceToHost, s->stream));
-        JG_TRY(sync(s));
-        bnorm = std::sqrt(bb);
-        const double goal = opt.stop_rule == JG_STOP_RELATIVE ? opt.rel_tol * bnorm : p->max_tol;
-        Ctl* ictl = s->ctl + 1;
-        for (unsigned outer = 0;; ++outer) {
-            double rr = 0.0;
-            if (outer == 0) {
-                // x = 0: b - A x is b itself (bit for bit), and its norm is known
-                k_convert<double, float><<<nb1, NT, 0, s->stream>>>(s->b, s->rhs32, n);
-                rr = bb;
-            } else {
-                const int nr = residual_dot64<float>(s, l0, s->rhs32, s->slot(3));
-                k_fin_sum<<<1, kFinThreads, 0, s->stream>>>(s->slot(3), nr, s->scal + 3);
-                JG_HIP(hipMemcpyAsync(&rr, s->scal + 3, sizeof(double), hipMemcpyDeviceToHost,
-                                      s->stream));
-                JG_TRY(sync(s));
-            }
-            last_res = std::sqrt(rr);
-            if (!std::isfinite(rr)) {
-                status = JG_ERR_NONFINITE;
-                break;
-            }
-            if (last_res <= goal || outer >= opt.max_refine || iters >= max_iter) break;
-            Ctl h;
-            // The last refinement only needs to close the remaining gap to
-            // the goal (with a factor 2 margin for the FP32 inner residual).
-            const double inner = std::max(opt.inner_rel_tol, std::min(0.5, 0.5 * goal / last_res));
-            init_ctl(&h, max_iter - iters, 0.0, 1, inner);
-            JG_TRY(upload_ctl(s, ictl, h));
-            k_fill<float><<<nb1, NT, 0, s->stream>>>(s->e32, 0.f, n);
-            JG_TRY(pcg_device<float>(s, Pcg<float>{l0.A32, s->rhs32, s->e32, s->r32, s->z32, s->d32A,
-                                                   s->d32B, s->q32, l0.d, ictl, &mg},
-                                     opt.check_every));
-            iters += s->ctl_host->iter;
-            if (s->ctl_host->nonfinite) {
-                // a value beyond FP32 range (or a NaN) in the inner solve: the
-                // correction is meaningless, and x keeps the last finite one
-                status = JG_ERR_NONFINITE;
-                break;
-            }
-            k_add_correction<<<nb1, NT, 0, s->stream>>>(s->x, s->e32, n);
-            JG_TRY(check_launch(s, "refinement"));
-            ++refinements;
-        }
-        mixed_goal = goal;
-    }
-    JG_HIP(hipEventRecord(s->ev1, s->stream));
-    JG_TRY(sync(s));
-    if (info) {
-        std::memset(info, 0, sizeof(*info));
-        float ms = 0.f;
-        JG_HIP(hipEventElapsedTime(&ms, s->ev0, s->ev1));
-        info->solve_ms = ms;
-        info->iterations = iters;
-        info->refinements = refinements;
-        info->last_residual = last_res;
-        // FP64: Jet's rule (cg-inl.h:93 and fdm_mgpcg_solver3.cpp:78). Mixed: the
-        // outer loop stops on the true residual, so converged means it reached
-        // the goal; running out of refinements or iterations above it is not.
-        info->converged = opt.precision == JG_MIXED ? last_res <= mixed_goal
-                                                    : (last_res <= p->max_tol) || (iters < max_iter);
-        if (status != JG_OK) info->converged = 0;
-        if (opt.precision == JG_MIXED && bnorm > 0.0)
-            info->rel_residual = last_res / bnorm;  // the FP64 b - A x of the final x
-        else
-            JG_TRY(true_rel_residual(s, &info->rel_residual));
-        if (opt.stop_rule == JG_STOP_RELATIVE && status == JG_OK)
-            info->converged = info->rel_residual <= opt.rel_tol;
-    }
-    if (status == JG_ERR_NONFINITE) s->err = "non-finite value in MGPCG reduction";
-    return status;
+    return solve_in_box(s, s->lv.size(), kBoxMgCells, mixed ? FLT_MAX : DBL_MAX, mixed,
+                        [&](jg_solver* v, const std::function<int()>& finish) {
+                            return mgpcg_run(v, max_iter, p, opt, omega, info, finish);
+                        });
 }
 
 int jg_cg_solve_host(jg_solver* s, size_t nx, size_t ny, size_t nz, const double* rows,
@@ -2005,27 +2002,25 @@ Vecs<float> vecs32(jg_solver* s) { return {s->e32, s->rhs32, s->r32, s->z32, s->
 // the restriction; post: the coarse correction of level 1 is added as x is
 // loaded).
 template <typename T>
-int level0_plan(jg_solver* s, bool post) {
-    return sweep_plan<T>(s->lv[0], 2, post ? kSweepCorrect : kSweepZero, 0).front();
+int level0_plan(jg_solver* s) {
+    return sweep_plan<T>(s, s->lv[0].d, 2, 0).front();
 }
 
 template <typename T>
 void level0_launch(jg_solver* s, const Vecs<T>& v, bool post, T omega) {
     Level& l0 = s->lv[0];
     const Row<T>* A = Prec<T>::A(l0);
-    const int mode = level0_plan<T>(s, post);
+    const int mode = level0_plan<T>(s);
     const T* xin = post ? Prec<T>::y(l0) : nullptr;
     const T* coarse = post && s->lv.size() > 1 ? Prec<T>::x(s->lv[1]) : nullptr;
-    const int kind = post ? kSweepCorrect : kSweepZero;
     if (mode == kLaunchBrick)
         launch_brick2<T>(s, A, v.r, xin, v.z, l0.d, post ? 1 : 0, coarse, omega, s->ctl);
     else if (mode == kLaunchMarch)
         launch_sweep2<T>(s, A, v.r, xin, v.z, l0.d, post ? 1 : 0, coarse,
-                         post ? nullptr : Prec<T>::t(l0), omega, s->ctl,
-                         post ? Prec<T>::zc2(l0, kind) : Prec<T>::zc2res(l0));
+                         post ? nullptr : Prec<T>::t(l0), omega, s->ctl);
     else
         launch_sweep<T>(s, A, v.r, xin, v.z, l0.d, post ? 1 : 0, coarse, nullptr, nullptr, omega,
-                        s->ctl, Prec<T>::zc(l0, kind), Prec<T>::sh(l0, kind));
+                        s->ctl);
 }
 
 // Algorithmic bytes per cell of that launch under the 4-coefficient model:
@@ -2036,7 +2031,7 @@ void level0_launch(jg_solver* s, const Vecs<T>& v, bool post, T omega) {
 template <typename T>
 double level0_launch_bytes(jg_solver* s, bool post) {
     const double sa = sizeof(Row<T>), sv = sizeof(T);
-    const int mode = level0_plan<T>(s, post);
+    const int mode = level0_plan<T>(s);
     const double sweeps = mode == kLaunchSingle ? 1.0 : 2.0;
     double b = sweeps * (sa + 3 * sv);
     if (post && s->lv.size() > 1) b += 2 * sv + sv / 8;
@@ -2084,12 +2079,10 @@ int time_kernel_t(jg_solver* s, const Vecs<T>& v, int kernel, unsigned reps, dou
                 k_dot<T, T><<<nb1, NT, 0, s->stream>>>(v.r, v.z, n, s->slot(0), s->ctl);
                 break;
             case JG_KERNEL_SWEEP:
-                launch_sweep<T>(s, A, bt, v.r, v.x, d, 1, nullptr, nullptr, nullptr, T(1), s->ctl,
-                                Prec<T>::zc(l0), Prec<T>::sh(l0));
+                launch_sweep<T>(s, A, bt, v.r, v.x, d, 1, nullptr, nullptr, nullptr, T(1), s->ctl);
                 break;
             case JG_KERNEL_SWEEP2:
-                launch_sweep2<T>(s, A, bt, v.r, v.x, d, 1, nullptr, nullptr, T(1), s->ctl,
-                                 Prec<T>::zc2(l0, kSweepPlain));
+                launch_sweep2<T>(s, A, bt, v.r, v.x, d, 1, nullptr, nullptr, T(1), s->ctl);
                 break;
             case JG_KERNEL_PRE0:
             case JG_KERNEL_POST0:
@@ -2141,10 +2134,8 @@ extern "C" int jg_solver_time_kernel(jg_solver* s, int kernel, int precision, un
     JG_HIP(hipSetDevice(s->device));
     if (precision == JG_MIXED) {
         JG_TRY(ensure_f32(s));
-        JG_TRY(autotune_sweeps<float>(s));
         return time_kernel_t<float>(s, vecs32(s), kernel, reps, avg_ms, bytes);
     }
-    JG_TRY(autotune_sweeps<double>(s));
     return time_kernel_t<double>(s, vecs64(s), kernel, reps, avg_ms, bytes);
 }
 
@@ -2498,19 +2489,6 @@ int batch_replay(jg_batch* B, hipGraphExec_t exec, int which, unsigned max_iter)
     return JG_OK;
 }
 
-// Sweep tuning once per group, with launches that cover the whole group.
-template <typename T>
-int batch_tune(jg_batch* B) {
-    for (auto* g : B->groups) {
-        const int st = autotune_sweeps<T>(g);
-        if (st != JG_OK) {
-            B->err = g->err;
-            return st;
-        }
-    }
-    return JG_OK;
-}
-
 // The FP32 copies of every group whose members' matrices changed.
 int batch_f32(jg_batch* B) {
     for (size_t gi = 0; gi < B->groups.size(); ++gi) {
@@ -2652,7 +2630,6 @@ int jg_batch_mgpcg(jg_batch* B, unsigned max_iter, const jg_mg_params* p, const 
     }
     const bool mixed = opt.precision == JG_MIXED;
     if (mixed) JG_TRY(batch_f32(B));
-    JG_TRY(mixed ? batch_tune<float>(B) : batch_tune<double>(B));
     for (auto* g : B->groups) JG_TRY(sync(g));
     std::vector<unsigned> iters(S, 0), refinements(S, 0);
     std::vector<double> last(S, 0.0);

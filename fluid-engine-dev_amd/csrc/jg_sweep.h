@@ -144,34 +144,18 @@ __device__ __forceinline__ void prolong_z(int t, const Dims& fd, int& k0, int& k
     }
 }
 
-// Launch shapes of the fused sweep: RP tile rows per thread (block of
-// 64 x 16/RP threads) and PD planes of loads in flight ahead of the plane
-// being committed.  The autotuner picks one per level and precision.
-struct SweepShape {
-    int rp, pd;
-};
-constexpr SweepShape kSweepShapes[] = {{2, 1}, {2, 2}, {1, 1}, {1, 2}};
-constexpr int kNumSweepShapes = 4;
-
-// Occupancy each shape is compiled for (waves per SIMD): as many blocks per
-// CU as the VGPR budget allows without spilling.  The correction variant
-// holds the coarse taps too; in FP32 with two rows per thread it gets a
-// larger budget (one block per CU fewer) instead of spilling.
-constexpr int sweep_waves_per_eu(int tsize, int rp, int pd, bool correct) {
-    return rp == 2 ? (pd == 1 ? (tsize == 4 ? (correct ? 5 : 6) : 4)
-                              : (tsize == 4 ? (correct ? 4 : 5) : 2))
-                   : (tsize == 4 ? 8 : 4);
-}
-
-template <typename T, int FIRST, bool ZERO, bool CORRECT, bool DOT, int RP, int PD>
-__global__ __launch_bounds__(kSwLX * kSwLY / RP, sweep_waves_per_eu(sizeof(T), RP, PD, CORRECT)) void k_rb_sweep(
+// One tile position per thread, one plane of loads in flight ahead of the
+// plane being committed.  (Two positions per thread, or two planes, measured
+// as fast at 256^3, where the sweep is bound by HBM, and 3 to 9% slower on
+// average over 43 level shapes; the occupancy is what the VGPR budget allows
+// without spilling.)
+template <typename T, int FIRST, bool ZERO, bool CORRECT, bool DOT>
+__global__ __launch_bounds__(kSwLX* kSwLY, sizeof(T) == 4 || (ZERO && !CORRECT) ? 8 : 4) void k_rb_sweep(
     const Row<T>* __restrict__ A, const T* __restrict__ b, const T* __restrict__ xin,
     T* __restrict__ xout, Dims d, int zc, T omega, const T* __restrict__ coarse,
     double* __restrict__ p_bx, double* __restrict__ p_bb, const Ctl* __restrict__ ctl) {
 #pragma clang fp contract(off)
-    static_assert(RP == 1 || RP == 2, "rows per thread");
-    static_assert(PD == 1 || PD == 2, "prefetch depth");
-    constexpr int TY = kSwLY / RP;
+    constexpr int TY = kSwLY;
     constexpr int NTH = kSwLX * TY;
     // FP32: the c ring holds w = omega / c (0 for a zero-centre row) and the
     // update is (1 - omega) x + w (b - s), one division per cell and sweep;
@@ -238,9 +222,9 @@ __global__ __launch_bounds__(kSwLX * kSwLY / RP, sweep_waves_per_eu(sizeof(T), R
         sz[e / kCzX][e % kCzX] = w0 * zc0 + w1 * zc1;
     };
 
-    // Each thread owns RP positions, rows ly = ty + TY * r.  Per position: c
-    // and b of planes t, t-1, t-2, f of planes t .. t-3, the held r/u of
-    // plane t (written to LDS one step later) and PD prefetched planes.
+    // Each thread owns the position (tx, ty) of the tile: c and b of planes
+    // t, t-1, t-2, f of planes t .. t-3, the held r/u of plane t (written to
+    // LDS one step later) and the prefetched plane.
     // Prefetched plane: raw loads (lanes outside the domain load cell 0),
     // masked only when committed, so nothing waits on them before then.
     struct Pre {
@@ -252,27 +236,24 @@ __global__ __launch_bounds__(kSwLX * kSwLY / RP, sweep_waves_per_eu(sizeof(T), R
         T c0, c1, c2, f0, f1, f2, f3, b0, b1, b2, hr, hu;
         T px;      // final value of the last second-colour plane, stored one step later
         bool pst;  // px is pending
-        Pre p[PD];
+        Pre p;
         int ly, gy;
     };
-    Pos P[RP];
+    Pos P;
+    P.ly = ty;
+    P.gy = gy0 + ty;
+    P.c0 = P.c1 = P.c2 = T(1);
+    P.f0 = P.f1 = P.f2 = P.f3 = T(0);
+    P.b0 = P.b1 = P.b2 = T(0);
+    P.hr = P.hu = T(0);
+    P.px = T(0);
+    P.pst = false;
 #pragma unroll
-    for (int r = 0; r < RP; ++r) {
-        P[r].ly = ty + TY * r;
-        P[r].gy = gy0 + ty + TY * r;
-        P[r].c0 = P[r].c1 = P[r].c2 = T(1);
-        P[r].f0 = P[r].f1 = P[r].f2 = P[r].f3 = T(0);
-        P[r].b0 = P[r].b1 = P[r].b2 = T(0);
-        P[r].hr = P[r].hu = T(0);
-        P[r].px = T(0);
-        P[r].pst = false;
+    for (int s = 0; s < 4; ++s) sx[s][P.ly][tx] = T(0);
 #pragma unroll
-        for (int s = 0; s < 4; ++s) sx[s][P[r].ly][tx] = T(0);
-#pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            sr[s][P[r].ly][tx] = T(0);
-            su[s][P[r].ly][tx] = T(0);
-        }
+    for (int s = 0; s < 2; ++s) {
+        sr[s][P.ly][tx] = T(0);
+        su[s][P.ly][tx] = T(0);
     }
     // Branch-free: lanes outside the domain load cell 0 (always valid); the
     // commit selects the neutral values for them (c = 1, everything else 0).
@@ -366,58 +347,33 @@ __global__ __launch_bounds__(kSwLX * kSwLY / RP, sweep_waves_per_eu(sizeof(T), R
         Q.pst = false;
     };
 
-    // Prologue: planes k0-2 .. k0-3+PD in flight, the coarse tile of k0-2.
+    // Prologue: plane k0-2 in flight, the coarse tile of k0-2.
     if (CORRECT) zfetch(k0 - 2);
-#pragma unroll
-    for (int s = 0; s < PD; ++s)
-#pragma unroll
-        for (int r = 0; r < RP; ++r) fetch(P[r].p[s], P[r].gy, k0 - 2 + s);
+    fetch(P.p, P.gy, k0 - 2);
     if (CORRECT) zstore(k0 - 2);
     __syncthreads();
 
-    // Step t: commit plane t from prefetch slot (t - k0 + 2) % PD and refill
-    // that slot with plane t + PD.  The loop is unrolled PD times so every
-    // slot index is static: no register moves wait on loads in flight.
-    // The step count is rounded up to a multiple of PD so the unrolled body
-    // has no exit (which would keep the compiler from counting the loads in
-    // flight); a step past k1 + 1 commits a re-read plane and its colour
-    // stages touch only planes no later stage reads.
-    const int tend = k0 - 2 + (k1 + 4 - k0 + PD - 1) / PD * PD;
-    for (int t0 = k0 - 2; t0 < tend; t0 += PD) {
-#pragma unroll
-        for (int u = 0; u < PD; ++u) {
-            const int t = t0 + u;
-            // ---- commit plane t (prefetched), then prefetch plane t+PD
-#pragma unroll
-            for (int r = 0; r < RP; ++r) commit(P[r], P[r].p[u], t);
-            if (CORRECT && t + 1 <= k1 + 1) zfetch(t + 1);
-            // unconditional (past the end it re-reads plane k1+1, unused) so
-            // the compiler can count the loads in flight
-#pragma unroll
-            for (int r = 0; r < RP; ++r) fetch(P[r].p[u], P[r].gy, min(t + PD, k1 + 1));
-            // the final values of plane t - 3 (second colour of the last step)
-#pragma unroll
-            for (int r = 0; r < RP; ++r) flush(P[r], t - 3);
-            __syncthreads();
-            // ---- first colour on plane t - 1
-            if (t - 1 >= 0 && t - 1 < d.nz) {
-#pragma unroll
-                for (int r = 0; r < RP; ++r) first_colour(P[r], t - 1);
-            }
-            __syncthreads();
-            // ---- second colour on plane t - 2, final values written back
-            if (t - 2 >= k0 && t - 2 < k1) {
-#pragma unroll
-                for (int r = 0; r < RP; ++r) second_colour(P[r], t - 2);
-            }
-            // the coarse tile of plane t+1 (read by the next commit)
-            if (CORRECT && t + 1 <= k1 + 1) zstore(t + 1);
-            __syncthreads();
-        }
+    for (int t = k0 - 2; t <= k1 + 1; ++t) {
+        // ---- commit plane t (prefetched), then prefetch plane t + 1
+        commit(P, P.p, t);
+        if (CORRECT && t + 1 <= k1 + 1) zfetch(t + 1);
+        // unconditional (past the end it re-reads plane k1+1, unused) so
+        // the compiler can count the loads in flight
+        fetch(P.p, P.gy, min(t + 1, k1 + 1));
+        // the final values of plane t - 3 (second colour of the last step)
+        flush(P, t - 3);
+        __syncthreads();
+        // ---- first colour on plane t - 1
+        if (t - 1 >= 0 && t - 1 < d.nz) first_colour(P, t - 1);
+        __syncthreads();
+        // ---- second colour on plane t - 2, final values written back
+        if (t - 2 >= k0 && t - 2 < k1) second_colour(P, t - 2);
+        // the coarse tile of plane t+1 (read by the next commit)
+        if (CORRECT && t + 1 <= k1 + 1) zstore(t + 1);
+        __syncthreads();
     }
     // the last second-colour plane, k1 - 1
-#pragma unroll
-    for (int r = 0; r < RP; ++r) flush(P[r], k1 - 1);
+    flush(P, k1 - 1);
     if (DOT) {
         // Block partials of b.x and b.b; the x ring is free after the last barrier.
         double* sh = reinterpret_cast<double*>(&sx[0][0][0]);
