@@ -173,6 +173,9 @@ struct jg_solver {
     jg::Ctl* ctl = nullptr;      // [0]: FP64 / outer, [1]: FP32 inner
     jg::Ctl* ctl_host = nullptr; // pinned mirror, two slots
     unsigned long long* cg_slots = nullptr;  // grid sums of k_cg_grid
+    // The copy of x that jg_relax_red_black's sweep reads.
+    double* relax_tmp = nullptr;
+    size_t relax_cap = 0;
     // Solves in a box (jg_box.h): the scan's result (and its pinned mirror),
     // the dense rows of every level, right-hand side and solution.
     jg::BoxScan *box_scan = nullptr, *box_host = nullptr;
@@ -188,6 +191,7 @@ struct jg_solver {
 
     ~jg_solver() {
         release();
+        (void)hipFree(relax_tmp);
         if (ctl_host) (void)hipHostFree(ctl_host);
         if (box_host) (void)hipHostFree(box_host);
         if (ev0) (void)hipEventDestroy(ev0);

@@ -703,6 +703,45 @@ __global__ __launch_bounds__(NT) void k_jacobi(const Row<TA>* __restrict__ A,
     }
 }
 
+// k_jacobi through the tiled z-march (jg_kernels.h's tm_march): the same
+// values in the same operand order, each cell's row, x and b read once.  At
+// 150 x 122 x 106 cells FP64 22 us against 41 for the per-cell kernel, whose
+// 13 loads a cell go through L1 (108 MB compulsory: 4.9 TB/s).
+template <typename T, bool ZC = false>
+__global__ __launch_bounds__(kTmX* kTmY) void k_jacobi_tile(const Row<T>* __restrict__ A,
+                                                           const T* __restrict__ b,
+                                                           const T* __restrict__ x, T* __restrict__ xo,
+                                                           Dims d, int zc, T omega,
+                                                           const Ctl* __restrict__ ctl) {
+#pragma clang fp contract(off)
+    int bx, by, bz;
+    xcd_tile(bx, by, bz);
+    if (ctl && ctl->done) return;
+    __shared__ T sv[2][kTmY][kTmX];
+    __shared__ T su[2][kTmY][kTmX];
+    const T* const src[1] = {x};
+    tm_march<T, 1>(
+        A, src, b, d, bx, by, bz * zc, min(d.nz, bz * zc + zc), sv, su, [](T xv) { return xv; },
+        [&](idx_t c, bool in, const TmCell<T>& e, bool hl, bool hr, bool hd, bool hu) {
+            if (!in) return;
+            // Jet's relax operand order (offdiag)
+            T s = hl ? e.rl * e.l : T(0);
+            s += hr ? e.row.r * e.r : T(0);
+            s += hd ? e.ud * e.d : T(0);
+            s += hu ? e.row.u * e.u : T(0);
+            s += e.fm * e.m;
+            s += e.row.f * e.p;
+            T v;
+            if (ZC && e.row.c == T(0))
+                v = T(0);
+            else if (omega == T(1))
+                v = (e.cen - s) / e.row.c;
+            else
+                v = e.v + omega * ((e.cen - s) / e.row.c - e.v);
+            xo[c] = v;
+        });
+}
+
 // ------------------------------------------------------------- transfers
 
 // FdmMgUtils3::restrict (src/jet/fdm_mg_linear_system3.cpp:43-98): coarse

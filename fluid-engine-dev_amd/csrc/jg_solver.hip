@@ -318,6 +318,22 @@ int launch_residual(jg_solver* s, const Row<T>* A, const T* x, const T* b, TR* r
     return nblocks(g);
 }
 
+// One (weighted) Jacobi sweep of a single system: the tiled z-march where
+// rows are long enough for it, else the per-cell kernel.
+template <typename T, bool ZC>
+void launch_jacobi(jg_solver* s, const Row<T>* A, const T* b, const T* x, T* xo, const Dims& d, T omega,
+                   const Ctl* ctl) {
+    if (use_tm(d)) {
+        dim3 grid;
+        int zc;
+        tm_grid(d, grid, zc);
+        k_jacobi_tile<T, ZC><<<grid, dim3(kTmX, kTmY, 1), 0, s->stream>>>(A, b, x, xo, d, zc, omega, ctl);
+        return;
+    }
+    const Geo g = geo_stencil(d);
+    k_jacobi<T, T, ZC><<<g.grid, g.block, 0, s->stream>>>(A, b, x, xo, d, g.zc, omega, ctl);
+}
+
 template <typename T>
 struct MgCfg {
     unsigned pre, post0, post, coarsest;
@@ -342,14 +358,12 @@ int vcycle_jacobi(jg_solver* s, const T* r0, T* z0, const MgCfg<T>& c, const Ctl
     auto sweeps = [&](size_t l, unsigned count) {
         Level& lv = s->lv[l];
         const Dims& d = lv.d;
-        const Geo g = geo_stencil(d);
         T* x = X(l);
         T* y = Prec<T>::y(lv);
         const T* in = x;
         for (unsigned k = 0; k < count; ++k) {
             T* out = in == x ? y : x;
-            k_jacobi<T, T, true><<<g.grid, g.block, 0, s->stream>>>(Prec<T>::A(lv), B(l), in, out, d,
-                                                                   g.zc, c.omega, ctl);
+            launch_jacobi<T, true>(s, Prec<T>::A(lv), B(l), in, out, d, c.omega, ctl);
             in = out;
         }
         if (in != x) k_convert<T, T><<<nblocks_1d(d.n()), NT, 0, s->stream>>>(in, x, d.n());
@@ -1489,8 +1503,9 @@ int find_box(jg_solver* s, size_t L, double most, Box* box, double* share) {
     if (!s->box_scan) JG_TRY(dalloc(s, &s->box_scan, 2));
     k_box_reset<<<1, 64, 0, s->stream>>>(s->box_scan);
     const unsigned gx = (d.nx + 63) / 64;
-    const unsigned sy = (d.ny + 8 * kBoxY - 1) / (8 * kBoxY), sz = (d.nz + 7) / 8;
-    k_box_scan<true><<<dim3(gx, sy, sz), 64 * kBoxY, 0, s->stream>>>(l0.A64, s->b, d, most, s->box_scan);
+    // at most 128 waves in all
+    k_box_scan<true><<<dim3(gx, std::max(1u, 32u / gx), 1), 64 * kBoxY, 0, s->stream>>>(
+        l0.A64, s->b, d, most, s->box_scan);
     const dim3 grid(gx, (d.ny + kBoxY - 1) / kBoxY, (d.nz + kBoxZ - 1) / kBoxZ);
     k_box_scan<false><<<grid, 64 * kBoxY, 0, s->stream>>>(l0.A64, s->b, d, most, s->box_scan);
     JG_TRY(check_launch(s, "box scan"));
@@ -2194,23 +2209,23 @@ int jg_relax_red_black(jg_solver* s, size_t nx, size_t ny, size_t nz, const doub
     if (!s || !valid_dims(nx, ny, nz) || !rows || !b || !x) return JG_ERR_INVALID_ARG;
     JG_HIP(hipSetDevice(s->device));
     Dims d{(int)nx, (int)ny, (int)nz};
-    // One fused forward sweep (red then black) reading a copy of x: the
-    // sweep is out of place because its tiles overlap.
-    double* tmp = nullptr;
-    JG_HIP(hipMalloc(&tmp, d.n() * sizeof(double)));
-    hipError_t e = hipMemcpyAsync(tmp, x, d.n() * sizeof(double), hipMemcpyDeviceToDevice, s->stream);
-    if (e == hipSuccess) {
-        launch_sweep<double>(s, (const Row<double>*)rows, b, tmp, x, d, 0, nullptr, nullptr, nullptr,
-                             sor, nullptr);
-        e = hipGetLastError();
+    // One fused forward sweep (red then black) reading a copy of x (the sweep
+    // is out of place because its tiles overlap), in a buffer that the solver
+    // keeps and grows; its allocation per call cost a third of a 2M-cell
+    // sweep's time.
+    const size_t n = (size_t)d.n();
+    if (n > s->relax_cap) {
+        double* grown = nullptr;
+        JG_HIP(hipMalloc(&grown, n * sizeof(double)));
+        (void)hipFree(s->relax_tmp);  // (no call is in flight: each ends synchronised)
+        s->relax_tmp = grown;
+        s->relax_cap = n;
     }
-    if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
-    (void)hipFree(tmp);
-    if (e != hipSuccess) {
-        s->err = std::string("relax_red_black: ") + hipGetErrorString(e);
-        return JG_ERR_HIP;
-    }
-    return JG_OK;
+    k_convert<double, double><<<nblocks_1d((idx_t)n), NT, 0, s->stream>>>(x, s->relax_tmp, (idx_t)n);
+    launch_sweep<double>(s, (const Row<double>*)rows, b, s->relax_tmp, x, d, 0, nullptr, nullptr, nullptr,
+                         sor, nullptr);
+    JG_TRY(check_launch(s, "relax_red_black"));
+    return sync(s);
 }
 
 int jg_relax_red_black_noalloc(jg_solver* s, size_t nx, size_t ny, size_t nz, const double* rows,
@@ -2245,9 +2260,7 @@ int jg_relax_jacobi(jg_solver* s, size_t nx, size_t ny, size_t nz, const double*
         return JG_ERR_INVALID_ARG;
     JG_HIP(hipSetDevice(s->device));
     Dims d{(int)nx, (int)ny, (int)nz};
-    Geo g = geo_stencil(d);
-    k_jacobi<double, double><<<g.grid, g.block, 0, s->stream>>>((const Row<double>*)rows, b, x,
-                                                               xtemp, d, g.zc, 1.0, nullptr);
+    launch_jacobi<double, false>(s, (const Row<double>*)rows, b, x, xtemp, d, 1.0, nullptr);
     JG_TRY(check_launch(s, "relax_jacobi"));
     return sync(s);
 }
