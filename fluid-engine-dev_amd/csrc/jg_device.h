@@ -148,9 +148,8 @@ __device__ __forceinline__ double lane_value(double v, int lane) {
 template <int NT>
 __device__ __forceinline__ double block_sum(double v, double* sh) {
     const int lane = threadIdx.x + threadIdx.y * blockDim.x;
-#pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_down(v, o, kWave);
-    if ((lane & (kWave - 1)) == 0) sh[lane / kWave] = v;
+    v = wave_sum(v);
+    if ((lane & (kWave - 1)) == kWave - 1) sh[lane / kWave] = v;
     __syncthreads();
     double s = 0.0;
     if (lane == 0) {
@@ -212,9 +211,8 @@ __device__ __forceinline__ void reduce_partials_k(const double* const (&p)[K], i
         for (int k = 0; k < K; ++k) s[k] += p[k][i];
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-#pragma unroll
-        for (int o = kWave / 2; o > 0; o >>= 1) s[k] += __shfl_down(s[k], o, kWave);
-        if ((t & (kWave - 1)) == 0) sh[k * (NT / kWave) + t / kWave] = s[k];
+        s[k] = wave_sum(s[k]);
+        if ((t & (kWave - 1)) == kWave - 1) sh[k * (NT / kWave) + t / kWave] = s[k];
     }
     __syncthreads();
 #pragma unroll

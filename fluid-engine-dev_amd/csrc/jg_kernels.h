@@ -419,16 +419,41 @@ __global__ __launch_bounds__(kTmX * kTmY) void k_dir_spmv_tile(
     block_partial<kTmX * kTmY>(acc, partial, part);
 }
 
-// r = b - A x (k_residual: the same values in Jet's residual operand order)
-// through the tiled z-march, stored as TR; DOT: one partial of r.r per
-// block; REFRESH / GATED: k_residual's control-block gates.  A grid z
-// extent of nsb z-blocks per system covers a batch group.
-template <typename T, typename TR, bool DOT, bool REFRESH, bool GATED>
+// One column of the tiled residual r = b - A x (k_residual's values, in
+// Jet's residual operand order, src/jet/fdm_linear_system3.cpp:107-115),
+// stored as TR; the block's r.r is added to acc.
+template <typename T, typename TR>
+__device__ __forceinline__ void tm_residual(const Row<T>* __restrict__ A, const T* __restrict__ x,
+                                            const T* __restrict__ b, TR* __restrict__ r, const Dims& d,
+                                            int bx, int by, int k0, int k1, T (&sv)[2][kTmY][kTmX],
+                                            T (&su)[2][kTmY][kTmX], double& acc) {
+#pragma clang fp contract(off)
+    const T* const src[1] = {x};
+    tm_march<T, 1>(
+        A, src, b, d, bx, by, k0, k1, sv, su, [](T xv) { return xv; },
+        [&](idx_t c, bool in, const TmCell<T>& e, bool hl, bool hr, bool hd, bool hu) {
+            T rv = e.cen - e.row.c * e.v;
+            rv -= hl ? e.rl * e.l : T(0);
+            rv -= hr ? e.row.r * e.r : T(0);
+            rv -= hd ? e.ud * e.d : T(0);
+            rv -= hu ? e.row.u * e.u : T(0);
+            rv -= e.fm * e.m;
+            rv -= e.row.f * e.p;
+            if (in) {
+                r[c] = (TR)rv;
+                acc += (double)rv * (double)rv;
+            }
+        });
+}
+
+// r = b - A x through the tiled z-march; DOT: one partial of r.r per block;
+// GATED: k_residual's control-block gate.  A grid z extent of nsb z-blocks
+// per system covers a batch group.
+template <typename T, typename TR, bool DOT, bool GATED>
 __global__ __launch_bounds__(kTmX * kTmY) void k_residual_tile(
     const Row<T>* __restrict__ A, const T* __restrict__ x, const T* __restrict__ b,
     TR* __restrict__ r, Dims d, int zc, double* __restrict__ partial,
     const Ctl* __restrict__ ctl) {
-#pragma clang fp contract(off)
     int bx, by, bz;
     xcd_tile(bx, by, bz);
     idx_t part;
@@ -442,29 +467,38 @@ __global__ __launch_bounds__(kTmX * kTmY) void k_residual_tile(
         if (DOT) partial += sys * kSysPart;
         if (ctl) ctl += sys * kSysCtl;
     }
-    if (REFRESH && (ctl->done || !ctl->refresh)) return;
     if (GATED && ctl && ctl->done) return;
     __shared__ T sv[2][kTmY][kTmX];
     __shared__ T su[2][kTmY][kTmX];
-    const T* const src[1] = {x};
     double acc = 0.0;
-    tm_march<T, 1>(
-        A, src, b, d, bx, by, bz * zc, min(d.nz, bz * zc + zc), sv, su, [](T xv) { return xv; },
-        [&](idx_t c, bool in, const TmCell<T>& e, bool hl, bool hr, bool hd, bool hu) {
-            // Jet's residual operand order (src/jet/fdm_linear_system3.cpp:107-115)
-            T rv = e.cen - e.row.c * e.v;
-            rv -= hl ? e.rl * e.l : T(0);
-            rv -= hr ? e.row.r * e.r : T(0);
-            rv -= hd ? e.ud * e.d : T(0);
-            rv -= hu ? e.row.u * e.u : T(0);
-            rv -= e.fm * e.m;
-            rv -= e.row.f * e.p;
-            if (in) {
-                r[c] = (TR)rv;
-                if (DOT) acc += (double)rv * (double)rv;
-            }
-        });
+    tm_residual<T, TR>(A, x, b, r, d, bx, by, bz * zc, min(d.nz, bz * zc + zc), sv, su, acc);
     if (DOT) block_partial<kTmX * kTmY>(acc, partial, part);
+}
+
+// PCG's true residual on the iterations whose control block asks for it (the
+// tiles of k_residual_tile): a bounded number of blocks per system (the
+// grid's y index) that loop over the tiles, since most iterations skip it and
+// a block that only finds that out still costs its launch (26 600 of them
+// in a batch: 52 us an iteration).  RR: the system's r.r, one partial per block.
+template <typename T, bool RR>
+__global__ __launch_bounds__(kTmX * kTmY) void k_refresh_tile(
+    const Row<T>* __restrict__ A, const T* __restrict__ x, const T* __restrict__ b, T* __restrict__ r,
+    Dims d, int zc, int tiles, double* __restrict__ partial, const Ctl* __restrict__ ctl) {
+    const int sys = blockIdx.y;
+    ctl += sys * kSysCtl;
+    if (ctl->done || !ctl->refresh) return;
+    const idx_t n = d.n();
+    __shared__ T sv[2][kTmY][kTmX];
+    __shared__ T su[2][kTmY][kTmX];
+    const int tx = (d.nx + kTmX - 1) / kTmX, ty = (d.ny + kTmY - 1) / kTmY;
+    double acc = 0.0;
+    for (int id = blockIdx.x; id < tiles; id += gridDim.x) {
+        const int bx = id % tx, by = id / tx % ty, bz = id / (tx * ty);
+        tm_residual<T, T>(A + sys * n, x + sys * n, b + sys * n, r + sys * n, d, bx, by, bz * zc,
+                          min(d.nz, bz * zc + zc), sv, su, acc);
+        __syncthreads();  // the next tile reuses the LDS rows
+    }
+    if (RR) block_partial<kTmX * kTmY>(acc, partial + sys * kSysPart, (idx_t)blockIdx.x);
 }
 
 // r = b - A x (FdmBlas3::residual, src/jet/fdm_linear_system3.cpp:98-116);
@@ -527,11 +561,15 @@ __global__ __launch_bounds__(NT) void k_residual(const Row<TA>* __restrict__ A,
 // ---------------------------------------------------- elementwise updates
 
 // CG step: x += alpha d; r -= alpha q (skipped on true-residual refresh
-// iterations, where k_residual<..., REFRESH> recomputes r from the new x).
-template <typename TX>
+// iterations, where a REFRESH residual recomputes r from the new x).  RR:
+// also one partial of r.r per block -- without a preconditioner that is the
+// iteration's sigma, and a dot of its own would read r again (8 of 48 + 8
+// bytes a cell in FP64, and a launch).
+template <typename TX, bool RR>
 __global__ __launch_bounds__(NT) void k_update_xr(TX* __restrict__ x, TX* __restrict__ r,
                                                   const TX* __restrict__ dd,
                                                   const TX* __restrict__ q, idx_t n,
+                                                  double* __restrict__ partial,
                                                   const Ctl* __restrict__ ctl) {
 #pragma clang fp contract(off)
     const int sys = blockIdx.y;  // the system of a batch group
@@ -543,10 +581,16 @@ __global__ __launch_bounds__(NT) void k_update_xr(TX* __restrict__ x, TX* __rest
     if (ctl->done) return;
     const double alpha = ctl->alpha;
     const bool upd_r = !ctl->refresh;
+    double acc = 0.0;
     for (idx_t c = blockIdx.x * (idx_t)NT + threadIdx.x; c < n; c += (idx_t)gridDim.x * NT) {
         x[c] = (TX)((double)x[c] + alpha * (double)dd[c]);
-        if (upd_r) r[c] = (TX)((double)r[c] - alpha * (double)q[c]);
+        if (upd_r) {
+            const TX rv = (TX)((double)r[c] - alpha * (double)q[c]);
+            r[c] = rv;
+            if (RR) acc += (double)rv * (double)rv;
+        }
     }
+    if (RR && upd_r) block_partial<NT>(acc, partial + sys * kSysPart, (idx_t)blockIdx.x);
 }
 
 template <typename TA, typename TB>
@@ -947,18 +991,23 @@ __global__ __launch_bounds__(NT) void k_residual_plane(const Row<T>* __restrict_
 // same values, over a bounded grid (a grid-stride loop), so the iterations
 // whose control block skips it cost one small launch rather than one
 // early-exit block per stencil tile.
-template <typename T>
+template <typename T, bool RR>
 __global__ __launch_bounds__(NT) void k_residual_plane_refresh(const Row<T>* __restrict__ A,
                                                                const T* __restrict__ x,
                                                                const T* __restrict__ b,
                                                                T* __restrict__ r, Dims d,
+                                                               double* __restrict__ partial,
                                                                const Ctl* __restrict__ ctl) {
     if (ctl->done || !ctl->refresh) return;
     const idx_t n = (idx_t)d.nx * d.ny;
+    double acc = 0.0;
     for (idx_t c = blockIdx.x * (idx_t)NT + threadIdx.x; c < n; c += (idx_t)gridDim.x * NT) {
         const int j = (int)(c / d.nx), i = (int)(c - (idx_t)j * d.nx);
-        r[c] = residual_plane_at(A, x, b, i, j, d);
+        const T rv = residual_plane_at(A, x, b, i, j, d);
+        r[c] = rv;
+        if (RR) acc += (double)rv * (double)rv;
     }
+    if (RR) block_partial<NT>(acc, partial, (idx_t)blockIdx.x);
 }
 
 // r = b - A x of an FP64 one-plane level (k_residual_plane's values) stored
@@ -1051,10 +1100,18 @@ __global__ __launch_bounds__(NT) void k_correct2(const TX* __restrict__ coarse,
 
 // ------------------------------------------------------------- finalize
 
+// The control block as the host sees it: two pinned slots, the one of
+// iteration k (0: the start) at k & 1.  The finalize kernels write it there
+// themselves; the host waits for an event behind them, and no copy runs
+// between the iterations.  host: nullptr when nobody polls (a batch's graph).
+__device__ __forceinline__ void ctl_to_host(const Ctl* ctl, Ctl* host, unsigned k) {
+    if (host) host[k & 1] = *ctl;
+}
+
 // Initial PCG scalars: sigma = r.z, rr = r.r, bb = b.b (for the relative
 // rule), beta = 0 so the first fused direction update gives d = z.
 __global__ __launch_bounds__(kFinThreads) void k_fin_init(Ctl* ctl, const double* p_rz,
-                                                          const double* p_rr, int n) {
+                                                          const double* p_rr, int n, Ctl* host) {
     ctl += blockIdx.x * kSysCtl;  // one block per system of a batch group
     p_rz += blockIdx.x * kSysPart;
     p_rr += blockIdx.x * kSysPart;
@@ -1076,56 +1133,66 @@ __global__ __launch_bounds__(kFinThreads) void k_fin_init(Ctl* ctl, const double
         ctl->nonfinite = !isfinite(rz) || !isfinite(rr);
         const bool go = (ctl->stop_rule == 1) ? (rr > ctl->rel2 * ctl->bb) : (rz > ctl->tol2);
         ctl->done = !(go && ctl->iter < ctl->max_iter) || ctl->nonfinite;
+        ctl_to_host(ctl, host, 0);
     }
 }
 
 // alpha = sigma / d.q ; Jet's refresh rule for this iteration.
-__global__ __launch_bounds__(kFinThreads) void k_fin_alpha(Ctl* ctl, const double* p_dq, int n) {
+__global__ __launch_bounds__(kFinThreads) void k_fin_alpha(Ctl* ctl, const double* p_dq, int n,
+                                                           Ctl* host) {
     ctl += blockIdx.x * kSysCtl;  // one block per system of a batch group
     p_dq += blockIdx.x * kSysPart;
-    if (ctl->done) return;
     __shared__ double sh[kFinThreads / kWave];
+    // (the partials' loads do not wait for the stop flag's; stale partials of
+    // a stopped solve are summed and dropped)
+    const bool done = ctl->done != 0;
+    const double sigma = ctl->sigma;
+    const unsigned iter = ctl->iter;
+    const int trigger = ctl->trigger;
     const double dq = reduce_partials<kFinThreads>(p_dq, n, sh);
-    if (threadIdx.x == 0) {
+    if (threadIdx.x == 0 && !done) {
+        const double alpha = sigma / dq;
         ctl->dq = dq;
-        ctl->alpha = ctl->sigma / dq;
-        ctl->refresh = ctl->trigger || (ctl->iter % 50 == 0 && ctl->iter > 0);
+        ctl->alpha = alpha;
+        ctl->refresh = trigger || (iter % 50 == 0 && iter > 0);
         ctl->trigger = 0;
-        if (!isfinite(ctl->alpha)) {
+        if (!isfinite(alpha)) {
             ctl->nonfinite = 1;
             ctl->done = 1;
+            ctl_to_host(ctl, host, iter + 1);
         }
     }
 }
 
 // End of a PCG iteration (include/jet/detail/cg-inl.h:65-90): sigma_new =
-// r.z, trigger on growth, beta, iteration count and the stop test.
+// r.z, trigger on growth, beta, iteration count and the stop test.  n
+// partials, n_refresh on an iteration that recomputed the true residual.
 __global__ __launch_bounds__(kFinThreads) void k_fin_sigma(Ctl* ctl, const double* p_rz,
-                                                           const double* p_rr, int n) {
+                                                           const double* p_rr, int n, int n_refresh,
+                                                           Ctl* host) {
     ctl += blockIdx.x * kSysCtl;  // one block per system of a batch group
     p_rz += blockIdx.x * kSysPart;
     p_rr += blockIdx.x * kSysPart;
-    if (ctl->done) return;
     __shared__ double sh[2 * kFinThreads / kWave];
     const double* const pp[2] = {p_rz, p_rr};
     double rs[2];
+    const Ctl old = *ctl;
+    if (n != n_refresh && old.refresh) n = n_refresh;
     reduce_partials_k<kFinThreads, 2>(pp, n, sh, rs);
     const double rz = rs[0], rr = rs[1];
-    if (threadIdx.x == 0) {
-        const double sold = ctl->sigma;
-        ctl->sigma_old = sold;
-        ctl->sigma = rz;
-        ctl->rr = rr;
-        if (rz > sold) ctl->trigger = 1;
-        ctl->beta = rz / sold;
-        ctl->iter += 1;
-        bool go;
-        if (ctl->stop_rule == 1)
-            go = rr > ctl->rel2 * ctl->bb;
-        else
-            go = rz > ctl->tol2;
-        if (!isfinite(rz) || !isfinite(rr)) ctl->nonfinite = 1;
-        ctl->done = !(go && ctl->iter < ctl->max_iter) || ctl->nonfinite;
+    if (threadIdx.x == 0 && !old.done) {
+        Ctl c = old;
+        c.sigma_old = old.sigma;
+        c.sigma = rz;
+        c.rr = rr;
+        if (rz > old.sigma) c.trigger = 1;
+        c.beta = rz / old.sigma;
+        c.iter += 1;
+        const bool go = c.stop_rule == 1 ? rr > c.rel2 * c.bb : rz > c.tol2;
+        if (!isfinite(rz) || !isfinite(rr)) c.nonfinite = 1;
+        c.done = !(go && c.iter < c.max_iter) || c.nonfinite;
+        *ctl = c;
+        if (host) host[c.iter & 1] = c;
     }
 }
 

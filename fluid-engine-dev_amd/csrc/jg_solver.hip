@@ -298,23 +298,48 @@ int rr_zc(const Dims& cd, long blocks = 1024) {
 inline bool use_tm(const Dims& d) { return d.nx >= 48; }
 
 // r = b - A x on shape d (nsys systems back to back) stored as TR, with
-// k_residual's DOT / REFRESH / GATED options; returns the partial count per
-// system.  Rows of at least 48 cells take the tiled z-march
-// (k_residual_tile), narrower grids the per-cell one (k_residual).
-template <typename T, typename TR, bool DOT, bool REFRESH, bool GATED>
+// k_residual's DOT / GATED options; returns the partial count per system.
+// Rows of at least 48 cells take the tiled z-march (k_residual_tile),
+// narrower grids the per-cell one (k_residual).
+template <typename T, typename TR, bool DOT, bool GATED>
 int launch_residual(jg_solver* s, const Row<T>* A, const T* x, const T* b, TR* r, const Dims& d,
                     double* partial, const Ctl* ctl) {
     if (use_tm(d)) {
         dim3 grid;
         int zc;
         tm_grid(d, grid, zc);
-        k_residual_tile<T, TR, DOT, REFRESH, GATED><<<grid_sys(grid, s), dim3(kTmX, kTmY, 1), 0,
-                                                      s->stream>>>(A, x, b, r, d, zc, partial, ctl);
+        k_residual_tile<T, TR, DOT, GATED><<<grid_sys(grid, s), dim3(kTmX, kTmY, 1), 0, s->stream>>>(
+            A, x, b, r, d, zc, partial, ctl);
         return (int)(grid.x * grid.y * grid.z);
     }
     const Geo g = geo_stencil(d);
-    k_residual<T, T, TR, DOT, REFRESH, GATED><<<grid_sys(g.grid, s), g.block, 0, s->stream>>>(
+    k_residual<T, T, TR, DOT, false, GATED><<<grid_sys(g.grid, s), g.block, 0, s->stream>>>(
         A, x, b, r, d, g.zc, partial, ctl);
+    return nblocks(g);
+}
+
+// PCG's true residual on the iterations that ask for it, over a bounded
+// number of blocks; RR: partials of r.r, whose count per system is returned.
+template <typename T, bool RR>
+int launch_refresh(jg_solver* s, const Row<T>* A, const T* x, const T* b, T* r, const Dims& d,
+                   double* partial, const Ctl* ctl) {
+    if (d.nz == 1 && s->nsys == 1) {
+        const int nb = std::min(nblocks_1d(d.n()), 1024);
+        k_residual_plane_refresh<T, RR><<<nb, NT, 0, s->stream>>>(A, x, b, r, d, partial, ctl);
+        return nb;
+    }
+    if (use_tm(d)) {
+        dim3 grid;
+        int zc;
+        tm_grid(d, grid, zc);
+        const int tiles = (int)(grid.x * grid.y * grid.z), nb = std::min(tiles, 1024);
+        k_refresh_tile<T, RR><<<dim3((unsigned)nb, (unsigned)s->nsys, 1), dim3(kTmX, kTmY, 1), 0,
+                                s->stream>>>(A, x, b, r, d, zc, tiles, partial, ctl);
+        return nb;
+    }
+    const Geo g = geo_stencil(d);
+    k_residual<T, T, T, RR, true><<<grid_sys(g.grid, s), g.block, 0, s->stream>>>(A, x, b, r, d, g.zc,
+                                                                                  partial, ctl);
     return nblocks(g);
 }
 
@@ -697,7 +722,7 @@ int vcycle(jg_solver* s, const T* r0, T* z0, const MgCfg<T>& c, const Ctl* ctl, 
             // FP64: residual into t, then restriction (the fused kernel's
             // register footprint halves its occupancy in FP64, and the pair
             // measures faster)
-            launch_residual<T, T, false, false, true>(s, A, in, B(l), Prec<T>::t(lv), d, nullptr, ctl);
+            launch_residual<T, T, false, true>(s, A, in, B(l), Prec<T>::t(lv), d, nullptr, ctl);
             k_restrict<T><<<grid_sys(gc.grid, s), gc.block, 0, s->stream>>>(Prec<T>::t(lv), Prec<T>::b(s->lv[l + 1]),
                                                                cd, ctl);
         } else if (in) {
@@ -775,6 +800,7 @@ struct Pcg {
     const MgCfg<T>* mg;  // nullptr: no preconditioner (z aliases r)
     const CsrDev* csr = nullptr;  // compressed system (FP64, no preconditioner): A unused, d = {rows, 1, 1}
     const EllDev* ell = nullptr;  // its ELL copy, when it has one
+    bool polled = true;  // the host polls the control block (not in a batch's graph)
 };
 
 // z = M r and the r.z / r.r partials in slots 0 / 1 (from the V-cycle's last
@@ -813,15 +839,10 @@ int pcg_precondition(jg_solver* s, const Pcg<T>& v, const Ctl* c) {
     const idx_t n = v.d.n();
     const int nb1 = nblocks_1d(n);
     int nb = 0;
-    if (v.mg) {
-        const int st = vcycle<T>(s, v.r, v.z, *v.mg, c, &nb);
-        if (st != JG_OK) return -st;
-    }
+    const int st = vcycle<T>(s, v.r, v.z, *v.mg, c, &nb);
+    if (st != JG_OK) return -st;
     if (nb == 0) {
-        if (v.mg)
-            k_dot_rz_rr<T><<<grid_1d(nb1, s), NT, 0, s->stream>>>(v.r, v.z, n, s->slot(0), s->slot(1), c);
-        else
-            k_dot<T, T><<<grid_1d(nb1, s), NT, 0, s->stream>>>(v.r, v.z, n, s->slot(0), c);
+        k_dot_rz_rr<T><<<grid_1d(nb1, s), NT, 0, s->stream>>>(v.r, v.z, n, s->slot(0), s->slot(1), c);
         nb = nb1;
     }
     return nb;
@@ -840,9 +861,14 @@ int pcg_init(jg_solver* s, const Pcg<T>& v) {
     k_fill<T><<<grid_1d(nb1, s), NT, 0, s->stream>>>(v.dB, T(0), n);
     // (a batch group gates the preconditioner by the control blocks, which
     // say which members take part; a single system's is not set up yet)
-    const int nb = pcg_precondition<T>(s, v, s->nsys > 1 ? v.ctl : nullptr);
+    int nb = nb1;
+    if (v.mg)
+        nb = pcg_precondition<T>(s, v, s->nsys > 1 ? v.ctl : nullptr);
+    else  // z = r
+        k_dot<T, T><<<grid_1d(nb1, s), NT, 0, s->stream>>>(v.r, v.r, n, s->slot(0), nullptr);
     if (nb < 0) return -nb;
-    k_fin_init<<<s->nsys, kFinThreads, 0, s->stream>>>(v.ctl, s->slot(0), v.mg ? s->slot(1) : s->slot(0), nb);
+    k_fin_init<<<s->nsys, kFinThreads, 0, s->stream>>>(
+        v.ctl, s->slot(0), v.mg ? s->slot(1) : s->slot(0), nb, s->nsys > 1 ? nullptr : s->ctl_host);
     return check_launch(s, "pcg init");
 }
 
@@ -868,32 +894,34 @@ int pcg_iteration(jg_solver* s, const Pcg<T>& v, bool odd) {
             } else
                 k_csr_dir_spmv<<<nb1, NT, 0, s->stream>>>(*v.csr, v.z, dold, dnew, v.q, n,
                                                           s->slot(2), v.ctl);
-            k_fin_alpha<<<1, kFinThreads, 0, s->stream>>>(v.ctl, s->slot(2), nb1);
-            k_update_xr<T><<<nb1, NT, 0, s->stream>>>(v.x, v.r, dnew, v.q, n, v.ctl);
+            k_fin_alpha<<<1, kFinThreads, 0, s->stream>>>(v.ctl, s->slot(2), nb1, s->ctl_host);
+            k_update_xr<T, true><<<nb1, NT, 0, s->stream>>>(v.x, v.r, dnew, v.q, n, s->slot(0), v.ctl);
             if (v.ell)
-                k_ell_residual<false, true><<<nb1, NT, 0, s->stream>>>(*v.ell, v.x, v.b, v.r,
-                                                                       nullptr, v.ctl);
+                k_ell_residual<true, true><<<nb1, NT, 0, s->stream>>>(*v.ell, v.x, v.b, v.r, s->slot(0),
+                                                                      v.ctl);
             else
-                k_csr_residual<false, true><<<nb1, NT, 0, s->stream>>>(*v.csr, v.x, v.b, v.r, n,
-                                                                       nullptr, v.ctl);
-            const int nb = pcg_precondition<T>(s, v, v.ctl);
-            if (nb < 0) return -nb;
-            k_fin_sigma<<<1, kFinThreads, 0, s->stream>>>(v.ctl, s->slot(0), s->slot(0), nb);
+                k_csr_residual<true, true><<<nb1, NT, 0, s->stream>>>(*v.csr, v.x, v.b, v.r, n,
+                                                                      s->slot(0), v.ctl);
+            k_fin_sigma<<<1, kFinThreads, 0, s->stream>>>(v.ctl, s->slot(0), s->slot(0), nb1, nb1,
+                                                          s->ctl_host);
             return check_launch(s, "csr pcg iteration");
         }
     }
-    Geo g = geo_stencil(v.d);
+    Ctl* const host = v.polled ? s->ctl_host : nullptr;
     const int nsp = launch_dir_spmv<T>(s, v.A, v.z, dold, dnew, v.q, v.d, s->slot(2), v.ctl);
-    k_fin_alpha<<<s->nsys, kFinThreads, 0, s->stream>>>(v.ctl, s->slot(2), nsp);
-    k_update_xr<T><<<grid_1d(nb1, s), NT, 0, s->stream>>>(v.x, v.r, dnew, v.q, n, v.ctl);
-    if (v.d.nz == 1 && s->nsys == 1)
-        k_residual_plane_refresh<T><<<std::min(nb1, 1024), NT, 0, s->stream>>>(v.A, v.x, v.b, v.r,
-                                                                                v.d, v.ctl);
-    else
-        launch_residual<T, T, false, true, false>(s, v.A, v.x, v.b, v.r, v.d, nullptr, v.ctl);
+    k_fin_alpha<<<s->nsys, kFinThreads, 0, s->stream>>>(v.ctl, s->slot(2), nsp, host);
+    if (!v.mg) {  // z = r: sigma is r.r
+        k_update_xr<T, true><<<grid_1d(nb1, s), NT, 0, s->stream>>>(v.x, v.r, dnew, v.q, n, s->slot(0),
+                                                                    v.ctl);
+        const int nr = launch_refresh<T, true>(s, v.A, v.x, v.b, v.r, v.d, s->slot(0), v.ctl);
+        k_fin_sigma<<<s->nsys, kFinThreads, 0, s->stream>>>(v.ctl, s->slot(0), s->slot(0), nb1, nr, host);
+        return check_launch(s, "cg iteration");
+    }
+    k_update_xr<T, false><<<grid_1d(nb1, s), NT, 0, s->stream>>>(v.x, v.r, dnew, v.q, n, nullptr, v.ctl);
+    launch_refresh<T, false>(s, v.A, v.x, v.b, v.r, v.d, nullptr, v.ctl);
     const int nb = pcg_precondition<T>(s, v, v.ctl);
     if (nb < 0) return -nb;
-    k_fin_sigma<<<s->nsys, kFinThreads, 0, s->stream>>>(v.ctl, s->slot(0), v.mg ? s->slot(1) : s->slot(0), nb);
+    k_fin_sigma<<<s->nsys, kFinThreads, 0, s->stream>>>(v.ctl, s->slot(0), s->slot(1), nb, nb, host);
     return check_launch(s, "pcg iteration");
 }
 
@@ -945,7 +973,6 @@ int pcg_device(jg_solver* s, const Pcg<T>& v, unsigned check_every) {
         const int rows = cg_grid_rows(s, v);
         if (rows) return cg_grid(s, v, rows);
     }
-    JG_HIP(hipMemcpyAsync(s->ctl_host, v.ctl, sizeof(Ctl), hipMemcpyDeviceToHost, s->stream));
     JG_TRY(sync(s));
     if (s->ctl_host->done) return JG_OK;
     const unsigned max_iter = s->ctl_host->max_iter;
@@ -957,18 +984,17 @@ int pcg_device(jg_solver* s, const Pcg<T>& v, unsigned check_every) {
     // meets the stop test, the host waits first instead: a speculative
     // iteration after the last one still costs its launches.
     auto metric = [](const Ctl& c) { return c.stop_rule == 1 ? c.rr : c.sigma; };
-    const Ctl& c0 = *s->ctl_host;  // stable until the first poll below
+    const Ctl c0 = *s->ctl_host;
     const double lim = c0.stop_rule == 1 ? c0.rel2 * c0.bb : c0.tol2;
     double m_prev = -1.0, m_last = metric(c0);
     unsigned launched = 0;
-    int slot = 0;
+    int slot = 0;  // of the iteration polled: its number's parity (ctl_to_host)
     JG_TRY(pcg_iteration<T>(s, v, false));
     ++launched;
     while (true) {
         const bool poll = launched % check_every == 0 || launched >= max_iter;
         if (poll) {
-            JG_HIP(hipMemcpyAsync(s->ctl_host + slot, v.ctl, sizeof(Ctl), hipMemcpyDeviceToHost,
-                                  s->stream));
+            slot = (int)(launched & 1);
             JG_HIP(hipEventRecord(s->evp[slot], s->stream));
         }
         bool more = launched <= max_iter;  // the device stops by itself at max_iter
@@ -982,10 +1008,14 @@ int pcg_device(jg_solver* s, const Pcg<T>& v, unsigned check_every) {
         if (poll) {
             JG_HIP(hipEventSynchronize(s->evp[slot]));
             const Ctl& c = s->ctl_host[slot];
-            if (c.done) break;
+            if (c.done) {
+                // final state in slot 0 for the callers (the look-ahead
+                // iteration is a no-op and writes nothing)
+                if (slot != 0) s->ctl_host[0] = c;
+                return JG_OK;
+            }
             m_prev = m_last;
             m_last = metric(c);
-            slot ^= 1;
         }
         if (more) {  // the prediction was wrong: go on
             JG_TRY(pcg_iteration<T>(s, v, (launched & 1) != 0));
@@ -994,8 +1024,6 @@ int pcg_device(jg_solver* s, const Pcg<T>& v, unsigned check_every) {
             break;
         }
     }
-    // final state in slot 0 for the callers (the look-ahead iteration, a
-    // no-op, has drained by then)
     JG_HIP(hipMemcpyAsync(s->ctl_host, v.ctl, sizeof(Ctl), hipMemcpyDeviceToHost, s->stream));
     return sync(s);
 }
@@ -1032,7 +1060,7 @@ int residual_dot64(jg_solver* s, const Level& l0, TR* r, double* partial) {
         k_residual_plane_dot<TR><<<nb, NT, 0, s->stream>>>(l0.A64, s->x, s->b, r, l0.d, partial);
         return nb;
     }
-    return launch_residual<double, TR, true, false, false>(s, l0.A64, s->x, s->b, r, l0.d, partial,
+    return launch_residual<double, TR, true, false>(s, l0.A64, s->x, s->b, r, l0.d, partial,
                                                           nullptr);
 }
 
@@ -1153,7 +1181,6 @@ static int csr_solve(jg_solver* s, unsigned max_iter, double tol, jg_solve_info*
     if (c.ell_w > 0) v.ell = &e;
     JG_TRY(pcg_device<double>(s, v, 1));
     JG_HIP(hipEventRecord(s->ev1, s->stream));
-    JG_HIP(hipMemcpyAsync(s->ctl_host, s->ctl, sizeof(Ctl), hipMemcpyDeviceToHost, s->stream));
     JG_TRY(sync(s));
     const Ctl ch = *s->ctl_host;
     if (info) {
@@ -1351,7 +1378,6 @@ int cg_run(jg_solver* s, unsigned max_iter, double tol, jg_solve_info* info,
                               1));
     JG_TRY(finish());
     JG_HIP(hipEventRecord(s->ev1, s->stream));
-    JG_HIP(hipMemcpyAsync(s->ctl_host, s->ctl, sizeof(Ctl), hipMemcpyDeviceToHost, s->stream));
     JG_TRY(sync(s));
     const Ctl& c = *s->ctl_host;
     const bool nonfinite = c.nonfinite != 0;
@@ -1396,8 +1422,6 @@ int mgpcg_run(jg_solver* s, unsigned max_iter, const jg_mg_params* p, const jg_g
         JG_TRY(pcg_device<double>(s, Pcg<double>{l0.A64, s->b, s->x, s->r, s->z, s->dA, s->dB, s->q,
                                                   l0.d, ctl, &mg},
                                   opt.check_every));
-        JG_HIP(hipMemcpyAsync(s->ctl_host, ctl, sizeof(Ctl), hipMemcpyDeviceToHost, s->stream));
-        JG_TRY(sync(s));
         iters = s->ctl_host->iter;
         last_res = std::sqrt(std::fabs(s->ctl_host->sigma));
         if (s->ctl_host->nonfinite) status = JG_ERR_NONFINITE;
@@ -1822,12 +1846,12 @@ int jg_solver_mg(jg_solver* s, const jg_mg_params* p, const jg_gpu_options* o, j
     const idx_t n = l0.d.n();
     const int nb1 = nblocks_1d(n);
     JG_HIP(hipEventRecord(s->ev0, s->stream));
-    launch_residual<double, double, false, false, false>(s, l0.A64, s->x, s->b, s->r, l0.d, nullptr,
+    launch_residual<double, double, false, false>(s, l0.A64, s->x, s->b, s->r, l0.d, nullptr,
                                                          nullptr);
     JG_TRY(check_launch(s, "mg residual"));
     JG_TRY(jg_mg_vcycle(s, p, o, s->r, s->z));
     k_axpy<double><<<nb1, NT, 0, s->stream>>>(1.0, s->z, s->x, s->x, n);
-    const int nr = launch_residual<double, double, true, false, false>(s, l0.A64, s->x, s->b, s->r,
+    const int nr = launch_residual<double, double, true, false>(s, l0.A64, s->x, s->b, s->r,
                                                                        l0.d, s->slot(0), nullptr);
     k_fin_sum<<<1, kFinThreads, 0, s->stream>>>(s->slot(0), nr, s->scal + 0);
     k_dot<double, double><<<nb1, NT, 0, s->stream>>>(s->b, s->b, n, s->slot(1), nullptr);
@@ -2085,10 +2109,10 @@ int time_kernel_t(jg_solver* s, const Vecs<T>& v, int kernel, unsigned reps, dou
                 launch_dir_spmv<T>(s, A, v.z, v.dA, v.dB, v.q, d, s->slot(2), s->ctl);
                 break;
             case JG_KERNEL_RESIDUAL:
-                launch_residual<T, T, false, false, false>(s, A, v.x, bt, v.r, d, nullptr, nullptr);
+                launch_residual<T, T, false, false>(s, A, v.x, bt, v.r, d, nullptr, nullptr);
                 break;
             case JG_KERNEL_UPDATE_XR:
-                k_update_xr<T><<<nb1, NT, 0, s->stream>>>(v.x, v.r, v.dA, v.q, n, s->ctl);
+                k_update_xr<T, false><<<nb1, NT, 0, s->stream>>>(v.x, v.r, v.dA, v.q, n, nullptr, s->ctl);
                 break;
             case JG_KERNEL_DOT:
                 k_dot<T, T><<<nb1, NT, 0, s->stream>>>(v.r, v.z, n, s->slot(0), s->ctl);
@@ -2175,7 +2199,7 @@ int jg_blas_residual(jg_solver* s, size_t nx, size_t ny, size_t nz, const double
     if (!s || !valid_dims(nx, ny, nz) || !rows || !x || !b || !r) return JG_ERR_INVALID_ARG;
     JG_HIP(hipSetDevice(s->device));
     Dims d{(int)nx, (int)ny, (int)nz};
-    launch_residual<double, double, false, false, false>(s, (const Row<double>*)rows, x, b, r, d,
+    launch_residual<double, double, false, false>(s, (const Row<double>*)rows, x, b, r, d,
                                                          nullptr, nullptr);
     JG_TRY(check_launch(s, "residual"));
     return sync(s);
@@ -2436,12 +2460,13 @@ int batch_scal(jg_batch* B, int idx) {
 // its first member's pointers, which every launch extends to all members).
 Pcg<double> pcg64(jg_solver* s, const MgCfg<double>* mg) {
     Level& l0 = s->lv[0];
-    return Pcg<double>{l0.A64, s->b, s->x, s->r, s->z, s->dA, s->dB, s->q, l0.d, s->ctl, mg};
+    return Pcg<double>{l0.A64, s->b, s->x, s->r, s->z, s->dA, s->dB, s->q, l0.d, s->ctl, mg,
+                       nullptr, nullptr, false};
 }
 Pcg<float> pcg32(jg_solver* s, const MgCfg<float>* mg) {
     Level& l0 = s->lv[0];
     return Pcg<float>{l0.A32, s->rhs32, s->e32, s->r32, s->z32, s->d32A, s->d32B, s->q32, l0.d,
-                      s->ctl + 1, mg};
+                      s->ctl + 1, mg, nullptr, nullptr, false};
 }
 
 // Captures kBatchIters PCG iterations of every group into one graph (or
