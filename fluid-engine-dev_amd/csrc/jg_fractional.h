@@ -93,26 +93,40 @@ __device__ __forceinline__ float fr_weight(double p0, double p1, double p2, doub
     return (float)w;
 }
 
-// Face weights of one axis from the boundary SDF at the grid vertices
+// Face weights of all three axes from the boundary SDF at the grid vertices
 // ((nx+1)*(ny+1)*(nz+1), vertex (i,j,k) at origin + h*(i,j,k)); the four
-// corners of a face are vertices (buildWeights samples them, :553-617).
-template <int AXIS>
+// corners of a face are vertices (buildWeights samples them, :553-617).  A
+// thread marches the column of vertices (i, j) through a chunk of planes and
+// keeps the vertices (i .. i+1, j .. j+1) of two of them, so the SDF is read
+// from memory once for the three axes, not once for each.  At 512^3 (1.1 GB
+// in, 1.6 GB out) 850 us against 2020 for a launch per axis.
+constexpr int kFwZ = 16;
 __global__ __launch_bounds__(256) void k_fr_weights(const double* __restrict__ vs, Dims d,
-                                                    float* __restrict__ out) {
-    const int fx = d.nx + (AXIS == 0), fy = d.ny + (AXIS == 1), fz = d.nz + (AXIS == 2);
-    const idx_t n = (idx_t)fx * fy * fz;
+                                                    float* __restrict__ uw, float* __restrict__ vw,
+                                                    float* __restrict__ ww) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y * blockDim.y + threadIdx.y;
+    const int k0 = blockIdx.z * kFwZ, k1 = min(k0 + kFwZ, d.nz + 1);
+    if (i > d.nx || j > d.ny) return;
     const idx_t vx = d.nx + 1, vxy = vx * (d.ny + 1);
-    for (idx_t f = blockIdx.x * (idx_t)256 + threadIdx.x; f < n; f += (idx_t)gridDim.x * 256) {
-        const int i = (int)(f % fx), j = (int)((f / fx) % fy), k = (int)(f / ((idx_t)fx * fy));
-        auto V = [&](int a, int b, int c) { return vs[a + vx * b + vxy * c]; };
-        float w;
-        if (AXIS == 0)
-            w = fr_weight(V(i, j, k), V(i, j + 1, k), V(i, j, k + 1), V(i, j + 1, k + 1));
-        else if (AXIS == 1)
-            w = fr_weight(V(i, j, k), V(i, j, k + 1), V(i + 1, j, k), V(i + 1, j, k + 1));
-        else
-            w = fr_weight(V(i, j, k), V(i, j + 1, k), V(i + 1, j, k), V(i + 1, j + 1, k));
-        out[f] = w;
+    const int i1 = min(i + 1, d.nx), j1 = min(j + 1, d.ny);
+    struct Plane {
+        double a, b, c, e;  // (i,j) (i+1,j) (i,j+1) (i+1,j+1)
+    };
+    auto load = [&](int k) {
+        const double* p = vs + vxy * min(k, d.nz);
+        return Plane{p[i + vx * j], p[i1 + vx * j], p[i + vx * j1], p[i1 + vx * j1]};
+    };
+    Plane cur = load(k0), nxt = load(k0 + 1);
+    for (int k = k0; k < k1; ++k) {
+        const Plane ahead = load(k + 2);
+        if (j < d.ny && k < d.nz)
+            uw[i + vx * (j + (idx_t)d.ny * k)] = fr_weight(cur.a, cur.c, nxt.a, nxt.c);
+        if (i < d.nx && k < d.nz)
+            vw[i + (idx_t)d.nx * (j + (idx_t)(d.ny + 1) * k)] = fr_weight(cur.a, nxt.a, cur.b, nxt.b);
+        if (i < d.nx && j < d.ny)
+            ww[i + (idx_t)d.nx * (j + (idx_t)d.ny * k)] = fr_weight(cur.a, cur.c, cur.b, cur.e);
+        cur = nxt;
+        nxt = ahead;
     }
 }
 
@@ -126,52 +140,95 @@ __global__ __launch_bounds__(256) void k_fr_sdf_to_float(const double* __restric
 // Float restriction of a cell or face array (the anonymous restrict() of
 // src/jet/grid_fractional_single_phase_pressure_solver3.cpp:29-115): per
 // axis the centred kernel {1/8, 3/8, 3/8, 1/8} over fine 2c-1 .. 2c+2
-// (clamped), or injection {0, 1, 0} over 2c-1 .. 2c+1 along an axis whose
-// fine size is not twice the coarse size (the staggered axis of a face
-// array).  Jet's z, y, x accumulation order, float arithmetic.
+// (clamped), or injection of fine 2c along the staggered axis STAG (0, 1, 2:
+// x, y, z of a face array; 3: none, a cell array).  Jet sums the staggered
+// axis's neighbours too, with weight 0: face weights are finite, so that adds
+// nothing.  Jet's z, y, x accumulation order, float arithmetic.
+//
+// A wave takes 62 coarse columns of a row (lanes 1 .. 62; the outer lanes
+// only hold their neighbours' fine values) and marches a chunk of coarse
+// planes: of each fine row a lane loads its own two values and has the next
+// ones from the lanes beside it, and of the four fine planes of a coarse one
+// two are those of the last.  A load per tap (64 a cell, through L1) took
+// 0.80 ms of each 512^3 array against 0.11 of compulsory traffic, and with
+// the weights' fusion the whole build went from 8.9 to 4.5 ms.
+constexpr int kFrX = 62, kFrZ = 8;
+template <int STAG>
 __global__ __launch_bounds__(256) void k_fr_restrict(const float* __restrict__ fine, Dims fd,
                                                      float* __restrict__ coarse, Dims cd) {
 #pragma clang fp contract(off)
-    const idx_t n = cd.n();
-    const int stx = fd.nx != 2 * cd.nx, sty = fd.ny != 2 * cd.ny, stz = fd.nz != 2 * cd.nz;
-    for (idx_t e = blockIdx.x * (idx_t)256 + threadIdx.x; e < n; e += (idx_t)gridDim.x * 256) {
-        const int c3[3] = {(int)(e % cd.nx), (int)((e / cd.nx) % cd.ny), (int)(e / ((idx_t)cd.nx * cd.ny))};
-        const int cn[3] = {cd.nx, cd.ny, cd.nz};
-        const int st[3] = {stx, sty, stz};
-        int idx[3][4];
-        float kern[3][4];
+    constexpr int NY = STAG == 1 ? 1 : 4;
+    const int lane = threadIdx.x & 63;
+    const int i = (int)blockIdx.x * kFrX + lane - 1;
+    const int j = blockIdx.y * 4 + (threadIdx.x >> 6);
+    const int k0 = blockIdx.z * kFrZ, k1 = min(k0 + kFrZ, cd.nz);
+    if (j >= cd.ny) return;  // (whole waves)
+    const bool mine = lane >= 1 && lane <= kFrX && i < cd.nx;
+    const int ic = min(max(i, 0), cd.nx - 1);
+    idx_t row[NY];
 #pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            const int c = c3[a];
-            if (st[a]) {
-                idx[a][0] = c > 0 ? 2 * c - 1 : 2 * c;
-                idx[a][1] = 2 * c;
-                idx[a][2] = c + 1 < cn[a] ? 2 * c + 1 : 2 * c;
-                idx[a][3] = 2 * c;
-                kern[a][0] = 0.f;
-                kern[a][1] = 1.f;
-                kern[a][2] = 0.f;
-                kern[a][3] = 0.f;
+    for (int y = 0; y < NY; ++y) {
+        const int f = STAG == 1 ? 2 * j : min(max(2 * j - 1 + y, 0), 2 * cd.ny - 1);
+        row[y] = (idx_t)fd.nx * f + 2 * ic;
+    }
+    const idx_t fz = (idx_t)fd.nx * fd.ny;
+    struct Plane {
+        float a[NY], b[NY];  // fine 2i and 2i + 1 of each row
+    };
+    auto load = [&](int p) {
+        Plane v;
+#pragma unroll
+        for (int y = 0; y < NY; ++y) {
+            const float* f = fine + fz * p + row[y];
+            v.a[y] = f[0];
+            v.b[y] = STAG == 0 ? 0.f : f[1];
+        }
+        return v;
+    };
+    constexpr float kern[4] = {0.125f, 0.375f, 0.375f, 0.125f};
+    auto add = [&](float sum, const Plane& v, float kz) {
+#pragma unroll
+        for (int y = 0; y < NY; ++y) {
+            const float ky = STAG == 1 ? 1.f : kern[y];
+            if constexpr (STAG == 0) {
+                sum += (ky * kz) * v.a[y];
             } else {
-                idx[a][0] = c > 0 ? 2 * c - 1 : 2 * c;
-                idx[a][1] = 2 * c;
-                idx[a][2] = 2 * c + 1;
-                idx[a][3] = c + 1 < cn[a] ? 2 * c + 2 : 2 * c + 1;
-                kern[a][0] = 0.125f;
-                kern[a][1] = 0.375f;
-                kern[a][2] = 0.375f;
-                kern[a][3] = 0.125f;
+                float l = dpp_shift<kDppFromLeft>(v.b[y]), r = dpp_shift<kDppFromRight>(v.a[y]);
+                if (i == 0) l = v.a[y];
+                if (i + 1 == cd.nx) r = v.b[y];
+                sum += (kern[0] * ky * kz) * l;
+                sum += (kern[1] * ky * kz) * v.a[y];
+                sum += (kern[2] * ky * kz) * v.b[y];
+                sum += (kern[3] * ky * kz) * r;
             }
         }
-        const int kx = stx ? 3 : 4, ky = sty ? 3 : 4, kz = stz ? 3 : 4;
-        float sum = 0.0f;
-        for (int z = 0; z < kz; ++z)
-            for (int y = 0; y < ky; ++y)
-                for (int x = 0; x < kx; ++x) {
-                    const float w = kern[0][x] * kern[1][y] * kern[2][z];
-                    sum += w * fine[idx[0][x] + (idx_t)fd.nx * (idx[1][y] + (idx_t)fd.ny * idx[2][z])];
-                }
-        coarse[e] = sum;
+        return sum;
+    };
+    auto put = [&](int k, float v) {
+        if (mine) coarse[i + (idx_t)cd.nx * (j + (idx_t)cd.ny * k)] = v;
+    };
+    if constexpr (STAG == 2) {
+        Plane cur = load(2 * k0);
+        for (int k = k0; k < k1; ++k) {
+            const Plane next = load(2 * min(k + 1, cd.nz - 1));
+            put(k, add(0.0f, cur, 1.f));
+            cur = next;
+        }
+    } else {
+        auto plane = [&](int p) { return load(min(max(p, 0), 2 * cd.nz - 1)); };
+        Plane p0 = plane(2 * k0 - 1), p1 = plane(2 * k0), p2 = plane(2 * k0 + 1), p3 = plane(2 * k0 + 2);
+        for (int k = k0; k < k1; ++k) {
+            const Plane p4 = plane(2 * k + 3), p5 = plane(2 * k + 4);
+            float sum = add(0.0f, p0, kern[0]);
+            sum = add(sum, p1, kern[1]);
+            sum = add(sum, p2, kern[2]);
+            sum = add(sum, p3, kern[3]);
+            put(k, sum);
+            p0 = p2;
+            p1 = p3;
+            p2 = p4;
+            p3 = p5;
+        }
     }
 }
 
@@ -198,10 +255,13 @@ __global__ __launch_bounds__(256) void k_fr_build(
 #pragma clang fp contract(off)
     const double invH[3] = {1.0 / h.x, 1.0 / h.y, 1.0 / h.z};
     const double invHSqr[3] = {invH[0] * invH[0], invH[1] * invH[1], invH[2] * invH[2]};
-    const idx_t n = d.n();
     const idx_t ux = d.nx + 1, vy = d.ny + 1, sxy = (idx_t)d.nx * d.ny;
-    for (idx_t c = blockIdx.x * (idx_t)256 + threadIdx.x; c < n; c += (idx_t)gridDim.x * 256) {
-        const int i = (int)(c % d.nx), j = (int)((c / d.nx) % d.ny), k = (int)(c / sxy);
+    // (one plane per z-block: a flat loop's 64-bit divisions for i, j, k cost
+    // more than a cell's traffic)
+    const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y * blockDim.y + threadIdx.y;
+    const int k = blockIdx.z;
+    if (i < d.nx && j < d.ny) {
+        const idx_t c = i + (idx_t)d.nx * j + sxy * k;
         Row<double> row{0.0, 0.0, 0.0, 0.0};
         double bc = 0.0;
         const double cphi = fs[c];
@@ -314,10 +374,11 @@ __global__ __launch_bounds__(256) void k_fr_gradient(
     const double* v, const double* w, double* uo, double* vo, double* wo, Dims d, H3 h) {
 #pragma clang fp contract(off)
     const double invH[3] = {1.0 / h.x, 1.0 / h.y, 1.0 / h.z};
-    const idx_t n = d.n();
     const idx_t ux = d.nx + 1, vy = d.ny + 1, sxy = (idx_t)d.nx * d.ny;
-    for (idx_t c = blockIdx.x * (idx_t)256 + threadIdx.x; c < n; c += (idx_t)gridDim.x * 256) {
-        const int i = (int)(c % d.nx), j = (int)((c / d.nx) % d.ny), k = (int)(c / sxy);
+    const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y * blockDim.y + threadIdx.y;
+    const int k = blockIdx.z;
+    if (i < d.nx && j < d.ny) {
+        const idx_t c = i + (idx_t)d.nx * j + sxy * k;
         const double cphi = fs[c];
         if (i + 1 < d.nx) {
             const idx_t f = (i + 1) + ux * (j + (idx_t)d.ny * k);

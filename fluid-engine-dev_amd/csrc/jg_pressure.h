@@ -323,10 +323,12 @@ __global__ __launch_bounds__(256) void k_diffusion_build(const double* __restric
                                                          int dirichlet, Row<double>* __restrict__ A,
                                                          double* __restrict__ b) {
 #pragma clang fp contract(off)
-    const idx_t n = d.n(), oy = d.nx, oz = (idx_t)d.nx * d.ny;
+    const idx_t oy = d.nx, oz = (idx_t)d.nx * d.ny;
     auto mk = [&](idx_t q) -> int8_t { return bsdf[q] < 0 ? kBoundary : (fsdf[q] < 0 ? kFluid : kAir); };
-    for (idx_t q = blockIdx.x * (idx_t)256 + threadIdx.x; q < n; q += (idx_t)gridDim.x * 256) {
-        const int i = (int)(q % d.nx), j = (int)((q / d.nx) % d.ny), k = (int)(q / oz);
+    const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y * blockDim.y + threadIdx.y;
+    const int k = blockIdx.z;
+    if (i < d.nx && j < d.ny) {
+        const idx_t q = i + oy * j + oz * k;
         Row<double> row{1.0, 0.0, 0.0, 0.0};
         double bv = f[q];
         if (mk(q) == kFluid) {

@@ -306,28 +306,25 @@ int jg_fr_build(jg_solver* s, const double* u, const double* v, const double* w,
     auto faces = [](const Dims& d, int a) {
         return Dims{d.nx + (a == 0), d.ny + (a == 1), d.nz + (a == 2)};
     };
-    k_fr_weights<0><<<nblocks_1d(faces(d0, 0).n()), 256, 0, s->stream>>>(boundary_sdf_vertex, d0,
-                                                                         s->lv[0].uw);
-    k_fr_weights<1><<<nblocks_1d(faces(d0, 1).n()), 256, 0, s->stream>>>(boundary_sdf_vertex, d0,
-                                                                         s->lv[0].vw);
-    k_fr_weights<2><<<nblocks_1d(faces(d0, 2).n()), 256, 0, s->stream>>>(boundary_sdf_vertex, d0,
-                                                                         s->lv[0].ww);
+    k_fr_weights<<<dim3(d0.nx / 64 + 1, d0.ny / 4 + 1, d0.nz / kFwZ + 1), dim3(64, 4, 1), 0, s->stream>>>(
+        boundary_sdf_vertex, d0, s->lv[0].uw, s->lv[0].vw, s->lv[0].ww);
     k_fr_sdf_to_float<<<nblocks_1d(d0.n()), 256, 0, s->stream>>>(fluid_sdf, s->lv[0].fs, d0.n());
     for (size_t l = 1; l < s->lv.size(); ++l) {
-        const Dims& fd = s->lv[l - 1].d;
-        const Dims& cd = s->lv[l].d;
-        k_fr_restrict<<<nblocks_1d(cd.n()), 256, 0, s->stream>>>(s->lv[l - 1].fs, fd, s->lv[l].fs, cd);
-        float* fw[3] = {s->lv[l - 1].uw, s->lv[l - 1].vw, s->lv[l - 1].ww};
-        float* cw[3] = {s->lv[l].uw, s->lv[l].vw, s->lv[l].ww};
-        for (int a = 0; a < 3; ++a)
-            k_fr_restrict<<<nblocks_1d(faces(cd, a).n()), 256, 0, s->stream>>>(fw[a], faces(fd, a), cw[a],
-                                                                             faces(cd, a));
+        const Level &f = s->lv[l - 1], &c = s->lv[l];
+        auto grid = [](const Dims& n) {
+            return dim3((n.nx + kFrX - 1) / kFrX, (n.ny + 3) / 4, (n.nz + kFrZ - 1) / kFrZ);
+        };
+        k_fr_restrict<3><<<grid(c.d), 256, 0, s->stream>>>(f.fs, f.d, c.fs, c.d);
+        k_fr_restrict<0><<<grid(faces(c.d, 0)), 256, 0, s->stream>>>(f.uw, faces(f.d, 0), c.uw, faces(c.d, 0));
+        k_fr_restrict<1><<<grid(faces(c.d, 1)), 256, 0, s->stream>>>(f.vw, faces(f.d, 1), c.vw, faces(c.d, 1));
+        k_fr_restrict<2><<<grid(faces(c.d, 2)), 256, 0, s->stream>>>(f.ww, faces(f.d, 2), c.ww, faces(c.d, 2));
     }
     H3 h{hx, hy, hz};
     for (size_t l = 0; l < s->lv.size(); ++l) {
         Level& lv = s->lv[l];
         const bool top = l == 0;
-        k_fr_build<<<nblocks_1d(lv.d.n()), 256, 0, s->stream>>>(
+        const Geo g = geo_planes(lv.d);
+        k_fr_build<<<g.grid, g.block, 0, s->stream>>>(
             lv.fs, lv.uw, lv.vw, lv.ww, top ? u : nullptr, v, w, top ? bu : nullptr,
             top ? bv : nullptr, top ? bw : nullptr, lv.d, h, lv.A64, top ? s->b : nullptr);
         h.x *= 2.0;
@@ -348,8 +345,9 @@ int jg_fr_apply_gradient(jg_solver* s, const double* u, const double* v, const d
     }
     JG_HIP(hipSetDevice(s->device));
     const Level& l0 = s->lv[0];
-    k_fr_gradient<<<nblocks_1d(l0.d.n()), 256, 0, s->stream>>>(l0.fs, l0.uw, l0.vw, l0.ww, s->x, u, v,
-                                                                w, uo, vo, wo, l0.d, H3{hx, hy, hz});
+    const Geo g = geo_planes(l0.d);
+    k_fr_gradient<<<g.grid, g.block, 0, s->stream>>>(l0.fs, l0.uw, l0.vw, l0.ww, s->x, u, v, w, uo, vo,
+                                                     wo, l0.d, H3{hx, hy, hz});
     JG_TRY(check_launch(s, "fr_gradient"));
     return sync(s);
 }
@@ -580,7 +578,8 @@ int jg_diffusion_build(jg_solver* s, const double* f, const double* boundary_sdf
     // evaluates it (src/jet/grid_backward_euler_diffusion_solver3.cpp:33)
     const double sc = dt * mu;
     const double cx = sc / (hx * hx), cy = sc / (hy * hy), cz = sc / (hz * hz);
-    k_diffusion_build<<<nblocks_1d(l0.d.n()), 256, 0, s->stream>>>(
+    const Geo g = geo_planes(l0.d);
+    k_diffusion_build<<<g.grid, g.block, 0, s->stream>>>(
         f, boundary_sdf, fluid_sdf, l0.d, cx, cy, cz, dirichlet ? 1 : 0, l0.A64, s->b);
     JG_TRY(check_launch(s, "diffusion_build"));
     s->f32_valid = false;

@@ -189,3 +189,25 @@ def test_fr_torus_512_matches_oracle(solver):
         err = rel_err(x, sys_.x[0])
         print(f"  precision={prec} err_vs_oracle={err:.2e}", flush=True)
         assert err <= 1e-6
+
+
+@pytest.mark.parametrize("n,levels", [((124, 12, 10), 2), ((128, 10, 36), 2), ((248, 4, 34), 2),
+                                      ((252, 20, 8), 3), ((2, 2, 2), 2), ((66, 6, 70), 2)])
+def test_fr_weights_and_restriction_on_ragged_grids(solver, oracle, n, levels):
+    # rows of coarse cells and faces around 62 (what a wave of the restriction
+    # takes) and two of them, planes around its chunks of 8, vertices around
+    # the weights' tiles of 64 x 4 x 16; random distances, so that every
+    # corner case of a face occurs, infinite fluid distances among them
+    print(f"case fr ragged n={n}", flush=True)
+    nx, ny, nz = n
+    rng = np.random.default_rng(7)
+    s = {"u": rng.uniform(-1, 1, (nz, ny, nx + 1)), "v": rng.uniform(-1, 1, (nz, ny + 1, nx)),
+         "w": rng.uniform(-1, 1, (nz + 1, ny, nx)), "fsdf": rng.uniform(-1, 1, (nz, ny, nx)),
+         "vertex": rng.uniform(-1, 3, (nz + 1, ny + 1, nx + 1))}
+    s["fsdf"][0, 0, :] = np.finfo(np.float64).max
+    (fs, UW, VW, WW), sys_ = build_both(solver, oracle, s, levels)
+    for l in range(levels):
+        for which, ref in enumerate((UW[l], VW[l], WW[l], fs[l])):
+            got = np.empty(ref.shape, np.float32)
+            copy_to_host(solver.fr_array(l, which), got)
+            assert np.array_equal(got, ref, equal_nan=True), (l, which)
