@@ -672,11 +672,15 @@ __global__ __launch_bounds__(NT) void k_rows_to_f32(const Row<double>* __restric
     }
 }
 
-// Mixed precision: x64 += e32 (iterative-refinement correction).
+// Mixed precision: x64 += e32 (iterative-refinement correction).  ctl: a
+// batch's inner control blocks -- a system whose inner solve met a non-finite
+// value keeps its x.
 __global__ __launch_bounds__(NT) void k_add_correction(double* __restrict__ x,
-                                                       const float* __restrict__ e, idx_t n) {
+                                                       const float* __restrict__ e, idx_t n,
+                                                       const Ctl* __restrict__ ctl) {
     x += blockIdx.y * n;  // the system of a batch group
     e += blockIdx.y * n;
+    if (ctl && ctl[blockIdx.y * kSysCtl].nonfinite) return;
     for (idx_t c = blockIdx.x * (idx_t)NT + threadIdx.x; c < n; c += (idx_t)gridDim.x * NT)
         x[c] += (double)e[c];
 }

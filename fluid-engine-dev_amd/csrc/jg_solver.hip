@@ -1477,7 +1477,7 @@ int mgpcg_run(jg_solver* s, unsigned max_iter, const jg_mg_params* p, const jg_g
                 status = JG_ERR_NONFINITE;
                 break;
             }
-            k_add_correction<<<nb1, NT, 0, s->stream>>>(s->x, s->e32, n);
+            k_add_correction<<<nb1, NT, 0, s->stream>>>(s->x, s->e32, n, nullptr);
             JG_TRY(check_launch(s, "refinement"));
             ++refinements;
         }
@@ -2364,6 +2364,10 @@ __global__ void k_gather_scal(double* const* scal, int idx, int n, double* out) 
     for (int i = threadIdx.x; i < n; i += blockDim.x) out[i] = scal[i][idx];
 }
 
+__global__ void k_gather_sigma(Ctl* const* ctls, int n, double* out) {
+    for (int i = threadIdx.x; i < n; i += blockDim.x) out[i] = ctls[i]->sigma;
+}
+
 }  // namespace
 
 struct jg_batch {
@@ -2454,6 +2458,29 @@ int batch_scal(jg_batch* B, int idx) {
     JG_HIPB(hipMemcpyAsync(B->hvals, B->dvals, S * sizeof(double), hipMemcpyDeviceToHost, B->stream));
     JG_HIPB(hipStreamSynchronize(B->stream));
     return JG_OK;
+}
+
+// The control blocks of a group's members, both of each, in one copy.
+int batch_upload_ctl(jg_batch* B, jg_solver* g, const std::vector<Ctl>& h) {
+    JG_HIPB(hipMemcpyAsync(g->ctl, h.data(), h.size() * sizeof(Ctl), hipMemcpyHostToDevice, g->stream));
+    return JG_OK;
+}
+
+// ||b||^2 (into scal + at) and, with x, ||b - A x||^2 (into scal + at + 1,
+// the residual itself into r) of every member of a group, in FP64; one launch
+// covers the group.
+void group_bb(jg_solver* g, int at) {
+    const int nb1 = nblocks_1d(g->lv[0].d.n());
+    k_dot<double, double><<<grid_1d(nb1, g), NT, 0, g->stream>>>(g->b, g->b, g->lv[0].d.n(), g->slot(3),
+                                                                nullptr);
+    k_fin_sum<<<g->nsys, kFinThreads, 0, g->stream>>>(g->slot(3), nb1, g->scal + at);
+}
+template <typename TR>
+void group_residual(jg_solver* g, TR* r, int at) {
+    Level& l0 = g->lv[0];
+    const int nr = launch_residual<double, TR, true, false>(g, l0.A64, g->x, g->b, r, l0.d, g->slot(3),
+                                                            nullptr);
+    k_fin_sum<<<g->nsys, kFinThreads, 0, g->stream>>>(g->slot(3), nr, g->scal + at);
 }
 
 // Precision-specific views of a solver's level-0 PCG buffers (a group's:
@@ -2670,7 +2697,7 @@ int jg_batch_mgpcg(jg_batch* B, unsigned max_iter, const jg_mg_params* p, const 
     if (mixed) JG_TRY(batch_f32(B));
     for (auto* g : B->groups) JG_TRY(sync(g));
     std::vector<unsigned> iters(S, 0), refinements(S, 0);
-    std::vector<double> last(S, 0.0);
+    std::vector<double> last(S, 0.0), bnorm(S, 0.0);
     std::vector<int> status(S, JG_OK);
     JG_TRY(batch_join(B));
     JG_HIPB(hipEventRecord(B->ev0, B->stream));
@@ -2685,11 +2712,11 @@ int jg_batch_mgpcg(jg_batch* B, unsigned max_iter, const jg_mg_params* p, const 
             jg_solver* g = B->groups[gi];
             const Dims& d0 = g->lv[0].d;
             k_fill<double><<<grid_1d(nblocks_1d(d0.n()), g), NT, 0, g->stream>>>(g->x, 0.0, d0.n());
-            for (int m : B->members[gi]) {
-                Ctl h;
-                init_ctl(&h, max_iter, p->max_tol, opt.stop_rule == JG_STOP_RELATIVE ? 1 : 0, opt.rel_tol);
-                JG_TRY(upload_ctl(g, B->sys[m]->ctl, h));
-            }
+            std::vector<Ctl> h(kSysCtl * (size_t)g->nsys);
+            for (int q = 0; q < g->nsys; ++q)
+                init_ctl(&h[kSysCtl * q], max_iter, p->max_tol, opt.stop_rule == JG_STOP_RELATIVE ? 1 : 0,
+                         opt.rel_tol);
+            JG_TRY(batch_upload_ctl(B, g, h));
             JG_TRY(pcg_init<double>(g, pcg64(g, &mg)));
         }
         JG_TRY(batch_join(B));
@@ -2705,31 +2732,31 @@ int jg_batch_mgpcg(jg_batch* B, unsigned max_iter, const jg_mg_params* p, const 
         hipGraphExec_t exec = nullptr;
         JG_TRY(batch_graph<float>(B, JG_MIXED, mg, &exec));
         JG_TRY(batch_fork(B));
-        // ||b|| of every member
-        for (auto* s : B->sys) {
-            const Dims& d0 = s->lv[0].d;
+        // x = 0, ||b|| and the FP32 right-hand side of every member (b - A x is b)
+        for (auto* g : B->groups) {
+            const Dims& d0 = g->lv[0].d;
             const int nb1 = nblocks_1d(d0.n());
-            k_fill<double><<<nb1, NT, 0, s->stream>>>(s->x, 0.0, d0.n());
-            k_dot<double, double><<<nb1, NT, 0, s->stream>>>(s->b, s->b, d0.n(), s->slot(3), nullptr);
-            k_fin_sum<<<1, kFinThreads, 0, s->stream>>>(s->slot(3), nb1, s->scal + 2);
+            k_fill<double><<<grid_1d(nb1, g), NT, 0, g->stream>>>(g->x, 0.0, d0.n());
+            k_convert<double, float><<<grid_1d(nb1, g), NT, 0, g->stream>>>(g->b, g->rhs32, d0.n());
+            group_bb(g, 2);
         }
         JG_TRY(batch_join(B));
         JG_TRY(batch_scal(B, 2));
         std::vector<double> goal(S);
-        for (size_t i = 0; i < S; ++i)
-            goal[i] = opt.stop_rule == JG_STOP_RELATIVE ? opt.rel_tol * std::sqrt(B->hvals[i]) : p->max_tol;
+        for (size_t i = 0; i < S; ++i) {
+            bnorm[i] = std::sqrt(B->hvals[i]);
+            goal[i] = opt.stop_rule == JG_STOP_RELATIVE ? opt.rel_tol * bnorm[i] : p->max_tol;
+        }
         std::vector<char> done(S, 0);
         for (unsigned outer = 0;; ++outer) {
-            JG_TRY(batch_fork(B));
-            // FP64 residual r = b - A x of every unfinished member, into the FP32 right-hand side
-            for (size_t i = 0; i < S; ++i) {
-                if (done[i]) continue;
-                jg_solver* s = B->sys[i];
-                const int nr = residual_dot64<float>(s, s->lv[0], s->rhs32, s->slot(3));
-                k_fin_sum<<<1, kFinThreads, 0, s->stream>>>(s->slot(3), nr, s->scal + 3);
+            if (outer > 0) {
+                // FP64 residual r = b - A x into the FP32 right-hand side (of
+                // a finished member too: its x, and so its norm, is unchanged)
+                JG_TRY(batch_fork(B));
+                for (auto* g : B->groups) group_residual<float>(g, g->rhs32, 3);
+                JG_TRY(batch_join(B));
+                JG_TRY(batch_scal(B, 3));
             }
-            JG_TRY(batch_join(B));
-            JG_TRY(batch_scal(B, 3));
             bool any = false;
             for (size_t i = 0; i < S; ++i) {
                 if (done[i]) continue;
@@ -2749,18 +2776,20 @@ int jg_batch_mgpcg(jg_batch* B, unsigned max_iter, const jg_mg_params* p, const 
                 jg_solver* g = B->groups[gi];
                 // each member's inner control block: a finished member's
                 // blocks exit at once
-                for (int m : B->members[gi]) {
-                    Ctl h;
+                std::vector<Ctl> h(kSysCtl * (size_t)g->nsys);
+                for (int q = 0; q < g->nsys; ++q) {
+                    const int m = B->members[gi][q];
+                    Ctl& c = h[kSysCtl * q + 1];
                     if (done[m]) {
-                        init_ctl(&h, 0, 0.0, 1, 0.0);
-                        h.done = 1;
+                        init_ctl(&c, 0, 0.0, 1, 0.0);
+                        c.done = 1;
                     } else {
                         const double inner =
                             std::max(opt.inner_rel_tol, std::min(0.5, 0.5 * goal[m] / last[m]));
-                        init_ctl(&h, max_iter - iters[m], 0.0, 1, inner);
+                        init_ctl(&c, max_iter - iters[m], 0.0, 1, inner);
                     }
-                    JG_TRY(upload_ctl(g, B->sys[m]->ctl + 1, h));
                 }
+                JG_TRY(batch_upload_ctl(B, g, h));
                 const Dims& d0 = g->lv[0].d;
                 k_fill<float><<<grid_1d(nblocks_1d(d0.n()), g), NT, 0, g->stream>>>(g->e32, 0.f, d0.n());
                 JG_TRY(pcg_init<float>(g, pcg32(g, &mg)));
@@ -2771,17 +2800,18 @@ int jg_batch_mgpcg(jg_batch* B, unsigned max_iter, const jg_mg_params* p, const 
             JG_TRY(batch_fork(B));
             for (size_t i = 0; i < S; ++i) {
                 if (done[i]) continue;
-                jg_solver* s = B->sys[i];
                 iters[i] += (unsigned)B->hflags[2 * i + 1];
                 if (B->hflags[2 * i] & 2) {  // the inner FP32 solve met a non-finite value
                     status[i] = JG_ERR_NONFINITE;
                     done[i] = 1;
                     continue;
                 }
-                const Dims& d0 = s->lv[0].d;
-                k_add_correction<<<nblocks_1d(d0.n()), NT, 0, s->stream>>>(s->x, s->e32, d0.n());
                 ++refinements[i];
             }
+            // (a finished member's e32 is zero)
+            for (auto* g : B->groups)
+                k_add_correction<<<grid_1d(nblocks_1d(g->lv[0].d.n()), g), NT, 0, g->stream>>>(
+                    g->x, g->e32, g->lv[0].d.n(), g->ctl + 1);
         }
     }
     JG_TRY(batch_join(B));
@@ -2790,9 +2820,34 @@ int jg_batch_mgpcg(jg_batch* B, unsigned max_iter, const jg_mg_params* p, const 
     float ms = 0.f;
     JG_HIPB(hipEventElapsedTime(&ms, B->ev0, B->ev1));
     if (total_ms) *total_ms = ms;
+    std::vector<double> rel(S, 0.0);
+    if (infos) {
+        // mixed: last is the FP64 norm of the final x's residual already
+        JG_TRY(batch_fork(B));
+        if (!mixed)
+            for (auto* g : B->groups) {
+                group_bb(g, 0);
+                group_residual<double>(g, g->r, 1);
+            }
+        JG_TRY(batch_join(B));
+        if (!mixed) {
+            JG_TRY(batch_scal(B, 0));
+            for (size_t i = 0; i < S; ++i) bnorm[i] = std::sqrt(B->hvals[i]);
+            JG_TRY(batch_scal(B, 1));
+            for (size_t i = 0; i < S; ++i) rel[i] = std::sqrt(B->hvals[i]);
+            k_gather_sigma<<<1, 256, 0, B->stream>>>(B->dctl, (int)S, B->dvals);
+            JG_HIPB(hipGetLastError());
+            JG_HIPB(hipMemcpyAsync(B->hvals, B->dvals, S * sizeof(double), hipMemcpyDeviceToHost, B->stream));
+            JG_HIPB(hipStreamSynchronize(B->stream));
+            for (size_t i = 0; i < S; ++i) last[i] = std::sqrt(std::fabs(B->hvals[i]));
+        }
+        for (size_t i = 0; i < S; ++i) {
+            if (mixed) rel[i] = last[i];
+            if (bnorm[i] > 0) rel[i] /= bnorm[i];
+        }
+    }
     int worst = JG_OK;
     for (size_t i = 0; i < S; ++i) {
-        jg_solver* s = B->sys[i];
         if (status[i] != JG_OK) worst = status[i];
         if (!infos) continue;
         jg_solve_info& info = infos[i];
@@ -2800,11 +2855,7 @@ int jg_batch_mgpcg(jg_batch* B, unsigned max_iter, const jg_mg_params* p, const 
         info.iterations = iters[i];
         info.refinements = refinements[i];
         info.solve_ms = ms;
-        JG_TRY(true_rel_residual(s, &info.rel_residual));
-        if (!mixed) {
-            JG_HIPB(hipMemcpy(s->ctl_host, s->ctl, sizeof(Ctl), hipMemcpyDeviceToHost));
-            last[i] = std::sqrt(std::fabs(s->ctl_host->sigma));
-        }
+        info.rel_residual = rel[i];
         info.last_residual = last[i];
         if (status[i] != JG_OK)
             info.converged = 0;
