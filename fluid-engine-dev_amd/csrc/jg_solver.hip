@@ -718,7 +718,13 @@ int vcycle(jg_solver* s, const T* r0, T* z0, const MgCfg<T>& c, const Ctl* ctl, 
         pre_out[l] = in;  // nullptr: x is still zero
         const Dims& cd = s->lv[l + 1].d;
         Geo gc = geo_planes(cd);
-        if (in && sizeof(T) == 8) {
+        const bool from_t = in && sizeof(T) == 4 && pre_plan.back() == kLaunchMarch;  // t holds the residual
+        if (in && !from_t && d.n() <= kRbMaxCells) {
+            const dim3 grid = grid_sys(dim3((cd.nx + kRbX - 1) / kRbX, (cd.ny + kRbY - 1) / kRbY,
+                                            (cd.nz + kRbZ - 1) / kRbZ), s);
+            k_residual_restrict_brick<T><<<grid, kRbThreads, 0, s->stream>>>(
+                A, in, B(l), Prec<T>::b(s->lv[l + 1]), d, cd, ctl);
+        } else if (in && sizeof(T) == 8) {
             // FP64: residual into t, then restriction (the fused kernel's
             // register footprint halves its occupancy in FP64, and the pair
             // measures faster)
@@ -726,7 +732,6 @@ int vcycle(jg_solver* s, const T* r0, T* z0, const MgCfg<T>& c, const Ctl* ctl, 
             k_restrict<T><<<grid_sys(gc.grid, s), gc.block, 0, s->stream>>>(Prec<T>::t(lv), Prec<T>::b(s->lv[l + 1]),
                                                                cd, ctl);
         } else if (in) {
-            const bool from_t = pre_plan.back() == kLaunchMarch;  // that launch wrote the residual into t
             // restricting a stored residual is one load per cell: twice the
             // blocks (shorter chunks) keep more loads in flight
             const int zc = from_t ? rr_zc(cd, 2048) : rr_zc(cd);

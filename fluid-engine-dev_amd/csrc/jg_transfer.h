@@ -203,4 +203,115 @@ __global__ __launch_bounds__(kRrThreads, sizeof(T) == 4 ? 4 : 2) void k_residual
     }
 }
 
+// Residual and restriction of a small level in one launch, by bricks of
+// 8 x 4 x 4 coarse cells: a block forms the 18 x 10 x 10 residuals its taps
+// reach (FdmBlas3::residual's expression, src/jet/fdm_linear_system3.cpp:
+// 98-116) in LDS, every load of them independent, and restricts them with
+// FdmMgUtils3::restrict's sum (src/jet/fdm_mg_linear_system3.cpp:43-98).  On
+// levels of at most kRbMaxCells cells a launch costs its chain of latencies:
+// here one of loads and two barriers, where k_residual + k_restrict take two
+// launches and a round trip through memory, and k_residual_restrict a march
+// of planes.  16^3..64^3 cells, FP64: 5.6-7.2 us against 3.2 + 4.2 and the gap
+// between two launches; FP32: 5.2-5.6 us against 9.4.  A first version with
+// 8 x 8 x 4 tiles and a branch around each load took 7.6-9 us.  Past 2^18
+// cells (blocks of 32 KB LDS twice over the chip) the marches' fewer re-read
+// halo cells win.
+constexpr int kRbX = 8, kRbY = 4, kRbZ = 4, kRbThreads = 1024;
+constexpr idx_t kRbMaxCells = idx_t(1) << 18;
+
+template <typename T>
+__global__ __launch_bounds__(kRbThreads) void k_residual_restrict_brick(
+    const Row<T>* __restrict__ A, const T* __restrict__ x, const T* __restrict__ b,
+    T* __restrict__ coarse, Dims fd, Dims cd, const Ctl* __restrict__ ctl) {
+#pragma clang fp contract(off)
+    constexpr int FX = 2 * kRbX + 2, FY = 2 * kRbY + 2, FZ = 2 * kRbZ + 2;
+    const int nbz = (cd.nz + kRbZ - 1) / kRbZ;
+    const int sys = blockIdx.z / nbz, bz = blockIdx.z - sys * nbz;
+    if (sys > 0) {
+        A += sys * fd.n();
+        x += sys * fd.n();
+        b += sys * fd.n();
+        coarse += sys * cd.n();
+        if (ctl) ctl += sys * kSysCtl;
+    }
+    if (ctl && ctl->done) return;
+    __shared__ T r[FZ][FY][FX];
+    // fine cell of residual (0, 0, 0); taps beyond the grid are clamped into
+    // it when they are read, so what lies outside is never used
+    const int i0 = 2 * kRbX * (int)blockIdx.x - 1, j0 = 2 * kRbY * (int)blockIdx.y - 1, k0 = 2 * kRbZ * bz - 1;
+    const idx_t sy = fd.nx, sz = (idx_t)fd.nx * fd.ny;
+    // (addresses clamped into the grid instead of branches, so that all loads
+    // of a thread's cells are in flight together)
+    constexpr int N = (FX * FY * FZ + kRbThreads - 1) / kRbThreads;
+    struct Cell {
+        Row<T> row;
+        T rl, ud, fb, xc, xl, xr, xd, xu, xb, xf, bc;
+    } q[N];
+    auto coords = [&](int m, int& i, int& j, int& k) {
+        const int e = (int)threadIdx.x + kRbThreads * m;
+        i = min(max(i0 + e % FX, 0), fd.nx - 1);
+        j = min(max(j0 + e / FX % FY, 0), fd.ny - 1);
+        k = min(max(k0 + min(e / (FX * FY), FZ - 1), 0), fd.nz - 1);
+    };
+#pragma unroll
+    for (int m = 0; m < N; ++m) {
+        int i, j, k;
+        coords(m, i, j, k);
+        const idx_t c = i + sy * j + sz * k;
+        const idx_t l = i > 0 ? c - 1 : c, d = j > 0 ? c - sy : c, bk = k > 0 ? c - sz : c;
+        Cell& v = q[m];
+        v.row = A[c];
+        v.rl = A[l].r;
+        v.ud = A[d].u;
+        v.fb = A[bk].f;
+        v.xc = x[c];
+        v.xl = x[l];
+        v.xr = x[i + 1 < fd.nx ? c + 1 : c];
+        v.xd = x[d];
+        v.xu = x[j + 1 < fd.ny ? c + sy : c];
+        v.xb = x[bk];
+        v.xf = x[k + 1 < fd.nz ? c + sz : c];
+        v.bc = b[c];
+    }
+#pragma unroll
+    for (int m = 0; m < N; ++m) {
+        int i, j, k;
+        coords(m, i, j, k);
+        const Cell& v = q[m];
+        T s = v.bc - v.row.c * v.xc;
+        s -= i > 0 ? v.rl * v.xl : T(0);
+        s -= i + 1 < fd.nx ? v.row.r * v.xr : T(0);
+        s -= j > 0 ? v.ud * v.xd : T(0);
+        s -= j + 1 < fd.ny ? v.row.u * v.xu : T(0);
+        s -= k > 0 ? v.fb * v.xb : T(0);
+        s -= k + 1 < fd.nz ? v.row.f * v.xf : T(0);
+        const int e = (int)threadIdx.x + kRbThreads * m;
+        if (e < FX * FY * FZ) (&r[0][0][0])[e] = s;
+    }
+    __syncthreads();
+    const int t = threadIdx.x;
+    if (t >= kRbX * kRbY * kRbZ) return;
+    const int tx = t % kRbX, ty = t / kRbX % kRbY, tz = t / (kRbX * kRbY);
+    const int I = kRbX * blockIdx.x + tx, J = kRbY * blockIdx.y + ty, K = kRbZ * bz + tz;
+    if (I >= cd.nx || J >= cd.ny || K >= cd.nz) return;
+    const T kern[4] = {T(0.125), T(0.375), T(0.375), T(0.125)};
+    // tap a of coarse index C: fine 2C - 1 + a, clamped at the grid's edges
+    auto tap = [](int l, int a, int C, int n) {
+        return 2 * l + (a == 0 && C == 0 ? 1 : (a == 3 && C + 1 == n ? 2 : a));
+    };
+    T sum = 0;
+#pragma unroll
+    for (int z = 0; z < 4; ++z)
+#pragma unroll
+        for (int y = 0; y < 4; ++y) {
+            const T* row = r[tap(tz, z, K, cd.nz)][tap(ty, y, J, cd.ny)];
+#pragma unroll
+            for (int a = 0; a < 4; ++a) {
+                const T w = kern[a] * kern[y] * kern[z];
+                sum += w * row[tap(tx, a, I, cd.nx)];
+            }
+        }
+    coarse[I + (idx_t)cd.nx * (J + (idx_t)cd.ny * K)] = sum;
+}
+
 }  // namespace jg

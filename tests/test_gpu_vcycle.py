@@ -188,3 +188,21 @@ def test_vcycle_invalid_arguments(solver):
     bad = jetgpu.mg_params(sor=2.0)
     with pytest.raises(jetgpu.JgError):
         solver.mg_vcycle(bad, None, r, empty((8, 8, 8)))
+
+
+@pytest.mark.parametrize("shape,levels", [((30, 14, 18), 2), ((32, 16, 16), 2), ((34, 18, 14), 2),
+                                          ((18, 8, 256), 2), ((128, 32, 64), 2), ((130, 32, 64), 2)])
+def test_vcycle_residual_restriction_by_bricks(solver, oracle, shape, levels):
+    # the one-launch residual and restriction of small levels: coarse grids
+    # one less, equal to and one more than its 8 x 4 x 4 tiles, several tiles,
+    # the largest level that takes it (2^18 cells) and one that does not
+    print(f"case vcycle restrict brick shape={shape}", flush=True)
+    s = random_hierarchy(shape, levels, seed=41)
+    upload(solver, s)
+    r = np.random.default_rng(42).uniform(-1, 1, s.x[0].shape)
+    gp, op = params((2, 2, 4, 2), 1.3)
+    want = oracle.mg_clean_vcycle(s, op, r)
+    for precision, tol in ((jetgpu.JG_FP64, 1e-12), (jetgpu.JG_MIXED, 2e-5)):
+        z = empty(r.shape)
+        solver.mg_vcycle(gp, jetgpu.gpu_options(precision=precision, omega=1.3), dev(r), z)
+        assert rel_err(host(z), want) <= tol
