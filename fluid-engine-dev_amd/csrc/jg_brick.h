@@ -73,17 +73,40 @@ __global__ __launch_bounds__(kBkThreads, sizeof(T) == 4 ? 2 : 1) void k_brick_sw
     const int ib = (int)blockIdx.x * (kBkB / 2) - kBkH / 2 - 1;
     const int jb = (int)blockIdx.y * (kBkB / 2) - kBkH / 2 - 1;
     const int kb = bzl * (kBkB / 2) - kBkH / 2 - 1;
+    // Every global load of the block is issued here, the coarse cells' first,
+    // so that the barrier behind their staging does not add its latency to
+    // the rows'.
+    T cv = 0;
+    if (CORRECT && t < kCz * kCz * kCz) {
+        // coarse cell (ib, jb, kb) + (t % 10, t / 10 % 10, t / 100), each
+        // index clamped to the coarse grid
+        const int qi = t % kCz, qj = (t / kCz) % kCz, qk = t / (kCz * kCz);
+        const int cnx = d.nx / 2, cny = d.ny / 2, cnz = d.nz / 2;
+        const int ci = min(max(ib + qi, 0), cnx - 1);
+        const int cj = min(max(jb + qj, 0), cny - 1);
+        const int ck = min(max(kb + qk, 0), cnz - 1);
+        cv = coarse[ci + (idx_t)cnx * (cj + (idx_t)cny * ck)];
+    }
+    // Of two positions above each other a thread holds that of colour 0 first:
+    // a half-sweep then updates registers 0 and 2 or 1 and 3 of every lane
+    // (by height, every wave passed through four updates and their FP64
+    // divisions with half its lanes idle: 192x160x144 FP64 solve 2.88 ms, so
+    // 2.76 ms with the loads above).
+    Row<T> row[4];
+    T bv[4], xi[4];
+    bool ok[4];
+    const int odd = (gi + gj + gk0) & 1;
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+        const int gk = gk0 + (m ^ odd);
+        ok[m] = xyok && gk >= 0 && gk < d.nz;
+        const idx_t c = ok[m] ? gi + (idx_t)d.nx * (gj + (idx_t)d.ny * gk) : 0;
+        row[m] = A[c];
+        bv[m] = b[c];
+        xi[m] = ZERO ? T(0) : xin[c];
+    }
     if (CORRECT) {
-        // stage: thread t < 1000 loads coarse cell (ib, jb, kb) + (t % 10, t / 10 % 10, t / 100),
-        // each index clamped to the coarse grid
-        if (t < kCz * kCz * kCz) {
-            const int qi = t % kCz, qj = (t / kCz) % kCz, qk = t / (kCz * kCz);
-            const int cnx = d.nx / 2, cny = d.ny / 2, cnz = d.nz / 2;
-            const int ci = min(max(ib + qi, 0), cnx - 1);
-            const int cj = min(max(jb + qj, 0), cny - 1);
-            const int ck = min(max(kb + qk, 0), cnz - 1);
-            scz[qk][qj][qi] = coarse[ci + (idx_t)cnx * (cj + (idx_t)cny * ck)];
-        }
+        if (t < kCz * kCz * kCz) scz[t / (kCz * kCz)][(t / kCz) % kCz][t % kCz] = cv;
         __syncthreads();
         const int cnx = d.nx / 2, cny = d.ny / 2;
         const int hi = gi >> 1, hj = gj >> 1;  // gi, gj may be negative outside the grid
@@ -104,15 +127,10 @@ __global__ __launch_bounds__(kBkThreads, sizeof(T) == 4 ? 2 : 1) void k_brick_sw
     }
 
     T cw[4], bb[4];  // FP64: c; FP32: w = omega / c (0 for a zero-centre row)
-    bool ok[4];
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
-        const int lk = lk0 + m, gk = gk0 + m;
-        ok[m] = xyok && gk >= 0 && gk < d.nz;
-        const idx_t c = ok[m] ? gi + (idx_t)d.nx * (gj + (idx_t)d.ny * gk) : 0;
-        const Row<T> row = A[c];
-        const T bv = b[c];
-        T xv = ZERO ? T(0) : xin[c];
+        const int lk = lk0 + (m ^ odd), gk = gk0 + (m ^ odd);
+        T xv = xi[m];
         if (CORRECT && ok[m]) {
             int k0c, k1c;
             T w0, w1;
@@ -125,13 +143,13 @@ __global__ __launch_bounds__(kBkThreads, sizeof(T) == 4 ? 2 : 1) void k_brick_sw
             const T corr = wy0 * lo + wy1 * hi;
             xv += corr;
         }
-        const T cc = ok[m] ? row.c : T(1);
+        const T cc = ok[m] ? row[m].c : T(1);
         cw[m] = rb_coef<T>(omega, cc);  // FP32: w = omega / c; FP64: c
-        bb[m] = ok[m] ? bv : T(0);
+        bb[m] = ok[m] ? bv[m] : T(0);
         sx[lk][lj][li] = ok[m] ? xv : T(0);
-        sr[lk][lj][li] = ok[m] ? row.r : T(0);
-        su[lk][lj][li] = ok[m] ? row.u : T(0);
-        sf[lk][lj][li] = ok[m] ? row.f : T(0);
+        sr[lk][lj][li] = ok[m] ? row[m].r : T(0);
+        su[lk][lj][li] = ok[m] ? row[m].u : T(0);
+        sf[lk][lj][li] = ok[m] ? row[m].f : T(0);
     }
     __syncthreads();
 
@@ -139,10 +157,10 @@ __global__ __launch_bounds__(kBkThreads, sizeof(T) == 4 ? 2 : 1) void k_brick_sw
     for (int h = 1; h <= 4; ++h) {
         const int colour = (h & 1) ? FIRST : 1 - FIRST;
 #pragma unroll
-        for (int m = 0; m < 4; ++m) {
-            const int lk = lk0 + m;
+        for (int m = colour; m < 4; m += 2) {
+            const int lk = lk0 + (m ^ odd);
             const int ring = min(ring_xy, min(lk, kBkR - 1 - lk));
-            if (ring < h || !ok[m] || ((gi + gj + gk0 + m) & 1) != colour) continue;
+            if (ring < h || !ok[m]) continue;
             const T xo = sx[lk][lj][li];
             T xv;
             if (cw[m] == T(0)) {
@@ -166,10 +184,10 @@ __global__ __launch_bounds__(kBkThreads, sizeof(T) == 4 ? 2 : 1) void k_brick_sw
     // the brick: ring >= 4 in every direction
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
-        const int lk = lk0 + m;
+        const int lk = lk0 + (m ^ odd);
         const int ring = min(ring_xy, min(lk, kBkR - 1 - lk));
         if (ring >= kBkH && ok[m])
-            xout[gi + (idx_t)d.nx * (gj + (idx_t)d.ny * (gk0 + m))] = sx[lk][lj][li];
+            xout[gi + (idx_t)d.nx * (gj + (idx_t)d.ny * (gk0 + (m ^ odd)))] = sx[lk][lj][li];
     }
 }
 
