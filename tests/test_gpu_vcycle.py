@@ -206,3 +206,22 @@ def test_vcycle_residual_restriction_by_bricks(solver, oracle, shape, levels):
         z = empty(r.shape)
         solver.mg_vcycle(gp, jetgpu.gpu_options(precision=precision, omega=1.3), dev(r), z)
         assert rel_err(host(z), want) <= tol
+
+
+@pytest.mark.parametrize("shape,levels", [((14, 6, 6), 2), ((16, 8, 4), 2), ((10, 26, 2), 2), ((2, 2, 2), 2),
+                                          ((12, 4, 4), 3), ((3, 5, 7), 1), ((1, 3, 2), 1), ((16, 16, 8), 2),
+                                          ((16, 16, 16), 2), ((256, 4, 2), 2)])
+def test_vcycle_bottom_edges(solver, oracle, shape, levels):
+    # the one-workgroup bottom: coarsest grids of 63, 64 and 65 cells (one
+    # wave or several), of one cell, odd rows, a bottom of one level, the
+    # largest tops of both precisions, long thin rows
+    print(f"case vcycle bottom shape={shape}", flush=True)
+    s = random_hierarchy(shape, levels, seed=51)
+    upload(solver, s)
+    r = np.random.default_rng(52).uniform(-1, 1, s.x[0].shape)
+    gp, op = params((2, 2, 20, 2), 1.3)
+    want = oracle.mg_clean_vcycle(s, op, r)
+    for precision, tol in ((jetgpu.JG_FP64, 1e-12), (jetgpu.JG_MIXED, 2e-5)):
+        z = empty(r.shape)
+        solver.mg_vcycle(gp, jetgpu.gpu_options(precision=precision, omega=1.3), dev(r), z)
+        assert rel_err(host(z), want) <= tol
