@@ -144,12 +144,13 @@ def main():
             f"rel {infos[-1].rel_residual:.2e}")
 
     # Dominant kernel of the mixed solve: the finest level's smoothing.  A
-    # V(2,2) cycle on level 0 is two launches of it (the tuner pairs the two
-    # sweeps of each side into one launch wherever that is faster): the
+    # V(2,2) cycle on level 0 is two launches of it (the two sweeps of each
+    # side go into one launch wherever that is faster): the
     # pre-smoothing launch (x from zero, the residual written for the
     # restriction) and the post-smoothing launch (the coarse correction added
     # as x is loaded).  jg_solver_time_kernel replays exactly those launches,
-    # with the solve's sweep plan and tuning; HIP events on the solver's
+    # on the whole grid (a solve runs them on the box of cells that take
+    # part, where that is smaller); HIP events on the solver's
     # stream around 50 back-to-back launches.
     kern = {}
     for kname, kid in (("pre0", jg.JG_KERNEL_PRE0), ("post0", jg.JG_KERNEL_POST0),
@@ -294,7 +295,7 @@ def traffic_cells(traffic):
 
 def traffic_probe(args):
     """The program the counter passes run: the workload's system, warm-up
-    solves (tuning), then, each between two marker kernels (a torch fill that
+    solves, then, each between two marker kernels (a torch fill that
     the library never launches): one mixed solve, one FP64 solve, the pre- and
     the post-smoothing launch of level 0 and a copy kernel (the counters'
     scale), each 1 + 20 times."""
@@ -641,7 +642,7 @@ def diffusion_leg(jg, n, args):
             "build_and_coarsen_ms": round(build_ms + coarsen_ms, 3)}
     for name, prec in (("fp64", jg.JG_FP64), ("mixed", jg.JG_MIXED)):
         o = jg.gpu_options(precision=prec, stop_rule=jg.JG_STOP_RELATIVE, rel_tol=1e-8)
-        s.mgpcg(500, p, o)  # tuning
+        s.mgpcg(500, p, o)  # warm-up
         reps = 3
         torch.cuda.synchronize()
         t0 = time.perf_counter()
@@ -745,7 +746,7 @@ def mg2_leg(jg, args):
     out = {}
     for name, prec in (("fp64", jg.JG_FP64), ("mixed", jg.JG_MIXED)):
         o = jg.gpu_options(precision=prec, stop_rule=jg.JG_STOP_RELATIVE, rel_tol=1e-8)
-        s.mgpcg(200, p, o)  # warm-up: tuning and FP32 copies
+        s.mgpcg(200, p, o)  # warm-up: allocation and FP32 copies
         reps = 3
         torch.cuda.synchronize()
         t0 = time.perf_counter()
@@ -840,7 +841,7 @@ def _device_scene(jg, s, kind, n, seed):
 def _timed(fn, reps):
     import torch
 
-    fn()  # warm-up (allocation, tuning, FP32 copies)
+    fn()  # warm-up (allocation, FP32 copies)
     torch.cuda.synchronize()
     t0 = time.perf_counter()
     for _ in range(reps):
@@ -926,7 +927,7 @@ def batch_leg(jg, args):
     xs = {}
     for name, prec in (("fp64", jg.JG_FP64), ("mixed", jg.JG_MIXED)):
         o = jg.gpu_options(precision=prec, stop_rule=jg.JG_STOP_RELATIVE, rel_tol=1e-8)
-        b.mgpcg(500, p, o)  # tuning and graph capture
+        b.mgpcg(500, p, o)  # allocation and graph capture
         reps = 3
         torch.cuda.synchronize()
         t0 = time.perf_counter()
@@ -988,7 +989,7 @@ def torus_leg(jg, args):
     xs = {}
     for name, prec in (("fp64", jg.JG_FP64), ("mixed", jg.JG_MIXED)):
         o = jg.gpu_options(precision=prec, stop_rule=jg.JG_STOP_RELATIVE, rel_tol=1e-8)
-        s.mgpcg(300, p, o)  # tuning
+        s.mgpcg(300, p, o)  # warm-up
         torch.cuda.synchronize()
         t0 = time.perf_counter()
         info = s.mgpcg(300, p, o)

@@ -1323,7 +1323,7 @@ int levels_alloc(jg_solver* s, size_t nlev, const size_t* nx, const size_t* ny, 
     return JG_OK;
 }
 
-// Makes v a view of member i of group g: g's hierarchy and tuning, every
+// Makes v a view of member i of group g: g's hierarchy, every
 // pointer offset to member i's part of g's arrays, g's stream.
 void make_view(jg_solver* g, int i, jg_solver* v) {
     v->view = true;
@@ -2041,7 +2041,7 @@ Vecs<float> vecs32(jg_solver* s) { return {s->e32, s->rhs32, s->r32, s->z32, s->
 
 // The first level-0 launch of the pre-smoothing (post = false) or of the
 // post-smoothing (post = true) of a V(2,2) cycle, exactly as vcycle() issues
-// it: the sweep plan and tuning of the solve, b = r, the result in z (pre:
+// it: the sweep plan of the solve, b = r, the result in z (pre:
 // x starts at zero and, for a two-sweep launch, the residual is written for
 // the restriction; post: the coarse correction of level 1 is added as x is
 // loaded).

@@ -80,8 +80,8 @@ typedef struct {
     unsigned max_refine;     /* mixed: outer FP64 refinement steps (default 8) */
     double inner_rel_tol;    /* mixed: FP32 inner reduction per step (default 1e-4) */
     unsigned check_every;    /* host convergence poll interval in iterations (default 1) */
-    int sweep_pairs;         /* smoothing: two sweeps per launch where the tuner
-                                measured it faster (0, default), wherever two sweeps
+    int sweep_pairs;         /* smoothing: two sweeps per launch where it is
+                                the faster by size and type (0, default), wherever two sweeps
                                 follow each other (1), never (-1); the result is
                                 bit-identical either way */
 } jg_gpu_options;
@@ -324,8 +324,8 @@ enum {
     JG_KERNEL_SWEEP2 = 7,     /* two fused sweeps in one pass (JG_MIXED only);
                                  bytes = two sweeps' algorithmic bytes          */
     JG_KERNEL_PRE0 = 8,       /* the first level-0 pre-smoothing launch of a
-                                 V(2,2) cycle as the MGPCG solve issues it (its
-                                 sweep plan and tuning, omega 1.3); bytes = its
+                                 V(2,2) cycle as the MGPCG solve issues it on
+                                 the whole grid (omega 1.3); bytes = its
                                  sweeps plus the residual it writes           */
     JG_KERNEL_POST0 = 9       /* the first level-0 post-smoothing launch (the
                                  coarse correction added as x is loaded)      */
