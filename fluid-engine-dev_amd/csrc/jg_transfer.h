@@ -213,9 +213,9 @@ __global__ __launch_bounds__(kRrThreads, sizeof(T) == 4 ? 4 : 2) void k_residual
 // launches and a round trip through memory, and k_residual_restrict a march
 // of planes.  16^3..64^3 cells, FP64: 5.6-7.2 us against 3.2 + 4.2 and the gap
 // between two launches; FP32: 5.2-5.6 us against 9.4.  A first version with
-// 8 x 8 x 4 tiles and a branch around each load took 7.6-9 us.  Past 2^18
-// cells (blocks of 32 KB LDS twice over the chip) the marches' fewer re-read
-// halo cells win.
+// 8 x 8 x 4 tiles and a branch around each load took 7.6-9 us.  On a level
+// of 1.03 M cells the bricks' halo cells, read again, cost more than the
+// second launch (FP64 25.5 us against 14.1 + 7.0; 129 024 cells: 6.9).
 constexpr int kRbX = 8, kRbY = 4, kRbZ = 4, kRbThreads = 1024;
 constexpr idx_t kRbMaxCells = idx_t(1) << 18;
 
