@@ -322,7 +322,7 @@ __device__ __forceinline__ void bot_correct(const T* coarse, T* fine, const int*
                                             const Dims& fd) {
 #pragma clang fp contract(off)
     const int n = fd.nx * fd.ny * fd.nz;
-    const int cnx = fd.nx / 2, cnxy = cnx * (fd.ny / 2), kclamp = min(fd.ny, fd.nz);
+    const int cnx = fd.nx / 2, cnxy = cnx * (fd.ny / 2), kclamp = fd.kclamp();
     for (int c = threadIdx.x; c < n; c += kBotThreads) {
         int i, j, k;
         bot_unpack(Qf[c], i, j, k);
@@ -377,7 +377,7 @@ __global__ __launch_bounds__(kBotThreads) void k_bottom(BotLevels<T> bl, const T
         for (int m = 0; m < l; ++m) o += n0 >> (3 * m);
         return o;
     };
-    auto D = [&](int l) { return Dims{bl.d[0].nx >> l, bl.d[0].ny >> l, bl.d[0].nz >> l}; };
+    auto D = [&](int l) { return Dims{bl.d[0].nx >> l, bl.d[0].ny >> l, bl.d[0].nz >> l, bl.d[0].box}; };
     auto X = [&](int l) { return &sv[0][off(l)]; };
     auto B = [&](int l) { return &sv[1][off(l)]; };
     auto Rv = [&](int l) { return &sv[2][off(l)]; };

@@ -23,7 +23,15 @@ using idx_t = long;
 
 struct Dims {
     int nx, ny, nz;
+    bool box = false;  // the box of a solve (jg_box.h), not a grid of the caller's
     __host__ __device__ idx_t n() const { return (idx_t)nx * ny * nz; }
+    // Where the prolongation stops reaching up in z.  Jet's correct bounds k
+    // by min(ny, nz) (n.y in src/jet/fdm_mg_linear_system3.cpp:159), which only
+    // matters on grids with ny < nz.  A box of a cubic grid is often such a
+    // shape; bounding it so would make the cycle asymmetric where the
+    // grid's own is not (512^3 torus, a box of 512 x 192 x 512: 10 FP64
+    // iterations instead of 7).
+    __host__ __device__ int kclamp() const { return box || nz < ny ? nz : ny; }
 };
 
 // Smallest and largest cell that takes part in a solve, per axis (x, y, z;

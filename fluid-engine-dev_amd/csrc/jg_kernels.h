@@ -934,7 +934,7 @@ __global__ __launch_bounds__(NT) void k_correct(const TX* __restrict__ coarse,
     const int j = blockIdx.y * blockDim.y + threadIdx.y;
     if (i >= fd.nx || j >= fd.ny) return;
     const int cnx = fd.nx / 2, cny = fd.ny / 2;
-    const int kclamp = min(fd.ny, fd.nz);
+    const int kclamp = fd.kclamp();
     const int ci = i / 2, cj = j / 2, ck = k / 2;
     int i0, i1, j0, j1, k0, k1;
     TX wi0, wi1, wj0, wj1, wk0, wk1;

@@ -719,7 +719,7 @@ int vcycle(jg_solver* s, const T* r0, T* z0, const MgCfg<T>& c, const Ctl* ctl, 
         const Dims& cd = s->lv[l + 1].d;
         Geo gc = geo_planes(cd);
         const bool from_t = in && sizeof(T) == 4 && pre_plan.back() == kLaunchMarch;  // t holds the residual
-        if (in && !from_t && d.n() <= kRbMaxCells) {
+        if (in && !from_t && d.n() * s->nsys <= kRbMaxCells) {
             const dim3 grid = grid_sys(dim3((cd.nx + kRbX - 1) / kRbX, (cd.ny + kRbY - 1) / kRbY,
                                             (cd.nz + kRbZ - 1) / kRbZ), s);
             k_residual_restrict_brick<T><<<grid, kRbThreads, 0, s->stream>>>(
@@ -1624,7 +1624,7 @@ int solve_in_box(jg_solver* s, size_t L, idx_t from, double most, bool mixed, Ru
         const Dims full = lv.d;
         Box bl = box;
         for (int a = 0; a < 3; ++a) bl.o[a] >>= (a == 2 && s->twod) ? 0 : l;
-        bl.n = Dims{box.n.nx >> l, box.n.ny >> l, s->twod ? 1 : box.n.nz >> l};
+        bl.n = Dims{box.n.nx >> l, box.n.ny >> l, s->twod ? 1 : box.n.nz >> l, true};
         lv.d = bl.n;
         const Geo g = geo_planes(l == 0 ? bl.n : full);
         Row<double>* const to64 = !mixed || l == 0 ? rows : nullptr;

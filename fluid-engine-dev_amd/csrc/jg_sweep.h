@@ -99,13 +99,13 @@ constexpr int kCzX = kSwLX / 2 + 2, kCzY = kSwLY / 2 + 2;
 static_assert(kCzX * kCzY <= kSwLX * kSwLY / 2, "one coarse entry per thread");
 
 // Prolongation value at fine (i, j, k) (clamped trilinear 1/4-3/4, with the
-// k clamp bounded by min(ny, nz) like k_correct), in Jet's accumulation order.
+// k clamp of Dims::kclamp like k_correct), in Jet's accumulation order.
 template <typename T>
 __device__ __forceinline__ T prolong_at(const T* __restrict__ coarse, int i, int j, int k,
                                         const Dims& fd) {
 #pragma clang fp contract(off)
     const int cnx = fd.nx / 2, cny = fd.ny / 2;
-    const int kclamp = min(fd.ny, fd.nz);
+    const int kclamp = fd.kclamp();
     const int ci = i / 2, cj = j / 2, ck = k / 2;
     int iI[2], jI[2], kI[2];
     T iW[2], jW[2], kW[2];
@@ -138,7 +138,7 @@ __device__ __forceinline__ void prolong_z(int t, const Dims& fd, int& k0, int& k
         w1 = T(0.75);
     } else {
         k0 = ck;
-        k1 = tc + 1 < min(fd.ny, fd.nz) ? ck + 1 : ck;
+        k1 = tc + 1 < fd.kclamp() ? ck + 1 : ck;
         w0 = T(0.75);
         w1 = T(0.25);
     }

@@ -208,7 +208,7 @@ __global__ __launch_bounds__(kRrThreads, sizeof(T) == 4 ? 4 : 2) void k_residual
 // reach (FdmBlas3::residual's expression, src/jet/fdm_linear_system3.cpp:
 // 98-116) in LDS, every load of them independent, and restricts them with
 // FdmMgUtils3::restrict's sum (src/jet/fdm_mg_linear_system3.cpp:43-98).  On
-// levels of at most kRbMaxCells cells a launch costs its chain of latencies:
+// levels of at most kRbMaxCells cells (all systems together) a launch costs its chain of latencies:
 // here one of loads and two barriers, where k_residual + k_restrict take two
 // launches and a round trip through memory, and k_residual_restrict a march
 // of planes.  16^3..64^3 cells, FP64: 5.6-7.2 us against 3.2 + 4.2 and the gap
