@@ -1104,13 +1104,11 @@ __global__ __launch_bounds__(NT) void k_correct2(const TX* __restrict__ coarse,
 
 // ------------------------------------------------------------- finalize
 
-// The control block as the host sees it: two pinned slots, the one of
-// iteration k (0: the start) at k & 1.  The finalize kernels write it there
-// themselves; the host waits for an event behind them, and no copy runs
-// between the iterations.  host: nullptr when nobody polls (a batch's graph).
-__device__ __forceinline__ void ctl_to_host(const Ctl* ctl, Ctl* host, unsigned k) {
-    if (host) host[k & 1] = *ctl;
-}
+// host: the pinned copy of the control block that the launch's poll reads
+// (pcg_device), nullptr when nobody polls (a batch's graph).  The finalize
+// kernels write it themselves; the host waits for an event behind them, and no
+// copy runs between the iterations.  Once a solve has stopped, nothing is
+// written any more.
 
 // Initial PCG scalars: sigma = r.z, rr = r.r, bb = b.b (for the relative
 // rule), beta = 0 so the first fused direction update gives d = z.
@@ -1137,7 +1135,7 @@ __global__ __launch_bounds__(kFinThreads) void k_fin_init(Ctl* ctl, const double
         ctl->nonfinite = !isfinite(rz) || !isfinite(rr);
         const bool go = (ctl->stop_rule == 1) ? (rr > ctl->rel2 * ctl->bb) : (rz > ctl->tol2);
         ctl->done = !(go && ctl->iter < ctl->max_iter) || ctl->nonfinite;
-        ctl_to_host(ctl, host, 0);
+        if (host) *host = *ctl;
     }
 }
 
@@ -1163,7 +1161,7 @@ __global__ __launch_bounds__(kFinThreads) void k_fin_alpha(Ctl* ctl, const doubl
         if (!isfinite(alpha)) {
             ctl->nonfinite = 1;
             ctl->done = 1;
-            ctl_to_host(ctl, host, iter + 1);
+            if (host) *host = *ctl;
         }
     }
 }
@@ -1196,7 +1194,7 @@ __global__ __launch_bounds__(kFinThreads) void k_fin_sigma(Ctl* ctl, const doubl
         if (!isfinite(rz) || !isfinite(rr)) c.nonfinite = 1;
         c.done = !(go && c.iter < c.max_iter) || c.nonfinite;
         *ctl = c;
-        if (host) host[c.iter & 1] = c;
+        if (host) *host = c;
     }
 }
 

@@ -805,7 +805,6 @@ struct Pcg {
     const MgCfg<T>* mg;  // nullptr: no preconditioner (z aliases r)
     const CsrDev* csr = nullptr;  // compressed system (FP64, no preconditioner): A unused, d = {rows, 1, 1}
     const EllDev* ell = nullptr;  // its ELL copy, when it has one
-    bool polled = true;  // the host polls the control block (not in a batch's graph)
 };
 
 // z = M r and the r.z / r.r partials in slots 0 / 1 (from the V-cycle's last
@@ -880,9 +879,10 @@ int pcg_init(jg_solver* s, const Pcg<T>& v) {
 // One iteration of Jet's pcg loop (include/jet/detail/cg-inl.h:52-91) on the
 // device; every kernel is gated by the control block, so iterations can be
 // launched (or replayed from a graph) past convergence.  odd: the two
-// direction buffers swap roles every iteration.
+// direction buffers swap roles every iteration.  host: where the host polls
+// the control block (nullptr: nowhere).
 template <typename T>
-int pcg_iteration(jg_solver* s, const Pcg<T>& v, bool odd) {
+int pcg_iteration(jg_solver* s, const Pcg<T>& v, bool odd, Ctl* host) {
     const idx_t n = v.d.n();
     const int nb1 = nblocks_1d(n);
     T* dold = odd ? v.dB : v.dA;
@@ -899,7 +899,7 @@ int pcg_iteration(jg_solver* s, const Pcg<T>& v, bool odd) {
             } else
                 k_csr_dir_spmv<<<nb1, NT, 0, s->stream>>>(*v.csr, v.z, dold, dnew, v.q, n,
                                                           s->slot(2), v.ctl);
-            k_fin_alpha<<<1, kFinThreads, 0, s->stream>>>(v.ctl, s->slot(2), nb1, s->ctl_host);
+            k_fin_alpha<<<1, kFinThreads, 0, s->stream>>>(v.ctl, s->slot(2), nb1, host);
             k_update_xr<T, true><<<nb1, NT, 0, s->stream>>>(v.x, v.r, dnew, v.q, n, s->slot(0), v.ctl);
             if (v.ell)
                 k_ell_residual<true, true><<<nb1, NT, 0, s->stream>>>(*v.ell, v.x, v.b, v.r, s->slot(0),
@@ -907,12 +907,10 @@ int pcg_iteration(jg_solver* s, const Pcg<T>& v, bool odd) {
             else
                 k_csr_residual<true, true><<<nb1, NT, 0, s->stream>>>(*v.csr, v.x, v.b, v.r, n,
                                                                       s->slot(0), v.ctl);
-            k_fin_sigma<<<1, kFinThreads, 0, s->stream>>>(v.ctl, s->slot(0), s->slot(0), nb1, nb1,
-                                                          s->ctl_host);
+            k_fin_sigma<<<1, kFinThreads, 0, s->stream>>>(v.ctl, s->slot(0), s->slot(0), nb1, nb1, host);
             return check_launch(s, "csr pcg iteration");
         }
     }
-    Ctl* const host = v.polled ? s->ctl_host : nullptr;
     const int nsp = launch_dir_spmv<T>(s, v.A, v.z, dold, dnew, v.q, v.d, s->slot(2), v.ctl);
     k_fin_alpha<<<s->nsys, kFinThreads, 0, s->stream>>>(v.ctl, s->slot(2), nsp, host);
     if (!v.mg) {  // z = r: sigma is r.r
@@ -992,22 +990,30 @@ int pcg_device(jg_solver* s, const Pcg<T>& v, unsigned check_every) {
     const Ctl c0 = *s->ctl_host;
     const double lim = c0.stop_rule == 1 ? c0.rel2 * c0.bb : c0.tol2;
     double m_prev = -1.0, m_last = metric(c0);
+    // Iteration k (from 1) belongs to the poll after its check_every, and every
+    // iteration of a poll writes the poll's slot: the poll finds there the last
+    // iteration that ran, its own or the one that stopped the solve, and the
+    // iteration of look-ahead in flight by then writes the other slot.
+    auto slot_of = [&](unsigned k) { return (int)(((k - 1) / check_every + 1) & 1); };
     unsigned launched = 0;
-    int slot = 0;  // of the iteration polled: its number's parity (ctl_to_host)
-    JG_TRY(pcg_iteration<T>(s, v, false));
-    ++launched;
+    auto iterate = [&]() -> int {
+        const int st = pcg_iteration<T>(s, v, (launched & 1) != 0, s->ctl_host + slot_of(launched + 1));
+        ++launched;
+        return st;
+    };
+    int slot = 0;  // of the iteration polled
+    JG_TRY(iterate());
     while (true) {
         const bool poll = launched % check_every == 0 || launched >= max_iter;
         if (poll) {
-            slot = (int)(launched & 1);
+            slot = slot_of(launched);
             JG_HIP(hipEventRecord(s->evp[slot], s->stream));
         }
         bool more = launched <= max_iter;  // the device stops by itself at max_iter
         const bool likely_last = poll && m_prev > 0.0 && m_last > 0.0 && m_last < m_prev &&
                                  m_last * (m_last / m_prev) <= lim;
         if (more && !likely_last) {
-            JG_TRY(pcg_iteration<T>(s, v, (launched & 1) != 0));
-            ++launched;
+            JG_TRY(iterate());
             more = false;  // already launched this pass
         }
         if (poll) {
@@ -1023,8 +1029,7 @@ int pcg_device(jg_solver* s, const Pcg<T>& v, unsigned check_every) {
             m_last = metric(c);
         }
         if (more) {  // the prediction was wrong: go on
-            JG_TRY(pcg_iteration<T>(s, v, (launched & 1) != 0));
-            ++launched;
+            JG_TRY(iterate());
         } else if (launched > max_iter) {
             break;
         }
@@ -2492,13 +2497,12 @@ void group_residual(jg_solver* g, TR* r, int at) {
 // its first member's pointers, which every launch extends to all members).
 Pcg<double> pcg64(jg_solver* s, const MgCfg<double>* mg) {
     Level& l0 = s->lv[0];
-    return Pcg<double>{l0.A64, s->b, s->x, s->r, s->z, s->dA, s->dB, s->q, l0.d, s->ctl, mg,
-                       nullptr, nullptr, false};
+    return Pcg<double>{l0.A64, s->b, s->x, s->r, s->z, s->dA, s->dB, s->q, l0.d, s->ctl, mg};
 }
 Pcg<float> pcg32(jg_solver* s, const MgCfg<float>* mg) {
     Level& l0 = s->lv[0];
     return Pcg<float>{l0.A32, s->rhs32, s->e32, s->r32, s->z32, s->d32A, s->d32B, s->q32, l0.d,
-                      s->ctl + 1, mg, nullptr, nullptr, false};
+                      s->ctl + 1, mg};
 }
 
 // Captures kBatchIters PCG iterations of every group into one graph (or
@@ -2522,9 +2526,9 @@ int batch_graph(jg_batch* B, int precision, const MgCfg<T>& mg, hipGraphExec_t* 
         }
         for (int k = 0; k < kBatchIters && st == JG_OK; ++k) {
             if constexpr (sizeof(T) == 8)
-                st = pcg_iteration<double>(g, pcg64(g, &mg), (k & 1) != 0);
+                st = pcg_iteration<double>(g, pcg64(g, &mg), (k & 1) != 0, nullptr);
             else
-                st = pcg_iteration<float>(g, pcg32(g, &mg), (k & 1) != 0);
+                st = pcg_iteration<float>(g, pcg32(g, &mg), (k & 1) != 0, nullptr);
         }
         if (st == JG_OK && (hipEventRecord(B->join[gi], g->stream) != hipSuccess ||
                             hipStreamWaitEvent(B->stream, B->join[gi], 0) != hipSuccess))

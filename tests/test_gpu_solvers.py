@@ -174,6 +174,36 @@ def test_mgpcg_closed_sphere_singular(solver, oracle):
         assert rel_err_mean_free(x, xc, fluid) <= 1e-6
 
 
+@pytest.mark.parametrize("precision", [jetgpu.JG_FP64, jetgpu.JG_MIXED])
+def test_mgpcg_poll_interval(solver, precision):
+    # The host looks at the stop flag every check_every iterations; whichever
+    # iteration of an interval stops the solve, the host sees it at the next
+    # look.  A stop that goes unseen enqueues no-op iterations up to max_iter
+    # (20000 of 18 launches: about a second against a millisecond).
+    s = mg_poisson_hierarchy(4, 4)
+    upload_mg(solver, s)
+    p = jetgpu.mg_params(max_levels=4, restrict_iter=2, correct_iter=2, coarsest_iter=20,
+                         final_iter=2)
+    stops = set()
+    for tol in (1e-2, 1e-3, 1e-4, 1e-5, 1e-6, 1e-7, 1e-8, 1e-9):
+        base, want = None, None
+        for every in (1, 2, 3, 4, 8, 2 ** 32 - 1):
+            print(f"case poll interval precision={precision} tol={tol} every={every}", flush=True)
+            # (an interval beyond max_iter: the only look is at max_iter)
+            limit = 200 if every > 8 else 20000
+            info = solver.mgpcg(limit, p, jetgpu.gpu_options(
+                precision=precision, stop_rule=jetgpu.JG_STOP_RELATIVE, rel_tol=tol, check_every=every))
+            x = solver.download_x()
+            if every == 1:
+                base, want = info, x
+                stops.add(int(info.iterations) % 2)
+            assert info.iterations == base.iterations and info.rel_residual == base.rel_residual
+            assert np.array_equal(x, want)
+            if every <= 8:
+                assert info.solve_ms <= 10 * base.solve_ms, (every, info.solve_ms, base.solve_ms)
+    assert stops == {0, 1}
+
+
 def test_mgpcg_zero_rhs(solver):
     s = mg_poisson_hierarchy(4, 3)
     s.b[0][:] = 0.0
