@@ -21,7 +21,8 @@
 // atomics, which go through the XCDs' private L2s; a block waits for its
 // stores before its slot is written.  The blocks of a cooperative launch are
 // resident together, so the waits end; a wait that does not within
-// kCgSpins polls makes every block leave and the solve fail.
+// CgGridArgs::polls makes every block leave, and the solve starts again as the
+// loop of one launch per step (so does one whose launch is refused).
 //
 // At 64^3 an iteration takes 7.9 us: 2.7 and 3.2 (with the wait for the
 // published r) in the two sums, the rest the loads of the neighbours' r
@@ -44,7 +45,6 @@ constexpr int kCgCopies = 8;        // copies of the slots
 constexpr int kCgCopyWords = kCgMaxBlocks * 4;
 constexpr int kCgSumWords = kCgCopies * kCgCopyWords;  // of one kind of grid sum
 constexpr int kCgW = 7;             // entries of a row
-constexpr int kCgSpins = 1 << 23;
 constexpr int kCgChunk = 2048;      // iterations per launch
 
 struct CgGridArgs {
@@ -55,6 +55,7 @@ struct CgGridArgs {
     double *x, *r, *dir;   // state in and out: iterate, residual, last direction
     Ctl* ctl;
     unsigned long long* slots;  // [3][kCgSumWords], zero at launch
+    int polls;                  // bound of a wait for the other blocks
 };
 
 __device__ __forceinline__ void agent_store(unsigned long long* p, unsigned long long v) {
@@ -92,7 +93,7 @@ struct CgShared {
 // 1.6 with 64, 1.9 with 128, 2.6 with 256 (one packed copy and shuffles: 2.9,
 // 3.2, 4.1, 4.5).
 __device__ __forceinline__ bool grid_sum(double v, unsigned long long* slots, unsigned epoch,
-                                         CgShared& sh, double& sum) {
+                                         int polls, CgShared& sh, double& sum) {
     const int t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
     const int G = gridDim.x, step = G <= 128 ? 4 : 2;
     v = wave_sum(v);
@@ -117,11 +118,11 @@ __device__ __forceinline__ bool grid_sum(double v, unsigned long long* slots, un
         if (t < G) {
             const unsigned long long* from = slots + (blockIdx.x % kCgCopies) * kCgCopyWords + step * t;
             unsigned long long lo, hi;
-            int spins = 0;
+            int polled = 0;
             do {
                 lo = agent_load(from);
                 hi = agent_load(from + 1);
-                bad = ++spins > kCgSpins;
+                bad = ++polled > polls;
             } while (!bad && ((unsigned)(lo >> 32) != epoch || (unsigned)(hi >> 32) != epoch));
             p = __builtin_bit_cast(double, hi << 32 | (lo & 0xffffffffull));
         }
@@ -284,7 +285,7 @@ __global__ __launch_bounds__(kCgThreads) void k_cg_grid(CgGridArgs a) {
             for (int e = 0; e < kCgW; ++e) s[q] += val[q][e] * dl[at(q, e)];
             acc += d[q] * s[q];
         }
-        ok = grid_sum(acc, slot_dq, epoch, sh, dq);
+        ok = grid_sum(acc, slot_dq, epoch, a.polls, sh, dq);
         if (!ok) break;
         // k_fin_alpha
         dq = lane_value(dq, 0);
@@ -309,7 +310,7 @@ __global__ __launch_bounds__(kCgThreads) void k_cg_grid(CgGridArgs a) {
                 if (c < n) agent_store(at32(a.x, c), x[q]);
             }
             double none;
-            ok = grid_sum(0.0, slot_x, epoch, sh, none);
+            ok = grid_sum(0.0, slot_x, epoch, a.polls, sh, none);
             if (!ok) break;
 #pragma unroll
             for (int q = 0; q < C; ++q) {
@@ -337,7 +338,7 @@ __global__ __launch_bounds__(kCgThreads) void k_cg_grid(CgGridArgs a) {
             if (c < n) agent_store(at32(a.r, c), r[q]);
         }
         double rz;
-        ok = grid_sum(acc, slot_rr, epoch, sh, rz);
+        ok = grid_sum(acc, slot_rr, epoch, a.polls, sh, rz);
         if (!ok) break;
         // k_fin_sigma (z = r)
         rz = lane_value(rz, 0);

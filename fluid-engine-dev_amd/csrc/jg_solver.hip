@@ -936,17 +936,25 @@ int pcg_iteration(jg_solver* s, const Pcg<T>& v, bool odd, Ctl* host) {
 // cost less.
 int cg_grid_rows(jg_solver* s, const Pcg<double>& v) {
     const idx_t n = v.d.n(), per = (idx_t)std::min(s->cus, kCgMaxBlocks) * kCgThreads;
-    if (v.mg || s->nsys > 1 || !s->cooperative || n > 2 * per) return 0;
+    if (v.mg || s->nsys > 1 || !s->cooperative || s->cg_polls <= 0 || n > 2 * per) return 0;
     if (v.csr && (!v.ell || s->csr.ell_w > kCgW)) return 0;
     return n > per ? 2 : 1;
 }
 
 // pcg_device through k_cg_grid; the state after pcg_init in, x and the
-// control block out.
-int cg_grid(jg_solver* s, const Pcg<double>& v, int C) {
-    if (!s->cg_slots) JG_TRY(dalloc(s, &s->cg_slots, 3 * kCgSumWords));
+// control block out.  *ran is false where that launch is not to be had (no
+// room for its slots, refused, or a block did not arrive in time): the caller
+// starts again without it, and so does every later solve of s.
+int cg_grid(jg_solver* s, const Pcg<double>& v, int C, bool* ran) {
+    *ran = false;
+    if (!s->cg_slots && dalloc(s, &s->cg_slots, 3 * kCgSumWords) != JG_OK) {
+        (void)hipGetLastError();
+        s->err.clear();
+        s->cooperative = false;
+        return JG_OK;
+    }
     const idx_t n = v.d.n();
-    CgGridArgs a{v.A, v.ell ? *v.ell : EllDev{}, v.d, v.b, v.x, v.r, v.dA, v.ctl, s->cg_slots};
+    CgGridArgs a{v.A, v.ell ? *v.ell : EllDev{}, v.d, v.b, v.x, v.r, v.dA, v.ctl, s->cg_slots, s->cg_polls};
     const dim3 grid((unsigned)((n + (idx_t)C * kCgThreads - 1) / ((idx_t)C * kCgThreads)));
     const void* f = v.ell ? (C == 1 ? (const void*)k_cg_grid<1, true> : (const void*)k_cg_grid<2, true>)
                           : (C == 1 ? (const void*)k_cg_grid<1, false> : (const void*)k_cg_grid<2, false>);
@@ -954,14 +962,22 @@ int cg_grid(jg_solver* s, const Pcg<double>& v, int C) {
     do {
         k_fill<unsigned long long><<<nblocks_1d(3 * kCgSumWords), NT, 0, s->stream>>>(s->cg_slots, 0ull,
                                                                                   3 * kCgSumWords);
-        JG_HIP(hipLaunchCooperativeKernel(f, grid, dim3(kCgThreads), args, 0, s->stream));
+        const bool refused =
+            hipLaunchCooperativeKernel(f, grid, dim3(kCgThreads), args, 0, s->stream) != hipSuccess;
+        if (refused) (void)hipGetLastError();
         JG_HIP(hipMemcpyAsync(s->ctl_host, v.ctl, sizeof(Ctl), hipMemcpyDeviceToHost, s->stream));
         JG_TRY(sync(s));
+        if (refused || s->ctl_host->pad) {
+            s->cooperative = false;
+            return JG_OK;
+        }
     } while (!s->ctl_host->done);
-    if (s->ctl_host->pad) {
-        s->err = "CG: a block of the cooperative launch did not arrive";
-        return JG_ERR_HIP;
-    }
+    *ran = true;
+    return JG_OK;
+}
+
+int upload_ctl(jg_solver* s, Ctl* dev, const Ctl& h) {
+    JG_HIP(hipMemcpyAsync(dev, &h, sizeof(Ctl), hipMemcpyHostToDevice, s->stream));
     return JG_OK;
 }
 
@@ -974,7 +990,22 @@ int pcg_device(jg_solver* s, const Pcg<T>& v, unsigned check_every) {
     JG_TRY(pcg_init<T>(s, v));
     if constexpr (sizeof(T) == 8) {
         const int rows = cg_grid_rows(s, v);
-        if (rows) return cg_grid(s, v, rows);
+        if (rows) {
+            bool ran = false;
+            JG_TRY(cg_grid(s, v, rows, &ran));
+            if (ran) return JG_OK;
+            JG_TRY(sync(s));
+            const Ctl c = *s->ctl_host;
+            Ctl h;
+            std::memset(&h, 0, sizeof(Ctl));
+            h.max_iter = c.max_iter;
+            h.tol2 = c.tol2;
+            h.stop_rule = c.stop_rule;
+            h.rel2 = c.rel2;
+            JG_TRY(upload_ctl(s, v.ctl, h));
+            k_fill<T><<<nblocks_1d(v.d.n()), NT, 0, s->stream>>>(v.x, T(0), v.d.n());
+            JG_TRY(pcg_init<T>(s, v));
+        }
     }
     JG_TRY(sync(s));
     if (s->ctl_host->done) return JG_OK;
@@ -1044,11 +1075,6 @@ void init_ctl(Ctl* h, unsigned max_iter, double tol, int stop_rule, double rel_t
     h->tol2 = tol * tol;
     h->stop_rule = stop_rule;
     h->rel2 = rel_tol * rel_tol;
-}
-
-int upload_ctl(jg_solver* s, Ctl* dev, const Ctl& h) {
-    JG_HIP(hipMemcpyAsync(dev, &h, sizeof(Ctl), hipMemcpyHostToDevice, s->stream));
-    return JG_OK;
 }
 
 int ensure_f32(jg_solver* s) {
@@ -1596,6 +1622,7 @@ int solve_in_box(jg_solver* s, size_t L, idx_t from, double most, bool mixed, Ru
     v.device = s->device;
     v.cus = s->cus;
     v.cooperative = s->cooperative;
+    v.cg_polls = s->cg_polls;
     v.view = true;
     v.stream = s->stream;
     v.ev0 = s->ev0;
@@ -1656,6 +1683,7 @@ int solve_in_box(jg_solver* s, size_t L, idx_t from, double most, bool mixed, Ru
     // the solver's own parts stay with s
     bad = s->box_host->lo[0];
     s->cg_slots = v.cg_slots;
+    s->cooperative = v.cooperative;
     s->allocs.insert(s->allocs.end(), v.allocs.begin(), v.allocs.end());
     v.allocs.clear();
     if (!v.err.empty()) s->err = v.err;
@@ -1813,6 +1841,12 @@ int jg_solver_cg(jg_solver* s, unsigned max_iter, double tol, jg_solve_info* inf
                         [&](jg_solver* v, const std::function<int()>& finish) {
                             return cg_run(v, max_iter, tol, info, finish);
                         });
+}
+
+int jg_solver_cg_polls(jg_solver* s, unsigned polls) {
+    if (!s) return JG_ERR_INVALID_ARG;
+    s->cg_polls = (int)std::min(polls, 1u << 30);
+    return JG_OK;
 }
 
 int jg_mg_vcycle(jg_solver* s, const jg_mg_params* p, const jg_gpu_options* o, const double* r,

@@ -133,6 +133,7 @@ SIGNATURES = {
     "jg_sp_build2": (C.c_int, [_vp, _vp, _vp, _vp, _vp, C.c_double, C.c_double]),
     "jg_sp_apply_gradient2": (C.c_int, [_vp, _vp, _vp, _vp, _vp, C.c_double, C.c_double]),
     "jg_mg_correct2": (C.c_int, [_vp, _sz, _sz, _vp, _vp]),
+    "jg_solver_cg_polls": (C.c_int, [_vp, _u]),
     "jg_solver_time_kernel": (C.c_int, [_vp, C.c_int, C.c_int, _u, C.POINTER(_d), C.POINTER(_d)]),
     "jg_sp_build": (C.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _d, _d, _d]),
     "jg_sp_apply_gradient": (C.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _d, _d, _d]),
@@ -329,6 +330,10 @@ class Solver:
         info = SolveInfo()
         self.check(lib().jg_solver_cg(self.h, max_iter, tol, C.byref(info)), "cg")
         return info
+
+    def cg_polls(self, polls):
+        """Bound of a wait in the one-launch CG (0: one launch per step instead)."""
+        self.check(lib().jg_solver_cg_polls(self.h, polls), "cg_polls")
 
     def cg_host(self, A, b, max_iter, tol):
         """jg_cg_solve_host on host arrays: A (nz, ny, nx, 4) Jet rows, b (nz, ny, nx)."""

@@ -179,14 +179,22 @@ def test_compressed_free_surface_kat_on_device(solver, oracle):
     assert np.all(p[:, 2, :] == 0.0)
 
 
+@pytest.mark.parametrize("polls", [1 << 23, 0, 1])
 @pytest.mark.parametrize("n,fluid", [((11, 10, 10), 0.93), ((72, 64, 64), 0.95), ((80, 72, 72), 0.9),
                                      ((96, 96, 72), 0.95)])
-def test_csr_cg_one_launch_matches_oracle(solver, oracle, n, fluid):
+def test_csr_cg_one_launch_matches_oracle(oracle, n, fluid, polls):
     # compressed systems over the ranges of the one-launch CG: one block of
-    # rows, one row per thread, two rows per thread, and the per-kernel loop
-    print(f"case csr one launch n={n}", flush=True)
+    # rows, one row per thread, two rows per thread, and the per-kernel loop;
+    # and the same without that launch (polls 0) and where its blocks give up
+    # waiting (polls 1), which starts the solve again
+    print(f"case csr one launch n={n} polls={polls}", flush=True)
     m, _, (val, rp, ci, b) = pressure_csr(oracle, n, 9, fluid=fluid, solid=False)
     xo, oko, io, _ = oracle.csr_cg_solve(val, rp, ci, b, 400, 1e-8)
-    x, info = solver.csr_cg(val, rp, ci, b, 400, 1e-8)
+    s = jetgpu.Solver(0)
+    try:
+        s.cg_polls(polls)
+        x, info = s.csr_cg(val, rp, ci, b, 400, 1e-8)
+    finally:
+        s.close()
     assert abs(int(info.iterations) - io) <= 2 and bool(info.converged) == oko
     np.testing.assert_allclose(x, xo, rtol=0, atol=1e-7 * max(1.0, np.abs(xo).max()))

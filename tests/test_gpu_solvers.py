@@ -46,11 +46,14 @@ def test_cg_2x2_known_answer(solver):
     assert info.iterations <= 2 and info.last_residual <= 1e-15
 
 
-# (the last two take the tiled z-march: partial 64 x 8 x 16 tiles in x, y and z)
+# polls 0: one launch per step instead of the one cooperative launch these sizes
+# take (the last two then take the tiled z-march: partial 64 x 8 x 16 tiles in x,
+# y and z)
+@pytest.mark.parametrize("polls", [1 << 23, 0])
 @pytest.mark.parametrize("shape,tol", [((3, 3, 3), 1e-9), ((16, 12, 10), 1e-10), ((40, 40, 40), 1e-9),
                                        ((100, 20, 37), 1e-10), ((64, 13, 50), 1e-10)])
-def test_cg_matches_oracle(solver, oracle, shape, tol):
-    print(f"case cg shape={shape}", flush=True)
+def test_cg_matches_oracle(solver, oracle, shape, tol, polls):
+    print(f"case cg shape={shape} polls={polls}", flush=True)
     rng = np.random.default_rng(21)
     nx, ny, nz = shape
     A = random_stencil(nx, ny, nz, rng)
@@ -58,7 +61,11 @@ def test_cg_matches_oracle(solver, oracle, shape, tol):
     xo, io, ro, oko = oracle.cg_solve(A, b, 1000, tol)
     solver.set_levels([shape])
     solver.upload(0, A, b)
-    info = solver.cg(1000, tol)
+    solver.cg_polls(polls)
+    try:
+        info = solver.cg(1000, tol)
+    finally:
+        solver.cg_polls(1 << 23)
     x = solver.download_x()
     assert abs(int(info.iterations) - io) <= 2 and bool(info.converged) == oko
     assert info.last_residual <= tol
@@ -274,6 +281,34 @@ def test_cg_one_launch_matches_oracle(solver, oracle, shape):
     again = solver.cg(600, 1e-8)
     assert again.iterations == info.iterations and np.array_equal(solver.download_x(), x)
     assert solver.cg(37, 0.0).iterations == 37
+
+
+@pytest.mark.parametrize("shape", [(64, 64, 64), (65, 64, 64), (120, 100, 90), (1024, 512, 1)])
+def test_cg_wait_that_runs_out_is_no_error(shape):
+    # a block that gives up after two polls: every block leaves, and the solve
+    # starts again as the loop of one launch per step (the third grid in its box)
+    print(f"case cg wait runs out shape={shape}", flush=True)
+    nx, ny, nz = shape
+    A, _ = poisson_helper(nx, ny, nz)
+    A[..., 0] += 0.02
+    b = np.random.default_rng(33).uniform(-1, 1, (nz, ny, nx))
+    if shape == (120, 100, 90):
+        A[:, :, 48:, 0], A[:, :, 48:, 1:], A[:, :, 47, 1], b[:, :, 48:] = 1.0, 0.0, 0.0, 0.0
+    s = jetgpu.Solver(0)
+    try:
+        s.set_levels([shape])
+        s.upload(0, A, b)
+        s.cg_polls(0)
+        want = s.cg(600, 1e-8)
+        x = s.download_x()
+        s.cg_polls(1)
+        for _ in range(2):  # the one that fails, and the next, which does not try
+            info = s.cg(600, 1e-8)
+            assert info.converged and info.iterations == want.iterations
+            assert info.rel_residual == want.rel_residual
+            assert np.array_equal(s.download_x(), x)
+    finally:
+        s.close()
 
 
 def test_cg_one_launch_from_two_threads(solver):
