@@ -75,37 +75,77 @@ hipError_t scratch_address(int device, double** out) {
 
 // ------------------------------------------------------- level kernels
 
-// Planes per block of a z-marching launch of `tiles` columns (over all
-// systems) on nz planes, when `slots` blocks run at once and a block's
-// pipeline and halo cost `halo` plane steps: the chunk that makes the rounds
-// of blocks, each zc + halo steps, cheapest -- the mean of whole rounds (a
-// last round that is nearly empty costs like a full one while its blocks
-// wait on their own chains) and of the blocks' share (bandwidth).  Against
-// timing every chunk of {2, 4, 8, ... 64} on 43 level shapes from 24^3 to
-// 512^3, this picks within 0 to 3% of the fastest on average, and it is free
-// to take a chunk between them: 256 x 160 x 256 cells run 245 two-sweep
-// blocks of 38 planes instead of 210 of 48.
-int march_zc(int nz, long tiles, long slots, int halo) {
-    int best = nz;
-    double cost = 1e300;
-    for (int chunks = 1; chunks <= nz; ++chunks) {
-        const int zc = std::min(nz, (((nz + chunks - 1) / chunks) + 1) & ~1);  // even
-        if (zc > 64 && tiles > slots / 4) continue;  // longer only to cut the halo of few columns
-        const long blocks = tiles * ((nz + zc - 1) / zc);
-        const double share = (double)blocks / slots;
-        const double c = 0.5 * (std::ceil(share) + share) * (zc + halo);
-        if (c < cost) {
-            cost = c;
-            best = zc;
+// A z-marching launch of `tiles` columns (over all systems) on nz planes: the
+// planes per block zc that make it cheapest, and that cost, in plane steps of
+// a block that has its CU to itself.
+struct March {
+    int zc;
+    double cost;
+};
+// A block's pipeline and halo cost `halo` plane steps, and the CUs run `cus`
+// blocks at once, or (pair > 0) twice as many, when a step of two blocks on one
+// CU takes `pair` times the step of one.  A launch costs its rounds of blocks,
+// each zc + halo steps: whole rounds where the blocks wait on their own chains
+// (a last round that is nearly empty costs like a full one), the blocks' share
+// of the chip where they wait for memory; `whole` weighs the two.  Against
+// timing every chunk of {2, 4, 8, ... 64} on 76 level shapes from 2 x 2 x 32768
+// over 24^3 and 512 x 512 x 2 to 512^3, this picks within 1% of the fastest on
+// average, at worst 8%, and it is free to take a chunk between them:
+// 256 x 160 x 256 cells run 245 two-sweep blocks of 38 planes instead of 210
+// of 48.
+March march(int nz, long tiles, long cus, double halo, double pair, double whole) {
+    March best{nz, 1e300};
+    for (long chunks = 1; chunks <= nz;) {
+        const int zc = std::min<long>(nz, (((nz + chunks - 1) / chunks) + 1) & ~1l);  // even
+        if (zc <= 64 || tiles <= cus / 4) {  // longer only to cut the halo of few columns
+            const double share = (double)(tiles * ((nz + zc - 1) / zc)) / cus;
+            double rounds = std::ceil(share), work = share;
+            if (pair > 0.0) {
+                const double two = std::floor(share / 2), rest = share - 2 * two;
+                rounds = two * pair + (rest > 1 ? pair : (rest > 0 ? 1.0 : 0.0));
+                work = share * pair / 2;
+            }
+            const double c = (whole * rounds + (1.0 - whole) * work) * (zc + halo);
+            if (c < best.cost) best = March{zc, c};
         }
         if (zc <= 2) break;
+        chunks = (nz + zc - 3) / (zc - 2);  // the fewest of a smaller zc
     }
     return best;
 }
 
-int sweep_zc(const jg_solver* s, const Dims& d) {
-    const long tiles = (long)((d.nx + kSwIX - 1) / kSwIX) * ((d.ny + kSwIY - 1) / kSwIY);
-    return march_zc(d.nz, tiles * s->nsys, s->cus, 3);
+// How k_rb_sweep runs on shape d: tile rows per thread, planes per block, and
+// the cost in plane steps of one-row blocks.  FP32: one row, two blocks per CU.
+// FP64: one row and one block per CU, or (without a correction) two rows and
+// two blocks, whose step alone costs 1.2 times as much.  A sweep from zero is
+// as fast or faster with two on every shape measured; a plain one where two
+// rounds of blocks become one or many: 512 x 512 x 2 cells 18 -> 14 us,
+// 192 x 160 x 144 71 -> 59, 96^3 20 with one row and 23 with two.  Over 32
+// shapes this is 0.7% above the faster of the two on average (one row alone:
+// 10%).
+struct SweepShape {
+    int rows, zc;
+    double cost;
+};
+template <typename T>
+SweepShape sweep_shape(const jg_solver* s, const Dims& d, bool zero, bool correct) {
+    const long tiles = (long)((d.nx + kSwIX - 1) / kSwIX) * ((d.ny + kSwIY - 1) / kSwIY) * s->nsys;
+    if (sizeof(T) == 4) {
+        const March m = march(d.nz, tiles, s->cus, 2, 1.8, 0.85);
+        return {1, m.zc, m.cost};
+    }
+    const March one = march(d.nz, tiles, s->cus, 3, 0.0, 0.5);
+    if (!correct) {
+        const March two = march(d.nz, tiles, s->cus, zero ? 1 : 3, 1.5, 0.5);
+        if (zero || 1.2 * two.cost < one.cost) return {2, two.zc, 1.2 * two.cost};
+    }
+    return {1, one.zc, one.cost};
+}
+// k_rb_sweep2 on tiles of ix x iy cells: one block per CU; a chunk adds 8
+// planes of halo, some of them cheap.
+March sweep2_march(const jg_solver* s, const Dims& d, int ix, int iy) {
+    const long tiles = (long)((d.nx + ix - 1) / ix) * ((d.ny + iy - 1) / iy) * s->nsys;
+    return march(d.nz, tiles, s->cus, 6, 0.0, 0.5);
 }
 
 // Grids of a launch over every system of s (one, or a batch group): the
@@ -127,7 +167,8 @@ inline dim3 grid_1d(int nb, const jg_solver* s) { return dim3((unsigned)nb, (uns
 template <typename T>
 int launch_sweep(jg_solver* s, const Row<T>* A, const T* b, const T* xin, T* xout, const Dims& d,
                  int first, const T* coarse, double* p_bx, double* p_bb, T omega, const Ctl* ctl) {
-    int zc = sweep_zc(s, d);
+    const SweepShape shape = sweep_shape<T>(s, d, !xin && !coarse, coarse != nullptr);
+    int zc = shape.zc;
     const long cols = (long)((d.nx + kSwIX - 1) / kSwIX) * ((d.ny + kSwIY - 1) / kSwIY);
     // one b.x / b.b partial per block: keep the block count within a slot
     while (p_bx && zc < d.nz && cols * ((d.nz + zc - 1) / zc) > kMaxPartials) ++zc;
@@ -136,12 +177,19 @@ int launch_sweep(jg_solver* s, const Row<T>* A, const T* b, const T* xin, T* xou
     const int nb = (int)(grid.x * grid.y * grid.z);  // per system
     grid = grid_sys(grid, s);
     const int code = (first ? 8 : 0) | (xin ? 0 : 4) | (coarse ? 2 : 0) | (p_bx ? 1 : 0);
-    const dim3 block(kSwLX, kSwLY, 1);
+    const dim3 block(kSwLX, kSwLY / shape.rows, 1);
+    // the row counts that sweep_shape can ask for: R2 two, R1 one
 #define JG_SWEEP_CASE(C, F, Z, K, D)                                                              \
-    case C:                                                                                       \
-        k_rb_sweep<T, F, Z, K, D><<<grid, block, 0, s->stream>>>(A, b, xin, xout, d, zc, omega,   \
-                                                                 coarse, p_bx, p_bb, ctl);        \
-        break;
+    case C: {                                                                                     \
+        constexpr int R2 = sizeof(T) == 8 && !K ? 2 : 1, R1 = R2 == 2 && Z ? 2 : 1;               \
+        if (shape.rows == 2)                                                                      \
+            k_rb_sweep<T, F, Z, K, D, R2><<<grid, block, 0, s->stream>>>(                         \
+                A, b, xin, xout, d, zc, omega, coarse, p_bx, p_bb, ctl);                          \
+        else                                                                                      \
+            k_rb_sweep<T, F, Z, K, D, R1><<<grid, block, 0, s->stream>>>(                         \
+                A, b, xin, xout, d, zc, omega, coarse, p_bx, p_bb, ctl);                          \
+        break;                                                                                    \
+    }
     switch (code) {
         JG_SWEEP_CASE(0, 0, false, false, false)
         JG_SWEEP_CASE(1, 0, false, false, true)
@@ -182,9 +230,7 @@ int launch_sweep2(jg_solver* s, const Row<T>* A, const T* b, const T* xin, T* xo
                            : (z ? S2Tile<false, true>::IX : S2Tile<false>::IX);
         const int iy = res ? (z ? S2Tile<true, true>::IY : S2Tile<true>::IY)
                            : (z ? S2Tile<false, true>::IY : S2Tile<false>::IY);
-        // one block per CU; a chunk adds 8 planes of halo, some of them cheap
-        const long tiles = (long)((d.nx + ix - 1) / ix) * ((d.ny + iy - 1) / iy) * s->nsys;
-        const int zc = march_zc(d.nz, tiles, s->cus, 6);
+        const int zc = sweep2_march(s, d, ix, iy).zc;
         const dim3 grid = grid_sys(dim3((d.nx + ix - 1) / ix, (d.ny + iy - 1) / iy, (d.nz + zc - 1) / zc), s);
         const dim3 block(kS2LX, kS2TY, 1);
         const int code = (first ? 8 : 0) | (xin ? 0 : 4) | (coarse ? 2 : 0) | (res ? 1 : 0);
@@ -244,33 +290,41 @@ constexpr idx_t kBrickMaxCells = idx_t(1) << 21;
 
 // Sweeps of one smoothing step, grouped into launches: 1 = one sweep,
 // kLaunchMarch / kLaunchBrick = two sweeps in one launch of k_rb_sweep2 /
-// k_brick_sweep2.  A brick launch costs by its bricks (FP32 12.5 ns, FP64
-// 26 ns each once the chip is full), the marching ones a chain of planes
-// that no small grid shortens.  Measured pairs of plain sweeps, us, as two
-// launches / march / bricks:
-//   FP32  64^3 (512 bricks) 20 / 25 / 8.6   128x48x128 (1536) 26 / 26 / 22
-//         112x64x144 (2016) 26 / 26 / 28    128^3 (4096)      45 / 34 / 51
-//   FP64  64^3 (512) 24 / - / 12   80x48x80 (600) 24 / - / 22
-//         96x80x72 (1080) 25 / - / 30
-// and a march launch also writes the residual for the restriction.  So:
-// bricks up to 1536 (FP32) or 768 (FP64) over all systems; above, march in
-// FP32 (a single system or a group) and single sweeps in FP64.
+// k_brick_sweep2.  A brick launch costs by its bricks (FP32 16.5 ns, FP64
+// 34 ns each once the chip is full, less where a brick reaches out of the
+// grid), the marching ones a chain of plane steps (two-sweep FP32 1.55 us
+// each, single FP64 1.62 us) that a small grid does not shorten, and that a
+// narrow one pays for columns it does not have.  Measured, the mean of the
+// pre- and the post-smoothing pair, us, as two launches / march / bricks:
+//   FP32  64^3 (512 bricks) - / 22 / 10       96x80x72 (1080) - / 22 / 21
+//         128x48x128 (1536) - / 23 / 27       128^3 (4096) - / 35 / 63
+//         16x16x4096 (2048) - / 43 / 30       4x4x16384 (2048) - / 125 / 23
+//   FP64  64^3 (512) 30 / - / 18              80x48x80 (600) 30 / - / 30
+//         96x80x72 (1080) 31 / - / 42         128^3 (4096) 87 / - / 132
+//         16x16x4096 (2048) 122 / - / 67      8x8x8192 (1024) 105 / - / 28
+// So: bricks where these costs say so, else march in FP32 (a single system or
+// a group) and single sweeps in FP64.  With the bricks' number alone deciding
+// (768; FP32: 1536) a V-cycle of 4x4x16384 cells takes 1270 us in FP64 and 920
+// in FP32, so 370 and 185.
 // pairs > 0 forces two-sweep launches wherever two sweeps follow (FP32:
 // bricks up to 2^18 cells, else the z-marching kernel; FP64: bricks up to
 // kBrickMaxCells cells), pairs < 0 forbids them.
 constexpr int kLaunchSingle = 1, kLaunchMarch = 2, kLaunchBrick = 3;
 template <typename T>
 std::vector<int> sweep_plan(const jg_solver* s, const Dims& d, unsigned n, int pairs) {
-    const long bricks = (long)((d.nx + kBkB - 1) / kBkB) * ((d.ny + kBkB - 1) / kBkB) *
-                        ((d.nz + kBkB - 1) / kBkB) * s->nsys;
+    const long bricks_z = (long)((d.nz + kBkB - 1) / kBkB) * s->nsys;
+    const long bricks = (long)((d.nx + kBkB - 1) / kBkB) * ((d.ny + kBkB - 1) / kBkB) * bricks_z;
     int two;
     if (pairs > 0)  // FP32: bricks up to 64^3 cells, the z-marching kernel above
         two = sizeof(T) == 4 ? (d.n() <= (idx_t(1) << 18) ? kLaunchBrick : kLaunchMarch)
                              : (d.n() <= kBrickMaxCells ? kLaunchBrick : kLaunchSingle);
-    else if (sizeof(T) == 4)
-        two = bricks <= 1536 ? kLaunchBrick : kLaunchMarch;
-    else
-        two = bricks <= 768 ? kLaunchBrick : kLaunchSingle;
+    else if (sizeof(T) == 4) {
+        const double m = sweep2_march(s, d, S2Tile<false>::IX, S2Tile<false>::IY).cost;
+        two = bricks_z < 65536 && 3 + 0.0165 * bricks < 6.5 + 1.55 * (m + 2) ? kLaunchBrick : kLaunchMarch;
+    } else {
+        const double m = sweep_shape<T>(s, d, false, false).cost;
+        two = bricks_z < 65536 && 3 + 0.034 * bricks < 2 * (4.3 + 1.62 * m) ? kLaunchBrick : kLaunchSingle;
+    }
     if (pairs < 0 || s->twod || d.n() <= BotCfg<T>::MaxCells) two = kLaunchSingle;
     std::vector<int> v;
     for (unsigned k = 0; k < n;) {
@@ -684,13 +738,20 @@ int vcycle(jg_solver* s, const T* r0, T* z0, const MgCfg<T>& c, const Ctl* ctl, 
             break;
         }
         if (l + 1 == L) {
-            // coarsest level too large for one workgroup: symmetric fused sweeps
-            const int S = 2 * fwd;
+            // coarsest level too large for one workgroup: symmetric fused
+            // sweeps, fwd forward and fwd backward ones
+            const std::vector<int> plan = sweep_plan<T>(s, d, (unsigned)fwd, c.pairs);
+            const size_t half = plan.size(), M = 2 * half;
             const T* in = nullptr;
-            for (int k = 0; k < S; ++k) {
-                T* out = ((S - 1 - k) % 2 == 0) ? X(l) : Y;
-                launch_sweep<T>(s, A, B(l), in, out, d, k < fwd ? 0 : 1, nullptr, nullptr, nullptr,
-                                c.omega, ctl);
+            for (size_t m = 0; m < M; ++m) {
+                T* out = ((M - 1 - m) % 2 == 0) ? X(l) : Y;
+                const int first = m < half ? 0 : 1, mode = plan[m < half ? m : m - half];
+                if (mode == kLaunchBrick)
+                    launch_brick2<T>(s, A, B(l), in, out, d, first, nullptr, c.omega, ctl);
+                else if (mode == kLaunchMarch)
+                    JG_TRY(launch_sweep2<T>(s, A, B(l), in, out, d, first, nullptr, nullptr, c.omega, ctl));
+                else
+                    launch_sweep<T>(s, A, B(l), in, out, d, first, nullptr, nullptr, nullptr, c.omega, ctl);
                 in = out;
             }
             JG_TRY(check_launch(s, "coarsest"));

@@ -144,18 +144,22 @@ __device__ __forceinline__ void prolong_z(int t, const Dims& fd, int& k0, int& k
     }
 }
 
-// One tile position per thread, one plane of loads in flight ahead of the
-// plane being committed.  (Two positions per thread, or two planes, measured
-// as fast at 256^3, where the sweep is bound by HBM, and 3 to 9% slower on
-// average over 43 level shapes; the occupancy is what the VGPR budget allows
-// without spilling.)
-template <typename T, int FIRST, bool ZERO, bool CORRECT, bool DOT>
-__global__ __launch_bounds__(kSwLX* kSwLY, sizeof(T) == 4 || (ZERO && !CORRECT) ? 8 : 4) void k_rb_sweep(
+// RP tile positions per thread, one plane of loads in flight ahead of the
+// plane being committed.  FP64 sweeps without a correction take two positions
+// where the launch fills the chip (launch_sweep): blocks of 512 threads and at
+// most 128 VGPRs, so that two share a CU and one's loads and divisions overlap
+// the other's barriers.  On 192 x 160 x 144 cells a plain sweep takes 59 us
+// against 71 with one position (1024 threads, 78 VGPRs, one block per CU), one
+// from zero 47 against 51; at 256^3 255 against 265 and 203 against 221.  A
+// correction needs more registers than that (119 us against 85), and FP32 holds
+// two blocks of one position per CU.
+template <typename T, int FIRST, bool ZERO, bool CORRECT, bool DOT, int RP>
+__global__ __launch_bounds__(kSwLX* kSwLY / RP, sizeof(T) == 4 ? 8 : 4) void k_rb_sweep(
     const Row<T>* __restrict__ A, const T* __restrict__ b, const T* __restrict__ xin,
     T* __restrict__ xout, Dims d, int zc, T omega, const T* __restrict__ coarse,
     double* __restrict__ p_bx, double* __restrict__ p_bb, const Ctl* __restrict__ ctl) {
 #pragma clang fp contract(off)
-    constexpr int TY = kSwLY;
+    constexpr int TY = kSwLY / RP;
     constexpr int NTH = kSwLX * TY;
     // FP32: the c ring holds w = omega / c (0 for a zero-centre row) and the
     // update is (1 - omega) x + w (b - s), one division per cell and sweep;
@@ -222,9 +226,9 @@ __global__ __launch_bounds__(kSwLX* kSwLY, sizeof(T) == 4 || (ZERO && !CORRECT) 
         sz[e / kCzX][e % kCzX] = w0 * zc0 + w1 * zc1;
     };
 
-    // Each thread owns the position (tx, ty) of the tile: c and b of planes
-    // t, t-1, t-2, f of planes t .. t-3, the held r/u of plane t (written to
-    // LDS one step later) and the prefetched plane.
+    // Each thread owns the positions (tx, ty + TY r) of the tile, r < RP: c and
+    // b of planes t, t-1, t-2, f of planes t .. t-3, the held r/u of plane t
+    // (written to LDS one step later) and the prefetched plane.
     // Prefetched plane: raw loads (lanes outside the domain load cell 0),
     // masked only when committed, so nothing waits on them before then.
     struct Pre {
@@ -239,21 +243,24 @@ __global__ __launch_bounds__(kSwLX* kSwLY, sizeof(T) == 4 || (ZERO && !CORRECT) 
         Pre p;
         int ly, gy;
     };
-    Pos P;
-    P.ly = ty;
-    P.gy = gy0 + ty;
-    P.c0 = P.c1 = P.c2 = T(1);
-    P.f0 = P.f1 = P.f2 = P.f3 = T(0);
-    P.b0 = P.b1 = P.b2 = T(0);
-    P.hr = P.hu = T(0);
-    P.px = T(0);
-    P.pst = false;
+    Pos P[RP];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) sx[s][P.ly][tx] = T(0);
+    for (int r = 0; r < RP; ++r) {
+        P[r].ly = ty + TY * r;
+        P[r].gy = gy0 + ty + TY * r;
+        P[r].c0 = P[r].c1 = P[r].c2 = T(1);
+        P[r].f0 = P[r].f1 = P[r].f2 = P[r].f3 = T(0);
+        P[r].b0 = P[r].b1 = P[r].b2 = T(0);
+        P[r].hr = P[r].hu = T(0);
+        P[r].px = T(0);
+        P[r].pst = false;
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-        sr[s][P.ly][tx] = T(0);
-        su[s][P.ly][tx] = T(0);
+        for (int s = 0; s < 4; ++s) sx[s][P[r].ly][tx] = T(0);
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            sr[s][P[r].ly][tx] = T(0);
+            su[s][P[r].ly][tx] = T(0);
+        }
     }
     // Branch-free: lanes outside the domain load cell 0 (always valid); the
     // commit selects the neutral values for them (c = 1, everything else 0).
@@ -349,31 +356,42 @@ __global__ __launch_bounds__(kSwLX* kSwLY, sizeof(T) == 4 || (ZERO && !CORRECT) 
 
     // Prologue: plane k0-2 in flight, the coarse tile of k0-2.
     if (CORRECT) zfetch(k0 - 2);
-    fetch(P.p, P.gy, k0 - 2);
+#pragma unroll
+    for (int r = 0; r < RP; ++r) fetch(P[r].p, P[r].gy, k0 - 2);
     if (CORRECT) zstore(k0 - 2);
     __syncthreads();
 
     for (int t = k0 - 2; t <= k1 + 1; ++t) {
         // ---- commit plane t (prefetched), then prefetch plane t + 1
-        commit(P, P.p, t);
+#pragma unroll
+        for (int r = 0; r < RP; ++r) commit(P[r], P[r].p, t);
         if (CORRECT && t + 1 <= k1 + 1) zfetch(t + 1);
         // unconditional (past the end it re-reads plane k1+1, unused) so
         // the compiler can count the loads in flight
-        fetch(P.p, P.gy, min(t + 1, k1 + 1));
+#pragma unroll
+        for (int r = 0; r < RP; ++r) fetch(P[r].p, P[r].gy, min(t + 1, k1 + 1));
         // the final values of plane t - 3 (second colour of the last step)
-        flush(P, t - 3);
+#pragma unroll
+        for (int r = 0; r < RP; ++r) flush(P[r], t - 3);
         __syncthreads();
         // ---- first colour on plane t - 1
-        if (t - 1 >= 0 && t - 1 < d.nz) first_colour(P, t - 1);
+        if (t - 1 >= 0 && t - 1 < d.nz) {
+#pragma unroll
+            for (int r = 0; r < RP; ++r) first_colour(P[r], t - 1);
+        }
         __syncthreads();
         // ---- second colour on plane t - 2, final values written back
-        if (t - 2 >= k0 && t - 2 < k1) second_colour(P, t - 2);
+        if (t - 2 >= k0 && t - 2 < k1) {
+#pragma unroll
+            for (int r = 0; r < RP; ++r) second_colour(P[r], t - 2);
+        }
         // the coarse tile of plane t+1 (read by the next commit)
         if (CORRECT && t + 1 <= k1 + 1) zstore(t + 1);
         __syncthreads();
     }
     // the last second-colour plane, k1 - 1
-    flush(P, k1 - 1);
+#pragma unroll
+    for (int r = 0; r < RP; ++r) flush(P[r], k1 - 1);
     if (DOT) {
         // Block partials of b.x and b.b; the x ring is free after the last barrier.
         double* sh = reinterpret_cast<double*>(&sx[0][0][0]);

@@ -164,6 +164,30 @@ def test_mgpcg_two_sweep_kernels_bitwise(solver, oracle, precision):
     assert rel_err(out[-1][1], out[1][1]) <= 1e-12
 
 
+def test_mgpcg_two_row_sweeps(solver, oracle):
+    # more tiles than CUs on a flat grid: FP64 single sweeps hold two tile rows
+    # per thread, and the last one of level 0 writes the r.z / r.r partials
+    print("case mgpcg two-row sweeps", flush=True)
+    A, _ = poisson_helper(520, 500, 4)
+    A[..., 0] += 0.05
+    b = np.random.default_rng(35).uniform(-1, 1, A.shape[:3])
+    solver.set_levels([(520, 500, 4), (260, 250, 2)])
+    solver.upload(0, A, b)
+    solver.coarsen()
+    p = jetgpu.mg_params(max_levels=2, restrict_iter=2, correct_iter=2, coarsest_iter=20,
+                         final_iter=2)
+    out = {}
+    for pairs in (-1, 0, 1):
+        info = solver.mgpcg(200, p, jetgpu.gpu_options(stop_rule=jetgpu.JG_STOP_RELATIVE,
+                                                       rel_tol=1e-10, sweep_pairs=pairs))
+        out[pairs] = (info.iterations, solver.download_x())
+        assert info.rel_residual <= 1e-10
+    assert out[-1][0] == out[0][0] == out[1][0]
+    assert rel_err(out[-1][1], out[1][1]) <= 1e-12
+    xo, _, _, ok = oracle.cg_solve(A, b, 2000, 1e-9)
+    assert ok and rel_err(out[0][1], xo) <= 1e-6
+
+
 def test_mgpcg_closed_sphere_singular(solver, oracle):
     # All-Neumann (config-1 geometry): compare modulo the mean.
     markers, s = scene_system(oracle, 1, 32, 3, seed=2)

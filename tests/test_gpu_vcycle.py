@@ -120,7 +120,9 @@ def test_vcycle_symmetric_positive_linear(solver, shape, levels, precision, tol)
 
 @pytest.mark.parametrize("shape,levels", [((64, 64, 64), 5), ((48, 32, 16), 3), ((32, 64, 16), 3),
                                           ((40, 24, 20), 2), ((120, 56, 36), 2), ((96, 64, 48), 3),
-                                          ((34, 18, 10), 2), ((130, 70, 44), 2), ((108, 44, 60), 3)])
+                                          ((34, 18, 10), 2), ((130, 70, 44), 2), ((108, 44, 60), 3),
+                                          ((100, 70, 44), 1), ((131, 71, 1), 1), ((700, 391, 1), 1),
+                                          ((10, 6, 4000), 2), ((520, 500, 4), 2)])
 @pytest.mark.parametrize("sched", [(2, 2, 20, 2), (3, 3, 6, 3), (2, 4, 6, 4), (1, 2, 4, 0)])
 def test_vcycle_two_sweep_kernel_bitwise(solver, oracle, shape, levels, sched):
     # Two sweeps per launch wherever two sweeps follow each other must give
@@ -129,6 +131,11 @@ def test_vcycle_two_sweep_kernel_bitwise(solver, oracle, shape, levels, sched):
     # brick kernel.  Where the pre-smoothing ends with a z-marching pair, that
     # launch also writes the residual for the restriction (54 x 22 interiors),
     # which must equal the separate residual-restriction's bit for bit.
+    # The sweeps of a coarsest level too large for the one-workgroup bottom are
+    # paired the same way (single levels among them), and the launches that the
+    # sizes ask for by themselves (sweep_pairs 0) give the same values.  FP64
+    # single sweeps hold one or two tile rows per thread: two from zero, and on
+    # the last shape (more tiles than CUs) in the plain ones too.
     # Shapes cover partial tiles in x (56- and 54-wide interiors), y (24 and
     # 22 rows) and bricks (sizes not multiples of 8), z extents that are not
     # multiples of the chunk, and pairs that start with a zero-start, a
@@ -143,6 +150,7 @@ def test_vcycle_two_sweep_kernel_bitwise(solver, oracle, shape, levels, sched):
         single = apply(solver, gp, prec, r, sweep_pairs=-1)
         paired = apply(solver, gp, prec, r, sweep_pairs=1)
         assert np.array_equal(single, paired), prec
+        assert np.array_equal(single, apply(solver, gp, prec, r)), prec
         assert rel_err(paired, want) <= tol
 
 
