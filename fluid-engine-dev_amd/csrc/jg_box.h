@@ -43,18 +43,27 @@ __global__ void k_box_reset(BoxScan* box) {
     }
 }
 
-// One wave's row of 64 cells at (x0.., j, k), lane = x: widens the running
-// bounds.  in: the lane's cell is inside the grid.
-__device__ __forceinline__ void box_row(const Row<double>* __restrict__ A, const double* __restrict__ b,
-                                        const Dims& d, double most, int x0, int j, int k, bool in,
-                                        int lo[3], int hi[3]) {
-    Row<double> row{1.0, 0.0, 0.0, 0.0};
-    double bv = 0.0;
+// One wave's row of 64 cells at (x0.., j, k), lane = x.  in: the lane's cell is
+// inside the grid (one outside takes no part).
+struct BoxCell {
+    Row<double> row;
+    double b;
+};
+__device__ __forceinline__ BoxCell box_load(const Row<double>* __restrict__ A, const double* __restrict__ b,
+                                            const Dims& d, int x0, int j, int k, bool in) {
+    BoxCell v{{1.0, 0.0, 0.0, 0.0}, 0.0};
     if (in) {
         const idx_t c = x0 + (int)(threadIdx.x & 63) + (idx_t)d.nx * (j + (idx_t)d.ny * k);
-        row = A[c];
-        bv = b[c];
+        v.row = A[c];
+        v.b = b[c];
     }
+    return v;
+}
+// Widens the running bounds by that row.
+__device__ __forceinline__ void box_vote(const BoxCell& v, double most, int x0, int j, int k, int lo[3],
+                                         int hi[3]) {
+    const Row<double>& row = v.row;
+    const double bv = v.b;
     const bool cr = row.r != 0.0, cu = row.u != 0.0, cf = row.f != 0.0;
     const unsigned long long on = __ballot(cr || cu || cf || bv != 0.0 || !(fabs(row.c) <= most));
     if (!on) return;
@@ -81,15 +90,18 @@ __device__ __forceinline__ void box_widen(BoxScan* box, const int lo[3], const i
 
 // Cells of a block: 64 in x, kBoxY rows, kBoxZ planes.
 constexpr int kBoxY = 4, kBoxZ = 16;
-constexpr int kBoxSamples = 512;  // (an odd step apart: at every height)
+constexpr int kBoxSamples = 2048;  // rows of 64 cells that the sample reads
 
-// The scan, in two launches.  SAMPLE: kBoxSamples rows spread over the system,
-// for a first guess, a few per wave: with a row per wave the waves' first
-// atomics on the bounds took 75 us at 256^3 and 185 us on a 2048 x 1536 plane.
-// Otherwise a block looks at its cells only where they
-// reach beyond the box found so far: a dense system is hardly read, and of a
-// free-surface one what is read is the part that every pass of the solve
-// then leaves out.
+// The scan, in two launches.  SAMPLE: whole grid rows spread over the system,
+// an odd step apart (at every height), and the last one, for a first guess; a
+// few waves read some 16 rows of 64 cells each, four at a time.  (With a row per
+// wave the waves' first atomics on the bounds took 75 us at 256^3 and 185 us on
+// a 2048 x 1536 plane; 512 grid rows whatever their length, one after the
+// other, 26 us at 256^3, 82 on a 1000 x 1000 plane and 117 on 3000 x 2000; so
+// 28, 27 and 28.)
+// Otherwise a block looks at its cells only where they reach beyond the box
+// found so far: a dense system is hardly read, and of a free-surface one what
+// is read is the part that every pass of the solve then leaves out.
 template <bool SAMPLE>
 __global__ __launch_bounds__(64 * kBoxY) void k_box_scan(const Row<double>* __restrict__ A,
                                                          const double* __restrict__ b, Dims d, double most,
@@ -99,9 +111,18 @@ __global__ __launch_bounds__(64 * kBoxY) void k_box_scan(const Row<double>* __re
     const int w = threadIdx.x >> 6;
     int lo[3] = {0x7fffffff, 0x7fffffff, 0x7fffffff}, hi[3] = {-1, -1, -1};
     if (SAMPLE) {
-        const idx_t rows = (idx_t)d.ny * d.nz, step = rows / kBoxSamples | 1;
-        for (idx_t r = (blockIdx.y * kBoxY + w) * step; r < rows; r += (idx_t)gridDim.y * kBoxY * step)
-            box_row(A, b, d, most, x0, (int)(r % d.ny), (int)(r / d.ny), in, lo, hi);
+        const idx_t rows = (idx_t)d.ny * d.nz, step = rows * gridDim.x / kBoxSamples | 1;
+        const idx_t next = (idx_t)gridDim.y * kBoxY * step;
+        auto load = [&](idx_t r) { return box_load(A, b, d, x0, (int)(r % d.ny), (int)(r / d.ny), in && r < rows); };
+        auto vote = [&](const BoxCell& v, idx_t r) { box_vote(v, most, x0, (int)(r % d.ny), (int)(r / d.ny), lo, hi); };
+        for (idx_t r = (blockIdx.y * kBoxY + w) * step; r < rows; r += 4 * next) {
+            BoxCell v[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[q] = load(r + q * next);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) vote(v[q], r + q * next);
+        }
+        if (blockIdx.y == 0 && w == 0) vote(load(rows - 1), rows - 1);
     } else {
         const int y0 = blockIdx.y * kBoxY, k0 = blockIdx.z * kBoxZ;
         const int x1 = min(x0 + 63, d.nx - 1), y1 = min(y0 + kBoxY, d.ny) - 1, k1 = min(k0 + kBoxZ, d.nz) - 1;
@@ -118,8 +139,13 @@ __global__ __launch_bounds__(64 * kBoxY) void k_box_scan(const Row<double>* __re
         if (inside) return;
         const int j = y0 + w;
         if (j < d.ny) {
-#pragma unroll 4
-            for (int k = k0; k <= k1; ++k) box_row(A, b, d, most, x0, j, k, in, lo, hi);
+            for (int k = k0; k <= k1; k += 4) {
+                BoxCell v[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) v[q] = box_load(A, b, d, x0, j, k + q, in && k + q <= k1);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) box_vote(v[q], most, x0, j, k + q, lo, hi);
+            }
         }
     }
     box_widen(box, lo, hi);
