@@ -12,6 +12,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 namespace jg {
 
 template <typename T>
@@ -69,6 +71,28 @@ constexpr int NT = 256;  // threads per block of the streaming kernels
 // Per reduction slot.  A plane is reduced in tiles of 64 x 4 cells, one partial
 // each, so this bounds a plane (a 2-D grid) at about 2^24 cells.
 constexpr int kMaxPartials = 65536;
+
+// Geometry of the tiled z-march (tm_march): one wave per x row of a
+// 64 x kTmY tile of each plane, kTmZ planes per block (on the 256^3 sphere
+// pool 8 x 16 is within noise of the best of 4, 8, 16 rows and 8, 16, 32
+// planes for the SpMV).
+constexpr int kTmX = 64, kTmY = 8, kTmZ = 16;
+
+// Grid of a tm_march kernel on one system of shape d: 64 x 8 columns,
+// z-chunks of at most kTmZ planes, shortened on small grids so a system has
+// about 2048 blocks, and lengthened to at most kMaxPartials blocks where chunks
+// can do that.  A plane of more than kMaxPartials tiles (33.5 M cells) stays
+// above it: jg_solver_set_levels rejects one, so the launches that write
+// partials never meet it, and the operator entries (jg_relax_jacobi,
+// jg_blas_residual) write none.  The chunking depends on the shape alone, so a
+// member of a batch group is cut (and its reductions summed) as a solve of the
+// same cells alone.
+inline void tm_grid(const Dims& d, dim3& grid, int& zc) {
+    const long cols = (long)((d.nx + kTmX - 1) / kTmX) * ((d.ny + kTmY - 1) / kTmY);
+    zc = (int)std::max<long>(1, std::min<long>(std::min(d.nz, kTmZ), cols * d.nz / 2048));
+    while (zc < d.nz && cols * ((d.nz + zc - 1) / zc) > kMaxPartials) ++zc;
+    grid = dim3((d.nx + kTmX - 1) / kTmX, (d.ny + kTmY - 1) / kTmY, (unsigned)((d.nz + zc - 1) / zc));
+}
 
 // Several systems of one hierarchy solved by the same launches (a batch
 // group) keep their arrays back to back: per system every level's rows and

@@ -201,12 +201,6 @@ __global__ __launch_bounds__(NT) void k_dir_spmv(const Row<TA>* __restrict__ A,
     block_partial<NT>(acc, partial, part);
 }
 
-// Geometry of the tiled z-march (tm_march): one wave per x row of a
-// 64 x kTmY tile of each plane, kTmZ planes per block (on the 256^3 sphere
-// pool 8 x 16 is within noise of the best of 4, 8, 16 rows and 8, 16, 32
-// planes for the SpMV).
-constexpr int kTmX = 64, kTmY = 8, kTmZ = 16;
-
 // What a cell of the tiled z-march sees in plane k: its row, its value v
 // (the stencil source of the kernel), the values of its six neighbours
 // (zero outside the grid), the -x / -y / -z couplings and cen, the value
@@ -355,18 +349,6 @@ __device__ __forceinline__ void tm_march(const Row<T>* __restrict__ A,
         rn1 = rn2;
         cur = nxt;
     }
-}
-
-// Grid of a tm_march kernel on one system of shape d: 64 x 8 columns,
-// z-chunks of at most kTmZ planes, shortened on small grids so a system has
-// about 2048 blocks, and at most kMaxPartials blocks.  The chunking depends
-// on the shape alone, so a member of a batch group is cut (and its
-// reductions summed) exactly as the same system solved alone.
-inline void tm_grid(const Dims& d, dim3& grid, int& zc) {
-    const long cols = (long)((d.nx + kTmX - 1) / kTmX) * ((d.ny + kTmY - 1) / kTmY);
-    zc = (int)std::max<long>(1, std::min<long>(std::min(d.nz, kTmZ), cols * d.nz / 2048));
-    while (cols * ((d.nz + zc - 1) / zc) > kMaxPartials) ++zc;
-    grid = dim3((d.nx + kTmX - 1) / kTmX, (d.ny + kTmY - 1) / kTmY, (unsigned)((d.nz + zc - 1) / zc));
 }
 
 // k_dir_spmv through the tiled z-march: the same values, operand order and

@@ -98,6 +98,41 @@ def test_relax_jacobi(solver, oracle):
     assert np.array_equal(host(out), oracle.jacobi_relax(A, b, x))
 
 
+def test_plane_of_more_tiles_than_partials(solver):
+    # 66040 tiles of 64 x 8 cells a plane, above the bound on the reduction
+    # partials, which residual and Jacobi do not write: the tiled z-march in
+    # Jet's operand order, against the same expressions in torch
+    import torch
+
+    nx, ny, nz = shape = (65000, 520, 2)
+    print(f"case large plane shape={shape}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(19)
+    A = torch.rand((nz, ny, nx, 4), generator=g, device="cuda", dtype=torch.float64) - 0.5
+    A[..., 0] += 3.0
+    x = torch.rand((nz, ny, nx), generator=g, device="cuda", dtype=torch.float64)
+    b = torch.rand((nz, ny, nx), generator=g, device="cuda", dtype=torch.float64)
+
+    def terms():
+        for dim, e in ((2, 1), (1, 2), (0, 3)):  # coupling down, then up, along x, y, z
+            n, c = x.shape[dim], A[..., e]
+            down, up = torch.zeros_like(x), torch.zeros_like(x)
+            down.narrow(dim, 1, n - 1).copy_(c.narrow(dim, 0, n - 1) * x.narrow(dim, 0, n - 1))
+            up.narrow(dim, 0, n - 1).copy_(c.narrow(dim, 0, n - 1) * x.narrow(dim, 1, n - 1))
+            yield down
+            yield up
+
+    res, s = b - A[..., 0] * x, torch.zeros_like(x)
+    for t in terms():
+        res -= t
+        s += t
+    out = torch.empty_like(x)
+    torch.cuda.synchronize()
+    solver.residual(shape, A, x, b, out)
+    assert torch.equal(out, res)
+    solver.relax_jacobi(shape, A, b, x, out)
+    assert torch.equal(out, (b - s) / A[..., 0])
+
+
 @pytest.mark.parametrize("fshape", [(2, 2, 2), (8, 6, 4), (64, 64, 64), (34, 10, 22), (6, 4, 8)])
 def test_restrict_correct(solver, oracle, fshape):
     rng = np.random.default_rng(17)
