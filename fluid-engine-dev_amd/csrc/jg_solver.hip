@@ -1002,15 +1002,23 @@ int cg_grid_rows(jg_solver* s, const Pcg<double>& v) {
     return n > per ? 2 : 1;
 }
 
+// dalloc of something that a solve can do without: no room is no error.
+template <typename T>
+bool dalloc_spare(jg_solver* s, T** p, size_t count) {
+    const std::string before = s->err;
+    if (dalloc(s, p, count) == JG_OK) return true;
+    (void)hipGetLastError();
+    s->err = before;
+    return false;
+}
+
 // pcg_device through k_cg_grid; the state after pcg_init in, x and the
 // control block out.  *ran is false where that launch is not to be had (no
 // room for its slots, refused, or a block did not arrive in time): the caller
 // starts again without it, and so does every later solve of s.
 int cg_grid(jg_solver* s, const Pcg<double>& v, int C, bool* ran) {
     *ran = false;
-    if (!s->cg_slots && dalloc(s, &s->cg_slots, 3 * kCgSumWords) != JG_OK) {
-        (void)hipGetLastError();
-        s->err.clear();
+    if (!s->cg_slots && !dalloc_spare(s, &s->cg_slots, 3 * kCgSumWords)) {
         s->cooperative = false;
         return JG_OK;
     }
@@ -1621,7 +1629,6 @@ constexpr double kBoxShare = 0.85;
 int find_box(jg_solver* s, size_t L, double most, Box* box, double* share) {
     const Level& l0 = s->lv[0];
     const Dims& d = l0.d;
-    if (!s->box_scan) JG_TRY(dalloc(s, &s->box_scan, 2));
     k_box_reset<<<1, 64, 0, s->stream>>>(s->box_scan);
     const unsigned gx = (d.nx + 63) / 64;
     // at most 128 waves in all
@@ -1647,18 +1654,21 @@ int find_box(jg_solver* s, size_t L, double most, Box* box, double* share) {
 }
 
 // The arrays of box solves: rows of every level, b and x, for boxes of up to
-// kBoxShare of the grid; kept until the hierarchy changes.  false: no room.
+// kBoxShare of the grid; one allocation, so that there is all or nothing, kept
+// until the hierarchy changes.  false: no room.
 bool box_reserve(jg_solver* s, size_t L) {
     if (s->box_cells > 0 || s->box_failed) return !s->box_failed;
-    size_t cells = 0, first = 0;
-    for (size_t l = 0; l < L; ++l) cells += (size_t)(kBoxShare * (double)s->lv[l].d.n()) + 1;
-    first = (size_t)(kBoxShare * (double)s->lv[0].d.n()) + 1;
-    if (dalloc(s, &s->box_rows, cells) != JG_OK || dalloc(s, &s->box_b, first) != JG_OK ||
-        dalloc(s, &s->box_x, first) != JG_OK) {
-        (void)hipGetLastError();
+    auto room = [&](size_t l) { return ((size_t)(kBoxShare * (double)s->lv[l].d.n()) / 32 + 1) * 32; };
+    size_t cells = 0;
+    for (size_t l = 0; l < L; ++l) cells += room(l);
+    double* all = nullptr;
+    if (!dalloc_spare(s, &all, 4 * cells + 2 * room(0))) {
         s->box_failed = true;
         return false;
     }
+    s->box_rows = (Row<double>*)all;
+    s->box_b = all + 4 * cells;
+    s->box_x = s->box_b + room(0);
     s->box_cells = cells;
     return true;
 }
@@ -1673,6 +1683,7 @@ int solve_in_box(jg_solver* s, size_t L, idx_t from, double most, bool mixed, Ru
     auto whole = [&]() { return run(s, [] { return (int)JG_OK; }); };
     Level& l0 = s->lv[0];
     if (l0.d.n() < from || s->nsys > 1) return whole();
+    if (!s->box_scan && !dalloc_spare(s, &s->box_scan, 2)) return whole();
     Box box;
     double share = 1.0;
     JG_TRY(find_box(s, L, most, &box, &share));
