@@ -1,5 +1,5 @@
 // jg_cggrid.h -- Jet's plain CG (include/jet/detail/cg-inl.h:15-94) on a
-// system that fits the chip: one cooperative launch runs the iterations, and
+// system that fits the chip: one launch runs the iterations, and
 // matrix and vectors stay in registers.
 //
 // A CG iteration of a small grid is bound by its kernel boundaries: at 64^3
@@ -19,10 +19,18 @@
 // gets the same bits, and a run is deterministic.  What crosses blocks (r,
 // on refresh iterations x, the slots) is written and read by agent-scope
 // atomics, which go through the XCDs' private L2s; a block waits for its
-// stores before its slot is written.  The blocks of a cooperative launch are
-// resident together, so the waits end; a wait that does not within
-// CgGridArgs::polls makes every block leave, and the solve starts again as the
-// loop of one launch per step (so does one whose launch is refused).
+// stores before its slot is written.  The waits end because all blocks become
+// resident: there are at most as many as CUs, a block fits a free CU, other
+// work on the device ends without waiting for this kernel, and one process
+// runs one such launch on a device at a time (cg_grid).  Where that fails (a
+// device shared with another program that waits the same way, fewer CUs than
+// reported), a wait that does not end within CgGridArgs::polls makes every
+// block leave, and the solve starts again as the loop of one launch per step
+// (so does one whose launch is refused).
+// (hipLaunchCooperativeKernel, which guarantees residency, makes the runtime
+// add a queue of its own kind, and from then on graphs with many branches run
+// at half their rate for the rest of the process: a batch of 16 hierarchies 6
+// -> 16 ms.)
 //
 // At 64^3 an iteration takes 7.9 us: 2.7 and 3.2 (with the wait for the
 // published r) in the two sums, the rest the loads of the neighbours' r

@@ -117,8 +117,8 @@ inline int nblocks(const Geo& g) { return (int)(g.grid.x * g.grid.y * g.grid.z);
 struct jg_solver {
     int device = 0;
     int cus = 0;               // compute units of the device
-    bool cooperative = false;  // it takes cooperative launches (and none of this solver's failed)
-    int cg_polls = 1 << 23;    // bound of a wait in k_cg_grid (some seconds), 0: no such launch
+    bool cg_grid_ok = true;    // no k_cg_grid launch of this solver has failed
+    int cg_polls = 1 << 20;    // bound of a wait in k_cg_grid (about a second), 0: no such launch
     // Systems held back to back (a batch group of one hierarchy): every
     // array below holds nsys of them (jg_device.h, kSys*), and the V-cycle
     // and PCG launches cover all of them.  A view is one member of a group:

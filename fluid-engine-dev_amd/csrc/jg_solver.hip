@@ -990,14 +990,13 @@ int pcg_iteration(jg_solver* s, const Pcg<T>& v, bool odd, Ctl* host) {
 }
 
 // Rows per thread when the CG of v (FP64, no preconditioner) runs as one
-// cooperative launch (k_cg_grid), 0 when it does not: every row of the
-// system has to fit the registers of one block per CU, with at most kCgW
-// entries.  One row per thread as far as that goes: at 64^3 256 blocks of
+// launch (k_cg_grid), 0 when it does not: every row of the system has to fit
+// the registers of one block per CU, with at most kCgW entries.  One row per thread as far as that goes: at 64^3 256 blocks of
 // one take 8.2 us an iteration, 128 blocks of two 10.4, though their sums
 // cost less.
 int cg_grid_rows(jg_solver* s, const Pcg<double>& v) {
     const idx_t n = v.d.n(), per = (idx_t)std::min(s->cus, kCgMaxBlocks) * kCgThreads;
-    if (v.mg || s->nsys > 1 || !s->cooperative || s->cg_polls <= 0 || n > 2 * per) return 0;
+    if (v.mg || s->nsys > 1 || !s->cg_grid_ok || s->cg_polls <= 0 || n > 2 * per) return 0;
     if (v.csr && (!v.ell || s->csr.ell_w > kCgW)) return 0;
     return n > per ? 2 : 1;
 }
@@ -1019,25 +1018,27 @@ bool dalloc_spare(jg_solver* s, T** p, size_t count) {
 int cg_grid(jg_solver* s, const Pcg<double>& v, int C, bool* ran) {
     *ran = false;
     if (!s->cg_slots && !dalloc_spare(s, &s->cg_slots, 3 * kCgSumWords)) {
-        s->cooperative = false;
+        s->cg_grid_ok = false;
         return JG_OK;
     }
     const idx_t n = v.d.n();
     CgGridArgs a{v.A, v.ell ? *v.ell : EllDev{}, v.d, v.b, v.x, v.r, v.dA, v.ctl, s->cg_slots, s->cg_polls};
     const dim3 grid((unsigned)((n + (idx_t)C * kCgThreads - 1) / ((idx_t)C * kCgThreads)));
-    const void* f = v.ell ? (C == 1 ? (const void*)k_cg_grid<1, true> : (const void*)k_cg_grid<2, true>)
-                          : (C == 1 ? (const void*)k_cg_grid<1, false> : (const void*)k_cg_grid<2, false>);
-    void* args[] = {&a};
+    auto* const f = v.ell ? (C == 1 ? k_cg_grid<1, true> : k_cg_grid<2, true>)
+                          : (C == 1 ? k_cg_grid<1, false> : k_cg_grid<2, false>);
+    // two of these launches at once could each hold the CUs the other waits for
+    static std::mutex busy[16];
+    std::lock_guard<std::mutex> lock(busy[s->device % 16]);
     do {
         k_fill<unsigned long long><<<nblocks_1d(3 * kCgSumWords), NT, 0, s->stream>>>(s->cg_slots, 0ull,
                                                                                   3 * kCgSumWords);
-        const bool refused =
-            hipLaunchCooperativeKernel(f, grid, dim3(kCgThreads), args, 0, s->stream) != hipSuccess;
-        if (refused) (void)hipGetLastError();
+        JG_TRY(check_launch(s, "cg grid"));
+        f<<<grid, kCgThreads, 0, s->stream>>>(a);
+        const bool refused = hipGetLastError() != hipSuccess;
         JG_HIP(hipMemcpyAsync(s->ctl_host, v.ctl, sizeof(Ctl), hipMemcpyDeviceToHost, s->stream));
         JG_TRY(sync(s));
         if (refused || s->ctl_host->pad) {
-            s->cooperative = false;
+            s->cg_grid_ok = false;
             return JG_OK;
         }
     } while (!s->ctl_host->done);
@@ -1693,7 +1694,7 @@ int solve_in_box(jg_solver* s, size_t L, idx_t from, double most, bool mixed, Ru
     jg_solver v;
     v.device = s->device;
     v.cus = s->cus;
-    v.cooperative = s->cooperative;
+    v.cg_grid_ok = s->cg_grid_ok;
     v.cg_polls = s->cg_polls;
     v.view = true;
     v.stream = s->stream;
@@ -1755,7 +1756,7 @@ int solve_in_box(jg_solver* s, size_t L, idx_t from, double most, bool mixed, Ru
     // the solver's own parts stay with s
     bad = s->box_host->lo[0];
     s->cg_slots = v.cg_slots;
-    s->cooperative = v.cooperative;
+    s->cg_grid_ok = v.cg_grid_ok;
     s->allocs.insert(s->allocs.end(), v.allocs.begin(), v.allocs.end());
     v.allocs.clear();
     if (!v.err.empty()) s->err = v.err;
@@ -1811,13 +1812,10 @@ int jg_solver_create(int device, jg_solver** out) {
         delete s;
         return JG_ERR_HIP;
     }
-    int coop = 0;
-    if (hipDeviceGetAttribute(&s->cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
-        hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, device) != hipSuccess) {
+    if (hipDeviceGetAttribute(&s->cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) {
         delete s;
         return JG_ERR_HIP;
     }
-    s->cooperative = coop != 0;
     // this device's address of the no-allocation scratch array (a failure is
     // reported by jg_relax_red_black_noalloc, the only user)
     (void)scratch_init(device);

@@ -136,10 +136,9 @@ int jg_solver_matrices_changed(jg_solver* s);
 int jg_solver_cg(jg_solver* s, unsigned max_iter, double tol,
                  jg_solve_info* info);
 /* Plain CG of a system that fits the chip (jg_solver_cg, jg_csr_cg_*; at most
- * 524288 rows on 256 compute units) runs as one cooperative launch whose
- * blocks wait for each other.  polls bounds each wait (default 2^23, some
- * seconds); 0 turns that launch off, for instance on a GPU shared with other
- * programs.  A wait that runs out, or a launch that the device refuses, is no
+ * 524288 rows on 256 compute units) runs as one launch whose blocks wait for
+ * each other.  polls bounds each wait (default 2^20, about a second); 0 turns
+ * that launch off, for instance on a GPU shared with other programs.  A wait that runs out, or a launch that the device refuses, is no
  * error: the solve starts again with one launch per step of an iteration, and
  * so do the solver's later ones. */
 int jg_solver_cg_polls(jg_solver* s, unsigned polls);

@@ -126,3 +126,47 @@ def test_batch_64_uneven_systems(gpu):
             err = rel_err(res[precision][i], sys_.x[0])
             print(f"  member {i} n={n} precision={precision} err_vs_oracle={err:.2e}", flush=True)
             assert err <= 1e-6, (i, n, precision)
+
+
+CG_THEN_BATCH = r"""
+import sys
+sys.path[:0] = [sys.argv[1] + "/tests", sys.argv[1] + "/fluid-engine-dev_amd"]
+import numpy as np
+import jetgpu
+from test_gpu_batch import PARAMS
+from systems import random_stencil
+
+if sys.argv[2] == "cg":
+    c = jetgpu.Solver(0)
+    A = random_stencil(32, 32, 32, np.random.default_rng(1))
+    c.set_levels([(32, 32, 32)])
+    c.upload(0, A, np.ones(A.shape[:3]))
+    c.cg(100, 1e-6)
+sizes = [(16 + 8 * (i % 4), 16 + 8 * (i // 4), 32) for i in range(16)]
+b = jetgpu.Batch(sizes, [3] * 16)
+for s, (nx, ny, nz) in zip(b.systems, sizes):
+    A = random_stencil(nx, ny, nz, np.random.default_rng(nx + ny))
+    s.upload(0, A, np.random.default_rng(ny).uniform(-1, 1, (nz, ny, nx)))
+    s.coarsen()
+p, o = jetgpu.mg_params(max_levels=3, **PARAMS), jetgpu.gpu_options(rel_tol=1e-8, stop_rule=1)
+print("ms", min(b.mgpcg(100, p, o)[1] for _ in range(20)), flush=True)
+"""
+
+
+def test_batch_rate_after_a_cg(gpu):
+    # the one-launch CG leaves nothing behind in the process that slows down
+    # a batch's graph (16 branches; a cooperative launch before the batch is
+    # made did, to half its rate)
+    import subprocess
+    import sys
+
+    from jgtest import ROOT
+
+    ms = []
+    for first in ("batch", "cg"):
+        p = subprocess.run([sys.executable, "-u", "-c", CG_THEN_BATCH, ROOT, first],
+                           capture_output=True, text=True, timeout=50)
+        assert p.returncode == 0, p.stdout + p.stderr
+        ms.append(float(p.stdout.split()[-1]))
+    print("batch alone and after a CG, ms:", ms, flush=True)
+    assert ms[1] <= 1.5 * ms[0]

@@ -179,7 +179,7 @@ def test_compressed_free_surface_kat_on_device(solver, oracle):
     assert np.all(p[:, 2, :] == 0.0)
 
 
-@pytest.mark.parametrize("polls", [1 << 23, 0, 1])
+@pytest.mark.parametrize("polls", [1 << 20, 0, 1])
 @pytest.mark.parametrize("n,fluid", [((11, 10, 10), 0.93), ((72, 64, 64), 0.95), ((80, 72, 72), 0.9),
                                      ((96, 96, 72), 0.95)])
 def test_csr_cg_one_launch_matches_oracle(oracle, n, fluid, polls):

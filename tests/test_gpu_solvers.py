@@ -46,10 +46,10 @@ def test_cg_2x2_known_answer(solver):
     assert info.iterations <= 2 and info.last_residual <= 1e-15
 
 
-# polls 0: one launch per step instead of the one cooperative launch these sizes
+# polls 0: one launch per step instead of the one launch these sizes
 # take (the last two then take the tiled z-march: partial 64 x 8 x 16 tiles in x,
 # y and z)
-@pytest.mark.parametrize("polls", [1 << 23, 0])
+@pytest.mark.parametrize("polls", [1 << 20, 0])
 @pytest.mark.parametrize("shape,tol", [((3, 3, 3), 1e-9), ((16, 12, 10), 1e-10), ((40, 40, 40), 1e-9),
                                        ((100, 20, 37), 1e-10), ((64, 13, 50), 1e-10)])
 def test_cg_matches_oracle(solver, oracle, shape, tol, polls):
@@ -65,7 +65,7 @@ def test_cg_matches_oracle(solver, oracle, shape, tol, polls):
     try:
         info = solver.cg(1000, tol)
     finally:
-        solver.cg_polls(1 << 23)
+        solver.cg_polls(1 << 20)
     x = solver.download_x()
     assert abs(int(info.iterations) - io) <= 2 and bool(info.converged) == oko
     assert info.last_residual <= tol
@@ -336,7 +336,7 @@ def test_cg_wait_that_runs_out_is_no_error(shape):
 
 
 def test_cg_one_launch_from_two_threads(solver):
-    # cooperative launches of two solvers in flight at once: each equals its
+    # one-launch solves of two solvers at once: each equals its
     # solve alone, bit for bit
     import threading
 
