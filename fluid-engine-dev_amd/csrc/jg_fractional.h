@@ -99,13 +99,19 @@ __device__ __forceinline__ float fr_weight(double p0, double p1, double p2, doub
 // thread marches the column of vertices (i, j) through a chunk of planes and
 // keeps the vertices (i .. i+1, j .. j+1) of two of them, so the SDF is read
 // from memory once for the three axes, not once for each.  At 512^3 (1.1 GB
-// in, 1.6 GB out) 850 us against 2020 for a launch per axis.
+// in, 1.6 GB out) 850 us against 2020 for a launch per axis.  Chunks of kFwZ
+// planes, shorter ones (fr_weights_zc) where those leave the chip idle: a
+// chunk is a chain of dependent steps.
 constexpr int kFwZ = 16;
+inline int fr_weights_zc(const Dims& d) {
+    const long columns = (long)(d.nx / 64 + 1) * (d.ny / 4 + 1);
+    return (int)std::max<long>(2, std::min<long>(kFwZ, columns * (d.nz + 1) / 2048));
+}
 __global__ __launch_bounds__(256) void k_fr_weights(const double* __restrict__ vs, Dims d,
-                                                    float* __restrict__ uw, float* __restrict__ vw,
-                                                    float* __restrict__ ww) {
+                                                    int zc, float* __restrict__ uw,
+                                                    float* __restrict__ vw, float* __restrict__ ww) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y * blockDim.y + threadIdx.y;
-    const int k0 = blockIdx.z * kFwZ, k1 = min(k0 + kFwZ, d.nz + 1);
+    const int k0 = blockIdx.z * zc, k1 = min(k0 + zc, d.nz + 1);
     if (i > d.nx || j > d.ny) return;
     const idx_t vx = d.nx + 1, vxy = vx * (d.ny + 1);
     const int i1 = min(i + 1, d.nx), j1 = min(j + 1, d.ny);

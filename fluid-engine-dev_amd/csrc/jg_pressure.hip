@@ -306,8 +306,9 @@ int jg_fr_build(jg_solver* s, const double* u, const double* v, const double* w,
     auto faces = [](const Dims& d, int a) {
         return Dims{d.nx + (a == 0), d.ny + (a == 1), d.nz + (a == 2)};
     };
-    k_fr_weights<<<dim3(d0.nx / 64 + 1, d0.ny / 4 + 1, d0.nz / kFwZ + 1), dim3(64, 4, 1), 0, s->stream>>>(
-        boundary_sdf_vertex, d0, s->lv[0].uw, s->lv[0].vw, s->lv[0].ww);
+    const int wz = fr_weights_zc(d0);
+    k_fr_weights<<<dim3(d0.nx / 64 + 1, d0.ny / 4 + 1, d0.nz / wz + 1), dim3(64, 4, 1), 0, s->stream>>>(
+        boundary_sdf_vertex, d0, wz, s->lv[0].uw, s->lv[0].vw, s->lv[0].ww);
     k_fr_sdf_to_float<<<nblocks_1d(d0.n()), 256, 0, s->stream>>>(fluid_sdf, s->lv[0].fs, d0.n());
     for (size_t l = 1; l < s->lv.size(); ++l) {
         const Level &f = s->lv[l - 1], &c = s->lv[l];

@@ -192,11 +192,13 @@ def test_fr_torus_512_matches_oracle(solver):
 
 
 @pytest.mark.parametrize("n,levels", [((124, 12, 10), 2), ((128, 10, 36), 2), ((248, 4, 34), 2),
-                                      ((252, 20, 8), 3), ((2, 2, 2), 2), ((66, 6, 70), 2)])
+                                      ((252, 20, 8), 3), ((2, 2, 2), 2), ((66, 6, 70), 2),
+                                      ((300, 100, 130), 2)])
 def test_fr_weights_and_restriction_on_ragged_grids(solver, oracle, n, levels):
     # rows of coarse cells and faces around 62 (what a wave of the restriction
     # takes) and two of them, planes around its chunks of 8, vertices around
-    # the weights' tiles of 64 x 4 x 16; random distances, so that every
+    # the weights' tiles of 64 x 4 and chunks of 2 planes (of 8 in the last
+    # grid); random distances, so that every
     # corner case of a face occurs, infinite fluid distances among them
     print(f"case fr ragged n={n}", flush=True)
     nx, ny, nz = n

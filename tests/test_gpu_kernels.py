@@ -88,13 +88,19 @@ def test_relax_red_black(solver, oracle, shape, sor):
     assert np.array_equal(host(dx), oracle.gs_relax(A, b, sor, x, red_black=True))
 
 
-def test_relax_jacobi(solver, oracle):
+# per cell: one plane, fewer than 48 columns, fewer than 2^17 cells; the tiled
+# z-march: whole 64 x 8 tiles, and partial ones in x, y and z over several chunks
+@pytest.mark.parametrize("shape", [(20, 12, 9), (48, 8, 1), (63, 9, 5), (400, 330, 1), (47, 65, 43),
+                                   (64, 64, 32), (48, 53, 52), (65, 67, 33), (130, 43, 40)])
+def test_relax_jacobi(solver, oracle, shape):
+    print(f"case relax_jacobi shape={shape}", flush=True)
     rng = np.random.default_rng(16)
-    A = random_stencil(20, 12, 9, rng)
-    b = rng.uniform(-1, 1, (9, 12, 20))
-    x = rng.uniform(-1, 1, (9, 12, 20))
-    out = empty((9, 12, 20))
-    solver.relax_jacobi((20, 12, 9), dev(A), dev(b), dev(x), out)
+    nx, ny, nz = shape
+    A = random_stencil(nx, ny, nz, rng)
+    b = rng.uniform(-1, 1, (nz, ny, nx))
+    x = rng.uniform(-1, 1, (nz, ny, nx))
+    out = empty((nz, ny, nx))
+    solver.relax_jacobi(shape, dev(A), dev(b), dev(x), out)
     assert np.array_equal(host(out), oracle.jacobi_relax(A, b, x))
 
 
