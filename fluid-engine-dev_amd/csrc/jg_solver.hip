@@ -1622,9 +1622,12 @@ int mgpcg_run(jg_solver* s, unsigned max_iter, const jg_mg_params* p, const jg_g
 
 // ------------------------------------------------ solves in a box (jg_box.h)
 
-// Grids from which a solve looks for its box: below, the scan's launches
-// and its wait (about 30 us) outweigh the cells it could leave out.
-constexpr idx_t kBoxMgCells = (idx_t(1) << 18) + 1, kBoxCgCells = idx_t(1) << 16;
+// Grids above which a solve looks for its box: up to there, the scan's launches
+// and its wait (about 40 us) outweigh the cells it could leave out.  Whole
+// solves of a pool, time whole / in its box, FP64 and mixed: 64^3 (2^18 cells)
+// with 30% fluid 1.30 and 1.11, 60% 0.98 and 1.02, 75% 0.90 and 0.93; 512^2
+// 1.04 and 0.99, 1.00 and 0.97, 0.93 and 0.95.
+constexpr idx_t kBoxMgCells = idx_t(1) << 18, kBoxCgCells = idx_t(1) << 16;
 // A box of more than this share of the grid is not worth its copy.
 constexpr double kBoxShare = 0.85;
 
@@ -1635,7 +1638,7 @@ int find_box(jg_solver* s, size_t L, double most, Box* box, double* share) {
     const Dims& d = l0.d;
     k_box_reset<<<1, 64, 0, s->stream>>>(s->box_scan);
     const unsigned gx = (d.nx + 63) / 64;
-    // at most 128 waves in all
+    // at most 128 waves in all up to 2048 columns
     k_box_scan<true><<<dim3(gx, std::max(1u, 32u / gx), 1), 64 * kBoxY, 0, s->stream>>>(
         l0.A64, s->b, d, most, s->box_scan);
     const dim3 grid(gx, (d.ny + kBoxY - 1) / kBoxY, (d.nz + kBoxZ - 1) / kBoxZ);
@@ -1683,10 +1686,10 @@ bool box_reserve(jg_solver* s, size_t L) {
 // work vectors and control blocks are s's own, which are larger; A32 too, so
 // s's FP32 copy has to be made anew afterwards.
 template <typename Run>
-int solve_in_box(jg_solver* s, size_t L, idx_t from, double most, bool mixed, Run&& run) {
+int solve_in_box(jg_solver* s, size_t L, idx_t above, double most, bool mixed, Run&& run) {
     auto whole = [&]() { return run(s, [] { return (int)JG_OK; }); };
     Level& l0 = s->lv[0];
-    if (l0.d.n() < from || s->nsys > 1) return whole();
+    if (l0.d.n() <= above || s->nsys > 1) return whole();
     if (!s->box_scan && !dalloc_spare(s, &s->box_scan, 2)) return whole();
     Box box;
     double share = 1.0;
