@@ -1,10 +1,14 @@
 """Batched MGPCG: independent pressure systems of uneven sizes solved by one
 captured hipGraph with per-system convergence flags.
 
-Per system the batch runs the same kernels in the same order as a single
-jg_solver_mgpcg solve; the only differences are the sweep tiling the
-autotuner picks (tuning is shared between identical hierarchies) and the
-replayed no-op iterations after convergence.  So each batched solution must
+Per system the batch runs the same algorithm as a single jg_solver_mgpcg solve.
+What differs is how it is launched: the launch rules count the blocks of all
+systems of a group, so a level may take another kernel of the same values or
+another cut of a reduction; a member is always solved on its whole grid, where
+a single solve of more than 2^18 cells may run in the box of the cells that
+take part; and iterations after convergence are replayed as no-ops.  (The
+systems that are compared with a single solve here have at most 2^18 cells.)
+So each batched solution must
 match the single-system solve to rounding (1e-10 relative, iterations within
 one), and meet the parity bar: relative residual <= 1e-8, FP64 and mixed
 solutions within 1e-6 of each other.
@@ -96,7 +100,7 @@ def test_batch_64_uneven_systems(gpu):
             p = jetgpu.mg_params(max_levels=5, **PARAMS)
             o = jetgpu.gpu_options(precision=precision, stop_rule=jetgpu.JG_STOP_RELATIVE,
                                    rel_tol=1e-9)
-            b.mgpcg(500, p, o)  # tuning and graph capture
+            b.mgpcg(500, p, o)  # graph capture
             infos, ms = b.mgpcg(500, p, o)
             print(f"  precision={precision} batch ms={ms:.2f} "
                   f"max iterations={max(i.iterations for i in infos)}", flush=True)
