@@ -117,18 +117,20 @@ March march(int nz, long tiles, long cus, double halo, double pair, double whole
 // How k_rb_sweep runs on shape d: tile rows per thread, planes per block, and
 // the cost in plane steps of one-row blocks.  FP32: one row, two blocks per CU.
 // FP64: one row and one block per CU, or (without a correction) two rows and
-// two blocks, whose step alone costs 1.2 times as much.  A sweep from zero is
-// as fast or faster with two on every shape measured; a plain one where two
-// rounds of blocks become one or many: 512 x 512 x 2 cells 18 -> 14 us,
-// 192 x 160 x 144 71 -> 59, 96^3 20 with one row and 23 with two.  Over 32
-// shapes this is 0.7% above the faster of the two on average (one row alone:
-// 10%).
+// two blocks, whose step alone costs 1.2 times as much, and 1.5 times where it
+// sums b.x and b.b (that kernel spills).  Two rows are the better where they
+// make two rounds of blocks one or many; one / two, us: 512 x 512 x 2 cells
+// plain 18 / 14, from zero 17 / 14, with the sums 21 / 18; 192 x 160 x 144 75 /
+// 63, 67 / 58, 78 / 80; 256 x 160 x 256 175 / 165, 149 / 149, 187 / 206; 96^3
+// 20 / 23, 16 / 17, 22 / 27.  Over 22 such shapes the rule is 0.3% above the
+// faster of the two on average in plain sweeps, 1.3% from zero (at worst 12%, 250^3)
+// and 0.2% with the sums.
 struct SweepShape {
     int rows, zc;
     double cost;
 };
 template <typename T>
-SweepShape sweep_shape(const jg_solver* s, const Dims& d, bool zero, bool correct) {
+SweepShape sweep_shape(const jg_solver* s, const Dims& d, bool zero, bool correct, bool sums) {
     const long tiles = (long)((d.nx + kSwIX - 1) / kSwIX) * ((d.ny + kSwIY - 1) / kSwIY) * s->nsys;
     if (sizeof(T) == 4) {
         const March m = march(d.nz, tiles, s->cus, 2, 1.8, 0.85);
@@ -136,8 +138,11 @@ SweepShape sweep_shape(const jg_solver* s, const Dims& d, bool zero, bool correc
     }
     const March one = march(d.nz, tiles, s->cus, 3, 0.0, 0.5);
     if (!correct) {
-        const March two = march(d.nz, tiles, s->cus, zero ? 1 : 3, 1.5, 0.5);
-        if (zero || 1.2 * two.cost < one.cost) return {2, two.zc, 1.2 * two.cost};
+        const March two = march(d.nz, tiles, s->cus, 3, 1.5, 0.5);
+        const double cost = two.cost * (1.2 + (sums ? 0.3 * two.zc / (two.zc + 3) : 0.0));
+        // from zero nothing is loaded for the planes before the first
+        if (cost < one.cost)
+            return {2, zero ? march(d.nz, tiles, s->cus, 1, 1.5, 0.5).zc : two.zc, cost};
     }
     return {1, one.zc, one.cost};
 }
@@ -167,7 +172,7 @@ inline dim3 grid_1d(int nb, const jg_solver* s) { return dim3((unsigned)nb, (uns
 template <typename T>
 int launch_sweep(jg_solver* s, const Row<T>* A, const T* b, const T* xin, T* xout, const Dims& d,
                  int first, const T* coarse, double* p_bx, double* p_bb, T omega, const Ctl* ctl) {
-    const SweepShape shape = sweep_shape<T>(s, d, !xin && !coarse, coarse != nullptr);
+    const SweepShape shape = sweep_shape<T>(s, d, !xin && !coarse, coarse != nullptr, p_bx != nullptr);
     int zc = shape.zc;
     const long cols = (long)((d.nx + kSwIX - 1) / kSwIX) * ((d.ny + kSwIY - 1) / kSwIY);
     // one b.x / b.b partial per block: keep the block count within a slot
@@ -178,15 +183,14 @@ int launch_sweep(jg_solver* s, const Row<T>* A, const T* b, const T* xin, T* xou
     grid = grid_sys(grid, s);
     const int code = (first ? 8 : 0) | (xin ? 0 : 4) | (coarse ? 2 : 0) | (p_bx ? 1 : 0);
     const dim3 block(kSwLX, kSwLY / shape.rows, 1);
-    // the row counts that sweep_shape can ask for: R2 two, R1 one
 #define JG_SWEEP_CASE(C, F, Z, K, D)                                                              \
     case C: {                                                                                     \
-        constexpr int R2 = sizeof(T) == 8 && !K ? 2 : 1, R1 = R2 == 2 && Z ? 2 : 1;               \
+        constexpr int R2 = sizeof(T) == 8 && !K ? 2 : 1;                                          \
         if (shape.rows == 2)                                                                      \
             k_rb_sweep<T, F, Z, K, D, R2><<<grid, block, 0, s->stream>>>(                         \
                 A, b, xin, xout, d, zc, omega, coarse, p_bx, p_bb, ctl);                          \
         else                                                                                      \
-            k_rb_sweep<T, F, Z, K, D, R1><<<grid, block, 0, s->stream>>>(                         \
+            k_rb_sweep<T, F, Z, K, D, 1><<<grid, block, 0, s->stream>>>(                         \
                 A, b, xin, xout, d, zc, omega, coarse, p_bx, p_bb, ctl);                          \
         break;                                                                                    \
     }
@@ -322,7 +326,7 @@ std::vector<int> sweep_plan(const jg_solver* s, const Dims& d, unsigned n, int p
         const double m = sweep2_march(s, d, S2Tile<false>::IX, S2Tile<false>::IY).cost;
         two = bricks_z < 65536 && 3 + 0.0165 * bricks < 6.5 + 1.55 * (m + 2) ? kLaunchBrick : kLaunchMarch;
     } else {
-        const double m = sweep_shape<T>(s, d, false, false).cost;
+        const double m = sweep_shape<T>(s, d, false, false, false).cost;
         two = bricks_z < 65536 && 3 + 0.034 * bricks < 2 * (4.3 + 1.62 * m) ? kLaunchBrick : kLaunchSingle;
     }
     if (pairs < 0 || s->twod || d.n() <= BotCfg<T>::MaxCells) two = kLaunchSingle;

@@ -164,14 +164,16 @@ def test_mgpcg_two_sweep_kernels_bitwise(solver, oracle, precision):
     assert rel_err(out[-1][1], out[1][1]) <= 1e-12
 
 
-def test_mgpcg_two_row_sweeps(solver, oracle):
+@pytest.mark.parametrize("depth", [2, 4])
+def test_mgpcg_two_row_sweeps(solver, oracle, depth):
     # more tiles than CUs on a flat grid: FP64 single sweeps hold two tile rows
-    # per thread, and the last one of level 0 writes the r.z / r.r partials
-    print("case mgpcg two-row sweeps", flush=True)
-    A, _ = poisson_helper(520, 500, 4)
+    # per thread; on two planes also the last one of level 0, which writes the
+    # r.z / r.r partials (on four it holds one)
+    print(f"case mgpcg two-row sweeps depth={depth}", flush=True)
+    A, _ = poisson_helper(520, 500, depth)
     A[..., 0] += 0.05
     b = np.random.default_rng(35).uniform(-1, 1, A.shape[:3])
-    solver.set_levels([(520, 500, 4), (260, 250, 2)])
+    solver.set_levels([(520, 500, depth), (260, 250, depth // 2)])
     solver.upload(0, A, b)
     solver.coarsen()
     p = jetgpu.mg_params(max_levels=2, restrict_iter=2, correct_iter=2, coarsest_iter=20,
