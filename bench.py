@@ -111,8 +111,10 @@ def main():
     solver.sp_build(u, v, w, bs, fs, 1.0)
     torch.cuda.synchronize()
     build_ms = (time.perf_counter() - t0) * 1e3
-    fluid_fraction = float(((bs >= 0) & (fs < 0)).double().mean().item())
-    del u, v, w, bs, fs
+    fluid = (bs >= 0) & (fs < 0)
+    fluid_fraction = float(fluid.double().mean().item())
+    solved = box_cells(fluid, L)
+    del u, v, w, bs, fs, fluid
     torch.cuda.empty_cache()
     log(f"bench: system built n={n} levels={L} fluid={fluid_fraction:.3f}")
 
@@ -159,8 +161,8 @@ def main():
                        ("copy", jg.JG_KERNEL_COPY)):
         ms, nbytes = solver.time_kernel(kid, jg.JG_MIXED, 50)
         kern[kname] = {"avg_ms": ms, "bytes": nbytes, "gbs": nbytes / ms / 1e6}
-    traffic = load_traffic(n)
-    roof = roofline(kern, traffic)
+    traffic = load_traffic(args)
+    roof = roofline(kern, traffic, n)
     n_cells = n ** 3
     out = {
         "metric": METRIC,
@@ -188,14 +190,16 @@ def main():
         "kernels_mixed": {k: {"avg_us": round(vv["avg_ms"] * 1e3, 2), "alg_gbs": round(vv["gbs"], 1)}
                           for k, vv in kern.items()},
         "roofline": roof,
+        # the cells the solve visits: the box of the fluid, not the grid
         "solve_alg_gbs": {
-            "fp64": round(ALG_BYTES_PER_CELL["fp64"] * n_cells * res["fp64"]["iterations"]
+            "cells": solved,
+            "fp64": round(ALG_BYTES_PER_CELL["fp64"] * solved * res["fp64"]["iterations"]
                           / (res["fp64"]["ms"] * 1e-3) / 1e9, 1),
             "mixed": round((ALG_BYTES_PER_CELL["mixed"] * res["mixed"]["iterations"]
                             + ALG_BYTES_PER_CELL["refine"] * res["mixed"]["refinements"])
-                           * n_cells / (res["mixed"]["ms"] * 1e-3) / 1e9, 1)},
+                           * solved / (res["mixed"]["ms"] * 1e-3) / 1e9, 1)},
     }
-    if traffic and traffic.get("solve"):
+    if traffic:
         # the metric's HBM GB/s: counter-measured bytes of one whole solve
         # (every kernel of it, from the FETCH_SIZE / WRITE_SIZE passes) over
         # the solve time measured here
@@ -242,18 +246,56 @@ def main():
     solver.close()
 
 
-def load_traffic(n):
-    """The counter-measured traffic summary of this workload, if it is there
-    and was measured at this size."""
+def box_cells(fluid, levels):
+    """Cells of the box a solve of more than 2^18 cells runs in: the bounding
+    box of the fluid, its bounds multiples of the coarsest level's cells; the
+    grid where that is more than 85% of it."""
+    import torch
+
+    g = 1 << (levels - 1)
+    n = fluid.numel()
+    box = 1
+    for axis in range(3):
+        at = torch.nonzero(fluid.any(dim=(axis + 1) % 3, keepdim=True)
+                           .any(dim=(axis + 2) % 3, keepdim=True).flatten())
+        lo, hi = int(at[0].item()), int(at[-1].item()) + 1
+        box *= (hi + g - 1) // g * g - lo // g * g
+    return n if n <= 1 << 18 or box > 0.85 * n else box
+
+
+def traffic_key(args):
+    """What a traffic summary is a measurement of: the workload and the
+    sources of the library."""
+    import glob
+    import hashlib
+
+    h = hashlib.sha256()
+    for pattern in ("csrc/*.h", "csrc/*.hip", "Makefile"):
+        for fn in sorted(glob.glob(os.path.join(PKG, pattern))):
+            with open(fn, "rb") as f:
+                h.update(os.path.basename(fn).encode() + b"\0" + f.read())
+    return {"n": args.n, "levels": args.levels, "seed": args.seed, "rel_tol": args.rel_tol,
+            "omega": args.omega, "sources": h.hexdigest()[:16]}
+
+
+def load_traffic(args):
+    """The counter-measured traffic summary, if it is there and was measured
+    on this workload with these sources: bytes of another build's launches
+    over this one's times would be no measurement."""
     try:
         with open(TRAFFIC_FILE) as f:
             t = json.load(f)
     except (OSError, ValueError):
         return None
-    return t if t.get("n") == n else None
+    key = traffic_key(args)
+    stale = [k for k in key if t.get(k) != key[k]]
+    if stale:
+        log(f"bench: traffic summary left out: it was measured with another {', '.join(stale)}")
+        return None
+    return t
 
 
-def roofline(kern, traffic):
+def roofline(kern, traffic, n):
     """Roofline of the dominant kernel: the level-0 smoothing launches of one
     V-cycle (pre and post), per launch.  achieved = algorithmic bytes per
     launch / average launch duration (both measured here); traffic = the
@@ -264,7 +306,7 @@ def roofline(kern, traffic):
     achieved = alg / t_ms / 1e6
     names = None
     hbm = None
-    if traffic and traffic.get("launches"):
+    if traffic:
         tl = traffic["launches"]
         names = " + ".join(tl[k]["kernel"] for k in ("pre0", "post0"))
         hbm = (tl["pre0"]["hbm_bytes"] + tl["post0"]["hbm_bytes"]) / 2.0
@@ -278,8 +320,7 @@ def roofline(kern, traffic):
         "algorithmic_bytes": alg, "avg_us": round(t_ms * 1e3, 2),
         "launches": {k: {"avg_us": round(kern[k]["avg_ms"] * 1e3, 2),
                          "algorithmic_bytes": kern[k]["bytes"],
-                         "alg_bytes_per_cell": round(kern[k]["bytes"] / traffic_cells(traffic), 3)
-                         if traffic else None}
+                         "alg_bytes_per_cell": round(kern[k]["bytes"] / n ** 3, 3)}
                      for k in ("pre0", "post0")},
     }
     if hbm:
@@ -287,10 +328,6 @@ def roofline(kern, traffic):
         roof["measured_frac"] = round(hbm / t_ms / 1e6 / HBM_PEAK_GBS, 4)
         roof["traffic_source"] = TRAFFIC_FILE_REL
     return roof
-
-
-def traffic_cells(traffic):
-    return float(traffic["n"]) ** 3
 
 
 def traffic_probe(args):
@@ -387,8 +424,8 @@ def segments(disp):
 def collect_traffic(args):
     """Two rocprofv3 counter passes (FETCH_SIZE, then WRITE_SIZE) over the
     probe program, each a child process; writes the summary JSON (per-launch
-    bytes of the level-0 smoothing launches and whole-solve bytes) to
-    gpurun_out/traffic/."""
+    bytes of the level-0 smoothing launches and whole-solve bytes), which goes
+    under profiles/."""
     import subprocess
     from collections import Counter
 
@@ -400,7 +437,8 @@ def collect_traffic(args):
         d = os.path.join(out_root, counter.lower())
         cmd = ["rocprofv3", "--pmc", counter, "-f", "csv", "-d", d, "-o", "probe", "--",
                sys.executable, os.path.join(ROOT, "bench.py"), "--only", "traffic-probe",
-               "--n", str(args.n), "--levels", str(args.levels)]
+               "--n", str(args.n), "--levels", str(args.levels), "--seed", str(args.seed),
+               "--rel-tol", str(args.rel_tol), "--omega", str(args.omega)]
         log("bench: " + " ".join(cmd))
         subprocess.run(cmd, cwd="/tmp", env=env, check=True, timeout=600)
         segs = segments(read_counters(d, counter))
@@ -422,7 +460,7 @@ def collect_traffic(args):
     cname, cf = repeated(raw["FETCH_SIZE"]["copy"])
     _, cw = repeated(raw["WRITE_SIZE"]["copy"])
     fscale, wscale = copy_bytes / (cf * 1024.0), copy_bytes / (cw * 1024.0)
-    res = {"n": n, "levels": args.levels,
+    res = {**traffic_key(args),
            "command": "python3 bench.py --collect-traffic (rocprofv3 --pmc FETCH_SIZE, then "
                       "--pmc WRITE_SIZE, -- python3 bench.py --only traffic-probe)",
            "copy": {"kernel": cname, "bytes_each_way": copy_bytes, "fetch_kib": cf, "write_kib": cw,
